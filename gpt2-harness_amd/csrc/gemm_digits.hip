@@ -1,0 +1,498 @@
+// GEMM of fp32 activations with integer weights on the int8 matrix cores
+// (gfx950): the quantized Linears of a prompt (model.py:254,319,352,355 with
+// M = B*T rows) in a model that keeps fp32 activations:
+//     y[m, n] = scale[n] * sum_k x[m, k] * q[n, k] + bias[n]
+//
+// A row of x becomes a fixed-point row, x[m, k] = 2^(e_m - 29) X[m, k] with
+// 2^e_m <= max_k |x[m, k]| < 2^(e_m + 1) and X = rint(x 2^(29 - e_m)) a 31-bit
+// integer (exact for every element within 2^-6 of the row's largest; smaller
+// ones are rounded by at most 2^-30 of it), and X four signed base-256 digits, each an
+// int8 plane. Every product and sum the MFMAs form is then an exact integer
+// (|sum| <= K 2^14 < 2^31), four sums an output, which the epilogue combines in
+// fp32: an output carries one rounding of its inputs and a handful at the end,
+// where an fp32 accumulation rounds once a step. Relative 2-norm error against
+// 64 bits, unit-variance rows with one column in 256 eight times larger, as
+// three bf16 planes with fp32 sums before and as digits now: K = 768 1.0e-7 /
+// 5.1e-8, K = 1600 5.2e-7 / 5.1e-8, K = 6400 1.0e-6 / 5.1e-8.
+//
+// Why four int8 planes: int8 MFMAs run at twice the bf16 rate, so four planes
+// cost two bf16 passes over the product instead of three, and the codes enter
+// the matrix cores as they are stored, with no widening beside the MFMAs.
+// M = 4096, three planes before / digits now, the planes' pass included: 1600 x
+// 4800 242 / 154 us, 1600 x 1600 82 / 64, 6400 x 1600 310 / 200; M = 512, 768 x
+// 2304 25 / 15; M = 77, 768 x 3072 56 (the decode GEMV) / 11. What bounds the
+// large ones: the matrix cores at the clock the chip holds under them (a loop
+// of independent int8 MFMAs on random data reaches 3.0 of the nominal 5 POP/s:
+// 84 us of the 143 at 1600 x 4800), then the step's LDS traffic, which does not
+// hide wholly beside one wavefront's MFMAs a SIMD.
+#include <algorithm>
+
+#include "tiq_internal.hpp"
+
+namespace tiq {
+namespace {
+
+#include "gemm_staged_kernel.hpp"
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x16 __attribute__((ext_vector_type(16)));
+
+constexpr int kDigits = 4;
+
+// The digit planes in MFMA operand order: for row tile t (32 rows), unit u (32
+// columns) and digit d (0 lowest) a 1 KB block at ((t U + u) 4 + d) 1024, byte
+// 16 l + j of it the digit of row 32 t + l % 32, column 32 u + 16 (l / 32) + j
+// (NIB: the even columns of the 16 first, then the odd ones -- the order in
+// which nibble weights unpack), so the product's loads and LDS accesses are
+// all contiguous. One workgroup per 8 rows: 8 rows' chunks of a block are 128
+// consecutive bytes, a whole cache line a store. rs[m] = 2^(e_m - 29), NaN for
+// a row holding an infinity or NaN (every output of it is then NaN).
+// IT: 1024-column passes held in registers; 0: the row is read twice.
+constexpr int kSplitThreads = 512;
+
+__device__ __forceinline__ uint32_t digits_of(float v, float mul) {
+    const int t = (int)__builtin_rintf(v * mul) + 0x00808080;
+    return (uint32_t)t ^ 0x00808080u;
+}
+
+template <bool NIB>
+__device__ __forceinline__ void store_digits(const float (&v)[16], float mul, uint8_t* __restrict__ dst) {
+    u32x4 pl[kDigits];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {  // four columns -> one dword of each plane
+        uint32_t t[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int p = 4 * g + i;
+            t[i] = digits_of(v[NIB ? (p < 8 ? 2 * p : 2 * (p - 8) + 1) : p], mul);
+        }
+        const uint32_t a = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u);  // d0 d0 d1 d1 of t0, t1
+        const uint32_t b = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
+        const uint32_t c = __builtin_amdgcn_perm(t[1], t[0], 0x07030602u);  // d2 d2 d3 d3
+        const uint32_t d = __builtin_amdgcn_perm(t[3], t[2], 0x07030602u);
+        pl[0][g] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+        pl[1][g] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+        pl[2][g] = __builtin_amdgcn_perm(d, c, 0x05040100u);
+        pl[3][g] = __builtin_amdgcn_perm(d, c, 0x07060302u);
+    }
+#pragma unroll
+    for (int q = 0; q < kDigits; ++q) *reinterpret_cast<u32x4*>(dst + 1024 * q) = pl[q];
+}
+
+template <int IT, bool NIB>
+__global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float* __restrict__ x, int64_t ldx, int M,
+                                                                     int K, uint8_t* __restrict__ xt,
+                                                                     float* __restrict__ rs, bool gelu) {
+    constexpr int WV = kSplitThreads / 64, CT = kSplitThreads / 8;  // 16-column chunks a pass
+    __shared__ uint32_t am[WV][8];
+    const int tid = threadIdx.x, r8 = tid & 7, c0 = tid >> 3;
+    const int m = blockIdx.x * 8 + r8;
+    const int NC = K / 16, U = K / 32;
+    // A quad of lanes reads 64 consecutive bytes of each of its four rows in
+    // turn (16 segments a load instruction, not 64), then transposes: each lane
+    // ends with the 16 columns of its own row.
+    const int j4 = tid & 3;
+    const float* xq[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        xq[i] = x + (int64_t)min((int)blockIdx.x * 8 + (r8 & 4) + i, M - 1) * ldx + 4 * j4;
+    const bool odd = j4 & 1, high = j4 & 2;
+    auto load = [&](int c, float (&v)[16]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            *reinterpret_cast<float4*>(v + 4 * i) = *reinterpret_cast<const float4*>(xq[i] + 16 * c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int i = 0; i < 4; i += 2) {  // rows i, i + 1 with the neighbour lane
+                const float got = dpp_move<0xB1>(odd ? v[4 * i + e] : v[4 * i + 4 + e]);
+                v[4 * i + e] = odd ? got : v[4 * i + e];
+                v[4 * i + 4 + e] = odd ? v[4 * i + 4 + e] : got;
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {  // rows i, i + 2 with the lane two away
+                const float got = dpp_move<0x4E>(high ? v[4 * i + e] : v[4 * i + 8 + e]);
+                v[4 * i + e] = high ? got : v[4 * i + e];
+                v[4 * i + 8 + e] = high ? v[4 * i + 8 + e] : got;
+            }
+        }
+        if (gelu) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[i] = gelu_tanh(v[i]);
+        }
+    };
+    uint32_t mx = 0;
+    float v[IT ? IT : 1][16];
+    if constexpr (IT > 0) {
+#pragma unroll
+        for (int it = 0; it < IT; ++it) load(min(c0 + CT * it, NC - 1), v[it]);  // past the row: its last chunk again
+#pragma unroll
+        for (int it = 0; it < IT; ++it)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = max(mx, abs_bits(v[it][i]));
+    } else {
+        for (int c = c0; c < NC; c += CT) {
+            load(c, v[0]);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = max(mx, abs_bits(v[0][i]));
+        }
+    }
+#pragma unroll
+    for (int off = 32; off >= 8; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
+    if ((tid & 63) < 8) am[tid >> 6][r8] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < WV; ++w) mx = max(mx, am[w][r8]);
+    // rows below 2^-97 share its exponent: both powers of two stay normal
+    const int e = max((int)(mx >> 23) - 127, -97);
+    const bool finite = mx < 0x7f800000u;
+    const float mul = finite ? __uint_as_float((uint32_t)(29 - e + 127) << 23) : 0.f;
+    if (c0 == 0 && m < M)
+        rs[m] = finite ? __uint_as_float((uint32_t)(e - 29 + 127) << 23) : __uint_as_float(0x7fc00000u);
+    uint8_t* base = xt + (int64_t)(m >> 5) * U * 4096 + (m & 31) * 16;
+    if constexpr (IT > 0) {
+#pragma unroll
+        for (int it = 0; it < IT; ++it) {
+            const int c = c0 + CT * it;
+            if (c < NC && m < M) store_digits<NIB>(v[it], mul, base + (int64_t)(c >> 1) * 4096 + (c & 1) * 512);
+        }
+    } else {
+        for (int c = c0; c < NC; c += CT) {
+            load(c, v[0]);  // every lane of a quad: rows past M too
+            if (m < M) store_digits<NIB>(v[0], mul, base + (int64_t)(c >> 1) * 4096 + (c & 1) * 512);
+        }
+    }
+}
+
+// The product. A workgroup of four wavefronts, WMW x (4 / WMW) over its tile,
+// each with TM row tiles (32 rows of x) and TN column tiles (32 rows of w): BM =
+// 32 TM WMW, BN = 32 TN (4 / WMW). Per k64 step a wavefront issues 8 TM TN
+// MFMAs: each of its weight fragments meets the four digits of each row tile,
+// so a weight fragment is read once for four MFMAs. Digits and codes pass
+// through LDS (double buffered, one barrier a step) in operand blocks; their
+// loads wait in D register sets, issued D - 1 steps before their LDS store.
+// Beside each MFMA goes one of the step's other operations.
+// LDS blocks: the digits as they lie in memory; codes per 32-row tile 2 KB,
+// chunk c (16 columns) of row r at 512 c + 16 (r ^ 2 c) -- staging stores (two
+// rows' four chunks per 8 lanes) and fragment reads (8 rows of a chunk) both
+// cover every bank.
+// FMT kW8 (codes) or kW4 (the reference's nibbles, unpacked to 16 (n - 8) on
+// the LDS store: the 16 is taken out with the scale).
+// gridDim.z > 1: split over K, workgroup z writes fp32 slice z of y (no bias).
+template <int WMW, int TM, int TN, int D, int OCC, bool PERSIST, int FMT, typename TY>
+__global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
+    const uint8_t* __restrict__ xt, const float* __restrict__ rs, const uint8_t* __restrict__ w, int64_t ldw,
+    const float* __restrict__ scale, const float* __restrict__ bias, TY* __restrict__ y, int64_t ldy, int M, int N,
+    int K) {
+    static_assert(D >= 2, "register sets");
+    constexpr int WNW = 4 / WMW;
+    constexpr int MT = TM * WMW, NTL = TN * WNW;  // row and column tiles of the workgroup
+    constexpr int NF = TM * kDigits;              // activation fragments a k32 block
+    constexpr int NRD = NF + TN, NMF = NF * TN;   // fragment reads and MFMAs a k32 block
+    constexpr int XL = 2 * MT, WL = NTL / 2, NL = XL + WL;  // staging loads a thread and step
+    constexpr int XS = MT * 8192, STAGE = XS + NTL * 2048;
+    static_assert(NTL % 2 == 0 && NL <= 2 * NMF, "staging split");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WNW, wn = wave % WNW;
+    const int r = lane & 31, h = lane >> 5;
+    const int T = (M + 31) / 32, U = K / 32;
+    const int tiles_m = (T + MT - 1) / MT, tiles_n = (N + 32 * NTL - 1) / (32 * NTL);
+    const int NK = K / 64;
+    const int s0 = (int)blockIdx.z * NK / (int)gridDim.z;
+    const int nk = ((int)blockIdx.z + 1) * NK / (int)gridDim.z - s0;
+    const bool split = gridDim.z > 1;
+
+    // weight staging: rows wrow + 64 j, chunk wch (16 columns)
+    constexpr int WB = FMT == kW8 ? 16 : 8;  // bytes of 16 columns
+    const int wrow = tid >> 2, wch = tid & 3;
+    const int ws = XS + (wrow >> 5) * 2048 + wch * 512 + (((wrow & 31) ^ (2 * wch)) * 16);
+    const uint8_t* xp[MT];
+    uint32_t woff[WL];
+    int tm, tn;
+    u32x4 st[D][NL];
+    auto gload = [&](int s, int p, int q) {
+        if (q < XL) {
+            st[p][q] = *reinterpret_cast<const u32x4*>(xp[q >> 1] + (int64_t)s * 8192 + (q & 1) * 4096);
+        } else {
+            const uint8_t* src = w + (woff[q - XL] + (uint32_t)(4 * s) * WB);
+            if constexpr (FMT == kW8) {
+                st[p][q] = *reinterpret_cast<const u32x4*>(src);
+            } else {
+                const uint2 t = *reinterpret_cast<const uint2*>(src);
+                st[p][q] = u32x4{t.x, t.y, 0u, 0u};
+            }
+        }
+    };
+    // a tile's addresses and its first D stages
+    auto begin_tile = [&](int tile) {
+        staged_tile_of(tile, tm, tn, tiles_m, tiles_n);
+#pragma unroll
+        for (int i = 0; i < MT; ++i)  // row tiles past the last repeat it (not stored)
+            xp[i] = xt + ((int64_t)min(tm * MT + i, T - 1) * U + 2 * s0) * 4096 + tid * 16;
+#pragma unroll
+        for (int j = 0; j < WL; ++j)
+            woff[j] = (uint32_t)min(tn * 32 * NTL + wrow + 64 * j, N - 1) * (uint32_t)ldw +
+                      (uint32_t)(4 * s0 + wch) * WB;
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+#pragma unroll
+            for (int q = 0; q < NL; ++q) gload(min(d, nk - 1), d, q);
+    };
+    auto lstore = [&](int buf, int p, int q) {
+        uint8_t* base = smem + buf * STAGE;
+        if (q < XL) {
+            *reinterpret_cast<u32x4*>(base + q * 4096 + tid * 16) = st[p][q];
+        } else {
+            u32x4 v = st[p][q];
+            if constexpr (FMT == kW4) {
+                uint32_t e0, o0, e1, o1;
+                nibbles_x16(v.x, e0, o0);
+                nibbles_x16(v.y, e1, o1);
+                v = u32x4{e0, e1, o0, o1};
+            }
+            *reinterpret_cast<u32x4*>(base + ws + (q - XL) * 4096) = v;
+        }
+    };
+    i32x4 FX[2][NF], FW[2][TN];
+    int wo[2];  // chunk 2 kk + h of row r within a code tile
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) wo[kk] = XS + wn * TN * 2048 + (2 * kk + h) * 512 + ((r ^ (2 * (2 * kk + h))) * 16);
+    const int xo = wm * TM * 8192 + lane * 16;
+    auto fread = [&](int buf, int kk, int set, int f) {
+        const uint8_t* base = smem + buf * STAGE;
+        if (f < TN)
+            FW[set][f] = *reinterpret_cast<const i32x4*>(base + wo[kk] + f * 2048);
+        else
+            FX[set][f - TN] = *reinterpret_cast<const i32x4*>(base + xo + ((f - TN) >> 2) * 8192 + kk * 4096 +
+                                                              ((f - TN) & 3) * 1024);
+    };
+    // D[m][n]: result register q of lane (r, h) holds m = 8 (q / 4) + 4 h + q % 4, n = r
+    i32x16 acc[TN][TM][kDigits];
+    auto mfma = [&](int set, int t, bool fresh) {
+        const int f = t / TN, j = t % TN;
+        const i32x16 z = {};
+        acc[j][f >> 2][f & 3] = __builtin_amdgcn_mfma_i32_32x32x32_i8(FX[set][f], FW[set][j],
+                                                                      fresh ? z : acc[j][f >> 2][f & 3], 0, 0, 0);
+    };
+    // Step s (register set p = s % D): the first k32 block's MFMAs (of step 0
+    // from zero sums) beside the second's fragment reads and stage s + 1's LDS
+    // stores; the barrier; the second block's MFMAs beside the next step's first
+    // fragments and stage s + D's loads into set p. Past the last stage the
+    // loads repeat it, which keeps the body one path.
+    auto step = [&](int s, int p, bool fresh) {
+        const int cur = s & 1, nxt = cur ^ 1, pn = (p + 1) % D;
+        const int sl = min(s + D, nk - 1);
+#pragma unroll
+        for (int t = 0; t < NMF; ++t) {
+            mfma(0, t, fresh);
+#pragma unroll
+            for (int f = t * NRD / NMF; f < (t + 1) * NRD / NMF; ++f) fread(cur, 1, 1, f);
+#pragma unroll
+            for (int q = t * NL / NMF; q < (t + 1) * NL / NMF; ++q) lstore(nxt, pn, q);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < NMF; ++t) {
+            mfma(1, t, false);
+#pragma unroll
+            for (int f = t * NRD / NMF; f < (t + 1) * NRD / NMF; ++f) fread(nxt, 0, 0, f);
+#pragma unroll
+            for (int q = t * NL / NMF; q < (t + 1) * NL / NMF; ++q) gload(sl, p, q);
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    const int total = tiles_m * tiles_n;
+    begin_tile(blockIdx.x);
+    // the workgroup's tiles: one, or every gridDim.x-th of a persistent grid,
+    // where the next tile's first loads go out before the epilogue
+    for (int tile = blockIdx.x;;) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) lstore(0, 0, q);
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < NRD; ++f) fread(0, 0, 0, f);
+        step(0, 0, true);
+        int s = 1;
+        for (; s + D - 1 < nk; s += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) step(s + d, (1 + d) % D, false);
+        }
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (s + d < nk) step(s + d, (1 + d) % D, false);
+
+        // y = (((a3 256 + a2) 256 + a1) 256 + a0) 2^(e_m - 29) scale + bias; a
+        // store instruction writes 32 consecutive outputs of two rows
+        constexpr float unit = FMT == kW8 ? 1.f : 0.0625f;
+        const int n0 = tn * 32 * NTL + wn * 32 * TN, m0 = (tm * MT + wm * TM) * 32;
+        const bool full = m0 + 32 * TM <= M && n0 + 32 * TN <= N;
+        float sc[TN], bi[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = min(n0 + 32 * j + r, N - 1);
+            sc[j] = scale[n] * unit;
+            bi[j] = bias && !split ? bias[n] : 0.f;
+        }
+        float4 rm[TM][4];  // rows past M hold whatever the buffer holds: their outputs are not stored
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                rm[i][g] = *reinterpret_cast<const float4*>(rs + min(m0 / 32 + i, T - 1) * 32 + 8 * g + 4 * h);
+        tile += gridDim.x;
+        const bool more = PERSIST && tile < total;
+        if (more) begin_tile(tile);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            TY* yr = y + ((int64_t)blockIdx.z * M + m0 + 32 * i + 4 * h) * ldy + n0 + r;
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int q = 4 * g + e;
+                    const float rmq = e == 0 ? rm[i][g].x : e == 1 ? rm[i][g].y : e == 2 ? rm[i][g].z : rm[i][g].w;
+                    TY* dst = yr + (int64_t)(8 * g + e) * ldy;
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        float f = (float)acc[j][i][3][q];
+                        f = fmaf(f, 256.f, (float)acc[j][i][2][q]);
+                        f = fmaf(f, 256.f, (float)acc[j][i][1][q]);
+                        f = fmaf(f, 256.f, (float)acc[j][i][0][q]);
+                        const float v = fmaf(f * rmq, sc[j], bi[j]);
+                        if (full || (m0 + 32 * i + 8 * g + 4 * h + e < M && n0 + 32 * j + r < N)) {
+                            if constexpr (sizeof(TY) == 4) dst[32 * j] = v;
+                            else dst[32 * j] = f32_to_bf16_bits(v);
+                        }
+                    }
+                }
+            }
+        }
+        if (!more) break;
+        __syncthreads();  // every wavefront's last LDS reads are done
+    }
+}
+
+template <int WMW, int TM, int TN, int D, int OCC, bool PERSIST, int FMT, typename TY>
+int run_digits(const LinearArgs& a, const uint8_t* xt, const float* rs, TY* y, int64_t ldy, int64_t S) {
+    constexpr int BM = 32 * TM * WMW, BN = 32 * TN * (4 / WMW);
+    const int64_t tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+    const int64_t grid = PERSIST ? std::min<int64_t>(tiles, 256 * OCC) : tiles;
+    hipLaunchKernelGGL((gemm_digits_kernel<WMW, TM, TN, D, OCC, PERSIST, FMT, TY>), dim3((unsigned)grid, 1, (unsigned)S),
+                       dim3(256), 0, a.stream, xt, rs, a.w, a.ldw, a.scale, a.bias, y, ldy, (int)a.M, (int)a.N,
+                       (int)a.K);
+    return launch_status();
+}
+
+// Tiles, measured on MI355X (graph-timed products, fp32 out; us):
+//   32 x 128, two or more workgroups a CU: ahead while the 64 x 128 tiles are
+//     fewer than the 512 that run at once (M = 1001, 1024 x 3072: 18.9 against
+//     20.2; M = 77, 768 x 3072: 7.5 against 9.6);
+//   64 x 128, two a CU, persistent: the larger products (M = 4096: 1600 x 4800
+//     143 against 146 at 64 x 256 and 166 at 32 x 128; 1600 x 1600 53 / 55 / 60);
+//   64 x 256, one a CU: a long K, where its fewer LDS bytes a MFMA weigh more
+//     than its tile's fixed cost (M = 4096, 6400 x 1600: 171 against 187).
+enum DigitTile : int { kTile32x128 = 0, kTile64x128 = 1, kTile64x256 = 2 };
+
+DigitTile digits_tile(int64_t M, int64_t N, int64_t K) {
+    const int64_t rows = (M + 63) / 64;
+    if (rows * ((N + 127) / 128) < 512) return kTile32x128;
+    return K >= 3200 && rows * ((N + 255) / 256) >= 256 ? kTile64x256 : kTile64x128;
+}
+
+// Splits over K: only where the 32 x 128 tiles leave half of the CUs without
+// work and K is long enough for the slices' sum to cost less than it saves (M
+// = 77, 3072 x 768, 18 tiles: 15.1 us unsplit, 6.9 in eight; K = 768: 7.5
+// unsplit, 6.3 in two, less than the reduction's launch). At least six k64
+// steps a split, at most eight splits.
+int64_t digits_splits(int64_t M, int64_t N, int64_t K) {
+    const int64_t tiles = (M + 31) / 32 * ((N + 127) / 128);
+    if (tiles * 2 > 256 || K < 1536) return 1;
+    return std::max<int64_t>(1, std::min<int64_t>({256 / tiles, K / 64 / 6, 8}));
+}
+
+size_t round256(size_t b) { return (b + 255) / 256 * 256; }
+
+template <int FMT, typename TY>
+int dispatch_digits(const LinearArgs& a, DigitTile tile, const uint8_t* xt, const float* rs, TY* y, int64_t ldy,
+                    int64_t S) {
+    switch (tile) {
+        case kTile64x256: return run_digits<2, 1, 4, 2, 1, false, FMT, TY>(a, xt, rs, y, ldy, S);
+        case kTile64x128: return run_digits<2, 1, 2, 2, 2, true, FMT, TY>(a, xt, rs, y, ldy, S);
+        default: return run_digits<1, 1, 1, 4, 2, false, FMT, TY>(a, xt, rs, y, ldy, S);
+    }
+}
+
+template <bool NIB>
+int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu) {
+    const dim3 grid((unsigned)((a.M + 7) / 8)), block(kSplitThreads);
+    const float* x = static_cast<const float*>(a.x);
+    const int M = (int)a.M, K = (int)a.K;
+    if (K <= 1024) hipLaunchKernelGGL((split_digits_kernel<1, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
+    else if (K <= 2048) hipLaunchKernelGGL((split_digits_kernel<2, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
+    else if (K <= 4096) hipLaunchKernelGGL((split_digits_kernel<4, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
+    else if (K <= 7168) hipLaunchKernelGGL((split_digits_kernel<7, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
+    else hipLaunchKernelGGL((split_digits_kernel<0, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
+    return launch_status();
+}
+
+template <int FMT>
+int run_digits_linear(const LinearArgs& a, uint8_t* xt, float* rs, float* part, int64_t S, bool gelu) {
+    int rc = launch_split_digits<FMT == kW4>(a, xt, rs, gelu);
+    if (rc != TIQ_OK) return rc;
+    const DigitTile tile = S > 1 ? kTile32x128 : digits_tile(a.M, a.N, a.K);
+    if (S > 1) {
+        rc = dispatch_digits<FMT, float>(a, tile, xt, rs, part, a.N, S);
+        return rc != TIQ_OK ? rc : launch_splitk_reduce(a, part, S, nullptr);
+    }
+    if (a.y_dtype == TIQ_F32) return dispatch_digits<FMT, float>(a, tile, xt, rs, static_cast<float*>(a.y), a.ldy, 1);
+    return dispatch_digits<FMT, uint16_t>(a, tile, xt, rs, static_cast<uint16_t*>(a.y), a.ldy, 1);
+}
+
+}  // namespace
+
+size_t digits_workspace(int64_t M, int64_t K) {
+    const int64_t rows = (M + 31) / 32 * 32;
+    return round256((size_t)(rows * K * kDigits + rows * 4));
+}
+
+size_t digits_split_workspace(int64_t M, int64_t N, int64_t K) {
+    const int64_t S = digits_splits(M, N, K);
+    return S > 1 ? round256((size_t)(S * M * N * 4)) : 0;
+}
+
+bool digits_supported(const LinearArgs& a) {
+    if (a.x_dtype != TIQ_F32 || (a.fmt != kW8 && a.fmt != kW4) || a.kw) return false;
+    // int32 sums: K 2^14 < 2^31
+    if (a.K % 64 != 0 || a.K > 65536) return false;
+    if (!aligned(a.x, 16) || a.ldx % 4 != 0 || !aligned(a.w, 16) || a.ldw % 16 != 0) return false;
+    // 32-bit byte offsets into the weights, tile counts within a grid
+    if (a.N * a.ldw > 0xffffffffLL) return false;
+    return ((a.M + 31) / 32) * ((a.N + 127) / 128) <= 0x7fffffffLL && a.M <= 0x7fffffff - 64;
+}
+
+int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu) {
+    if (!digits_supported(a)) return TIQ_EUNSUPPORTED;
+    const size_t need = digits_workspace(a.M, a.K);
+    if (!ws || ws_bytes < need || !aligned(ws, 16)) return TIQ_EWORKSPACE;
+    uint8_t* xt = static_cast<uint8_t*>(ws);
+    const int64_t rows = (a.M + 31) / 32 * 32;
+    float* rs = reinterpret_cast<float*>(xt + rows * a.K * kDigits);
+    float* part = reinterpret_cast<float*>(xt + need);
+    // the split needs room for its slices and the reduction's 16-byte accesses
+    // (N % 8 for either output type: both then sum in the same order)
+    const int unit = a.y_dtype == TIQ_F32 ? 4 : 8;
+    int64_t S = digits_splits(a.M, a.N, a.K);
+    if (a.N % 8 != 0 || a.ldy % unit != 0 || !aligned(a.y, 16) || (a.bias && !aligned(a.bias, 16))) S = 1;
+    S = std::min<int64_t>(S, (int64_t)((ws_bytes - need) / (size_t)(a.M * a.N * 4)));
+    S = std::max<int64_t>(S, 1);
+    return a.fmt == kW4 ? run_digits_linear<kW4>(a, xt, rs, part, S, gelu)
+                        : run_digits_linear<kW8>(a, xt, rs, part, S, gelu);
+}
+
+}  // namespace tiq

@@ -1,5 +1,6 @@
 // Linear entry points of the C ABI: argument checks and the choice between
 // the decode GEMV (vector ALUs) and the prefill GEMM (matrix cores).
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 #include <utility>
@@ -56,11 +57,11 @@ namespace {
 // vector-ALU GEMV (below it the GEMM wastes most of each tile).
 constexpr int64_t kGemmMinRows = 128;
 
-// fp32 rows against reference-layout int4 codes take the three-plane
-// matrix-core path (split over K where the tiles are few) from 32 rows, or
+// fp32 rows against reference-layout int4 codes take the matrix cores through
+// digit planes (split over K where the tiles are few) from 32 rows, or
 // from 16 on matrices of 2048 rows or more: below 128 rows there is no
 // batched kernel for int4, and the LDS-staged GEMV, four activation rows a
-// tile, grows with M (GPT-2 small shapes at M = 64: 18-57 us against 12-19 us
+// tile, grows with M (GPT-2 small shapes at M = 64: 18-57 us against 10-13 us
 // through the planes; int8 has the batched kernel up to 64 rows).
 bool w4_planes_rows(int64_t M, int64_t N) { return M >= 32 || (M >= 16 && N >= 2048); }
 
@@ -126,14 +127,31 @@ __global__ void split_bf16x3_kernel(const float* __restrict__ x, int64_t ldx, in
 
 size_t split_workspace(int64_t M, int64_t K) { return (size_t)(M * 3 * K * 2 + 255) / 256 * 256; }
 
-// fp32 activations through the matrix cores when a GEMM takes the three-plane
-// problem (the staged kernel, else the LDS-dequant one); TIQ_EUNSUPPORTED
-// otherwise (the caller falls back). gelu_in: the product takes gelu_tanh(x).
+// Rows at and above which fp32 activations take the int8 matrix cores (digit
+// planes): int8 has the batched kernel up to 64 rows; from 65 the decode GEMV,
+// four activation rows a tile, was the only other one below kGemmMinRows (77
+// rows, 768 x 3072: 56 us against 11 us). int4 as w4_planes_rows.
+bool digits_rows(WFormat fmt, int64_t M, int64_t N) {
+    return M >= kGemmMinRows || (fmt == kW8 ? M > 64 : fmt == kW4 && w4_planes_rows(M, N));
+}
+
+// fp32 activations through the matrix cores: int8 and reference-layout int4
+// weights as exact integer products of digit planes (gemm_digits.hip), else
+// (group-wise int4, or K past the int32 sums) split into three bf16 planes for
+// a GEMM that takes the three-plane problem; TIQ_EUNSUPPORTED otherwise (the
+// caller falls back). gelu_in: the product takes gelu_tanh(x).
 int run_linear_split(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu_in = false) {
     if (a.x_dtype != TIQ_F32 || a.fmt == kF32 || a.K % 4 != 0) return TIQ_EUNSUPPORTED;
-    const bool few = a.M < kGemmMinRows;  // below the GEMM's own row count: int4 from fewer rows
-    if (few && !(a.fmt == kW4 && w4_planes_rows(a.M, a.N))) return TIQ_EUNSUPPORTED;
+    const bool few = a.M < kGemmMinRows;  // below the documented row count: the workspace is optional
+    if (!digits_rows(a.fmt, a.M, a.N)) return TIQ_EUNSUPPORTED;
     if (!aligned(a.x, 16) || a.ldx % 4 != 0 || a.M * 3 * a.K > 0x7fffffffLL) return TIQ_EUNSUPPORTED;
+    if (digits_supported(a)) {
+        // from kGemmMinRows the documented size covers the planes
+        if (!few && (!ws || ws_bytes < split_workspace(a.M, a.K) || !aligned(ws, 16))) return TIQ_EWORKSPACE;
+        const int rc = launch_digits(a, ws, ws_bytes, gelu_in);
+        return few && rc == TIQ_EWORKSPACE ? TIQ_EUNSUPPORTED : rc;
+    }
+    if (few) return TIQ_EUNSUPPORTED;
     LinearArgs g = a;
     g.x = ws;
     g.x_dtype = TIQ_BF16;
@@ -142,8 +160,7 @@ int run_linear_split(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu_i
     g.kw = a.K;
     const bool staged = staged_gemm_supported(g);
     if (!staged && !gemm_supported(g)) return TIQ_EUNSUPPORTED;
-    if (!ws || ws_bytes < split_workspace(a.M, a.K) || !aligned(ws, 16))
-        return few ? TIQ_EUNSUPPORTED : TIQ_EWORKSPACE;  // with fewer rows the GEMV path takes it
+    if (!ws || ws_bytes < split_workspace(a.M, a.K) || !aligned(ws, 16)) return TIQ_EWORKSPACE;
     const int64_t n = a.M * (a.K / 4);
     hipLaunchKernelGGL(split_bf16x3_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, a.stream,
                        static_cast<const float*>(a.x), a.ldx, (int)a.M, (int)a.K, static_cast<uint16_t*>(ws),
@@ -151,10 +168,6 @@ int run_linear_split(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu_i
     int rc = launch_status();
     if (rc != TIQ_OK) return rc;
     if (!staged) return launch_gemm(g);
-    // a workspace sized by tiq_gemm_w8_workspace also holds split-K partials
-    const size_t planes = split_workspace(a.M, a.K);
-    rc = launch_staged_gemm_split(g, static_cast<uint8_t*>(ws) + planes, ws_bytes - planes);
-    if (rc != TIQ_EUNSUPPORTED) return rc;
     return launch_staged_gemm(g, staged_gemm_choice(g));
 }
 
@@ -172,7 +185,7 @@ int run_linear(const LinearArgs& a) {
 
 using namespace tiq;
 
-extern "C" int tiq_version(void) { return 126; }
+extern "C" int tiq_version(void) { return 127; }
 
 extern "C" const char* tiq_status_string(int status) {
     switch (status) {
@@ -245,7 +258,9 @@ extern "C" int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K
 extern "C" size_t tiq_gemm_w8_workspace(int x_dtype, int64_t M, int64_t K, int64_t N) {
     if ((x_dtype != TIQ_F32 && x_dtype != TIQ_BF16) || K <= 0 || K % 64 != 0 || N <= 0) return 0;
     if (M < kGemmMinRows && !(x_dtype == TIQ_F32 && w4_planes_rows(M, N))) return 0;
-    if (x_dtype == TIQ_F32) return split_workspace(M, K) + staged_split_workspace(M, N, 3 * K);
+    if (x_dtype == TIQ_F32)
+        return std::max(split_workspace(M, K), digits_workspace(M, K)) +
+               std::max(staged_split_workspace(M, N, 3 * K), digits_split_workspace(M, N, K));
     return staged_split_workspace(M, N, K);
 }
 

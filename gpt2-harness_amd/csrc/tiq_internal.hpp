@@ -143,4 +143,14 @@ int launch_gemm_w4g_split(const LinearArgs& a, void* ws, size_t ws_bytes);
 bool staged_w4g_supported(const LinearArgs& a);
 int launch_staged_w4g(const LinearArgs& a, void* ws, size_t ws_bytes);
 
+// fp32 activations with int8 or reference-layout int4 weights on the int8
+// matrix cores (gemm_digits.hip): the rows as four base-256 digit planes in ws
+// (digits_workspace bytes, then the fp32 slices of a product split over K,
+// digits_split_workspace bytes: with less it runs unsplit or in fewer splits).
+// gelu: the product takes gelu_tanh(x). Any M and N, K % 64 == 0.
+size_t digits_workspace(int64_t M, int64_t K);
+size_t digits_split_workspace(int64_t M, int64_t N, int64_t K);
+bool digits_supported(const LinearArgs& a);
+int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu);
+
 }  // namespace tiq

@@ -88,7 +88,7 @@ class QuantLinear(nn.Module):
     def forward_gelu_in(self, x: torch.Tensor) -> torch.Tensor | None:
         """``self(gelu_tanh(x))`` for fp32 GPU rows of a prefill (at least 128
         rows, ``K % 64 == 0``, no gradient wanted), the activation applied
-        while the library splits ``x`` into the matrix cores' bf16 planes
+        while the library splits ``x`` into the matrix cores' planes
         (``tiq_linear_gelu_in_ws``): bit for bit ``self(gelu_tanh(x))``
         without the activation's own pass. None where that entry point does
         not apply; the caller then takes the two steps."""
@@ -140,16 +140,16 @@ def linear_into(m: QuantLinear, x2: torch.Tensor, y: torch.Tensor) -> None:
     st = _lib.stream_of(x2)
     b = _lib.ptr(m.bias)
     if m.fmt == FMT_W8:
-        # fp32 activations over many rows (a prefill) take the matrix cores as
-        # three exact bf16 planes, and a product with few output tiles is split
-        # over K; the library sizes the workspace (0: none)
+        # fp32 activations over many rows (a prefill) take the int8 matrix cores
+        # as digit planes, and a product with few output tiles is split over K;
+        # the library sizes the workspace (0: none)
         ws_bytes = max(int(L.tiq_linear_w8_workspace(xd, M, K)), int(L.tiq_gemm_w8_workspace(xd, M, K, N)))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device) if ws_bytes else None
         rc = L.tiq_linear_w8_ws(x2.data_ptr(), xd, M, K, x2.stride(0), m.codes.data_ptr(), m.scale.data_ptr(), b, N,
                                 y.data_ptr(), yd, y.stride(0), None if ws is None else ws.data_ptr(), ws_bytes, st)
     else:
         # int4 formats: fp32 activations over many rows take the matrix cores
-        # through the same three exact bf16 planes; with bf16 rows a product
+        # too (group-wise as three exact bf16 planes); with bf16 rows a product
         # with few output tiles splits over K (workspace 0: none)
         ws_bytes = max(int(L.tiq_linear_w8_workspace(xd, M, K)), int(L.tiq_gemm_w8_workspace(xd, M, K, N)))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device) if ws_bytes else None

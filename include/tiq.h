@@ -159,12 +159,15 @@ size_t tiq_linear_w8_workspace(int x_dtype, int64_t M, int64_t K);
 
 /* tiq_linear_w8 with a caller workspace -- the same quantized Linear slot
  * (model.py:254,319,352,355), used by the prefill (M = B*T rows) of a model
- * that keeps fp32 activations. With fp32 x and M >= 128 the activations are
- * split exactly into three bf16 planes (x = hi + lo + lo2, written to the
- * workspace) and the product runs on the matrix cores: every product is exact
- * (int8 is exact in bf16), so the result is as accurate as an fp32 GEMM.
- * Other cases behave as tiq_linear_w8. TIQ_EWORKSPACE when the workspace is
- * smaller than tiq_linear_w8_workspace() or not 16-byte aligned. */
+ * that keeps fp32 activations. With fp32 x and M >= 128 each activation row
+ * becomes a fixed-point row of four int8 digit planes under its own power of
+ * two (31 bits below the row's largest element; written to the workspace) and
+ * the product runs on the int8 matrix cores with exact integer sums: more
+ * accurate than an fp32 GEMM. A row holding an infinity or NaN gives NaN
+ * outputs. 65 <= M <= 127 runs so too given a workspace of
+ * tiq_gemm_w8_workspace(TIQ_F32, M, K, N) bytes. Other cases behave as
+ * tiq_linear_w8. TIQ_EWORKSPACE when M >= 128 and the workspace is smaller
+ * than tiq_linear_w8_workspace() or not 16-byte aligned. */
 int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
                      const int8_t* q, const float* scale, const float* bias, int64_t N,
                      void* y, int y_dtype, int64_t ldy, void* workspace, size_t workspace_bytes,
@@ -173,10 +176,10 @@ int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_t l
 /* Workspace bytes with which tiq_gemm_w8_ws (and tiq_linear_w8_ws, and with
  * bf16 activations tiq_linear_w4_ws / tiq_linear_w4g_ws) run a product with
  * few output tiles split over K (fp32 partial slices, summed in a fixed order
- * by a second kernel), plus, for fp32 activations, their bf16 planes. 0 when
+ * by a second kernel), plus, for fp32 activations, their planes. 0 when
  * none is needed. Nonzero from M >= 128, and for fp32 activations also from
  * the fewer rows at which tiq_linear_w4_ws takes the planes (M >= 32, or
- * M >= 16 with N >= 2048; the int8 entry points do not use it there). */
+ * M >= 16 with N >= 2048; tiq_linear_w8_ws takes them from M = 65). */
 size_t tiq_gemm_w8_workspace(int x_dtype, int64_t M, int64_t K, int64_t N);
 /* tiq_gemm_w8 with a caller workspace (see tiq_gemm_w8_workspace): the
  * prefill product of the reference's Linears (model.py:254,319,352,355 at
@@ -230,10 +233,10 @@ int tiq_linear_w4g(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx
 
 /* tiq_linear_w4 / tiq_linear_w4g with a caller workspace of
  * tiq_linear_w8_workspace(x_dtype, M, K) bytes: with fp32 x and M >= 128 the
- * activations are split exactly into three bf16 planes there and the product
- * runs on the matrix cores (every product exact, fp32 accumulation; the
- * group-wise format scales each group's partial sum), as tiq_linear_w8_ws
- * does for int8 -- the prefill of a model quantized to int4 (model.py:254,
+ * product runs on the matrix cores, for reference-layout int4 as
+ * tiq_linear_w8_ws does for int8, for the group-wise format with the
+ * activations split exactly into three bf16 planes (every product exact, fp32
+ * accumulation, each group's partial sum scaled) -- the prefill of a model quantized to int4 (model.py:254,
  * 319,352,355 at M = B*T). With bf16 x, M >= 128 and a workspace of
  * tiq_gemm_w8_workspace(TIQ_BF16, M, K, N) bytes both split a product with few
  * output tiles over K (group-wise: whole groups a split), the fp32 slices
@@ -460,7 +463,7 @@ int tiq_gelu_tanh(const float* x, float* y, int64_t n, void* stream);
 /* A quantized Linear over gelu_tanh of fp32 rows: the MLP's
  * c_proj(gelu_tanh(c_fc(x))) of a prefill (model.py:57-75 and the c_proj
  * slot, model.py:355, at M = B * T rows). The activation is applied while x
- * is split into the three exact bf16 planes the matrix cores take, so y is
+ * is split into the planes the matrix cores take, so y is
  * bit for bit what tiq_linear_w8_ws / tiq_linear_w4_ws / tiq_linear_w4g_ws
  * compute on tiq_gelu_tanh(x), without the activation's own read and write of
  * x. w, w_format (TIQ_WF_INT8, TIQ_WF_INT4, TIQ_WF_INT4_GROUPWISE), scale,
