@@ -185,7 +185,7 @@ int run_linear(const LinearArgs& a) {
 
 using namespace tiq;
 
-extern "C" int tiq_version(void) { return 127; }
+extern "C" int tiq_version(void) { return 128; }
 
 extern "C" const char* tiq_status_string(int status) {
     switch (status) {

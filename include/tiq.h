@@ -442,7 +442,7 @@ int tiq_decode_qkv_attention(const uint16_t* x_planes, int64_t batch, int64_t n_
  * keys (CausalSelfAttention.forward, model.py:284-309, a prompt block or a
  * cached step): query t, at absolute position first + t, attends to keys
  * 0 .. first + t with softmax(q k^T / sqrt(head_dim)) in fp32 (an online
- * softmax over blocks of 64 keys). q (batch, n_head, T, 64), k and v (batch,
+ * softmax over blocks of 32 keys). q (batch, n_head, T, 64), k and v (batch,
  * n_head, S, 64) and y (batch, n_head, T, 64) are addressed through their
  * (batch, head, position) strides in floats with the 64 dims contiguous:
  * the rows of the q, k, v projection, a KV cache's buffers and the (batch,
