@@ -178,12 +178,18 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
 // cover every bank.
 // FMT kW8 (codes) or kW4 (the reference's nibbles, unpacked to 16 (n - 8) on
 // the LDS store: the 16 is taken out with the scale).
+// kW4G (group-wise nibbles, groups of gs k64 steps, an fp16 scale per row and
+// group): a group's four sums, exact integers below 2^29 as two combined pairs,
+// become one fp32 value a result, which times the group's scale is added to
+// fp32 sums -- the lanes of a result register share no column, so a scale is
+// one load a lane and column tile; the next group starts from zero.
 // gridDim.z > 1: split over K, workgroup z writes fp32 slice z of y (no bias).
 template <int WMW, int TM, int TN, int D, int OCC, bool PERSIST, int FMT, typename TY>
 __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
     const uint8_t* __restrict__ xt, const float* __restrict__ rs, const uint8_t* __restrict__ w, int64_t ldw,
     const float* __restrict__ scale, const float* __restrict__ bias, TY* __restrict__ y, int64_t ldy, int M, int N,
-    int K) {
+    int K, const uint16_t* __restrict__ scale16, int ngroups, int gs) {
+    constexpr bool GROUPED = FMT == kW4G;
     static_assert(D >= 2, "register sets");
     constexpr int WNW = 4 / WMW;
     constexpr int MT = TM * WMW, NTL = TN * WNW;  // row and column tiles of the workgroup
@@ -246,7 +252,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
             *reinterpret_cast<u32x4*>(base + q * 4096 + tid * 16) = st[p][q];
         } else {
             u32x4 v = st[p][q];
-            if constexpr (FMT == kW4) {
+            if constexpr (FMT != kW8) {
                 uint32_t e0, o0, e1, o1;
                 nibbles_x16(v.x, e0, o0);
                 nibbles_x16(v.y, e1, o1);
@@ -307,6 +313,31 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
         }
     };
 
+    // group-wise: fp32 sums, the current group's scales (fp16 bits as loaded)
+    float sum[GROUPED ? TN : 1][GROUPED ? TM : 1][16];
+    uint16_t sg[TN];
+    auto load_scales = [&](int g) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+            sg[j] = scale16[(int64_t)min(tn * 32 * NTL + wn * 32 * TN + 32 * j + r, N - 1) * ngroups + g];
+    };
+    auto fold = [&]() {
+        if constexpr (GROUPED) {
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const float sc = f16_bits_to_f32(sg[j]);
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        const float hi = (float)((acc[j][i][3][q] << 8) + acc[j][i][2][q]);
+                        const float lo = (float)((acc[j][i][1][q] << 8) + acc[j][i][0][q]);
+                        sum[j][i][q] = fmaf(fmaf(hi, 65536.f, lo), sc, sum[j][i][q]);
+                    }
+            }
+        }
+    };
+
     const int total = tiles_m * tiles_n;
     begin_tile(blockIdx.x);
     // the workgroup's tiles: one, or every gridDim.x-th of a persistent grid,
@@ -317,15 +348,45 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
         __syncthreads();
 #pragma unroll
         for (int f = 0; f < NRD; ++f) fread(0, 0, 0, f);
-        step(0, 0, true);
-        int s = 1;
-        for (; s + D - 1 < nk; s += D) {
+        if constexpr (GROUPED) {
+            load_scales(s0 / gs);
 #pragma unroll
-            for (int d = 0; d < D; ++d) step(s + d, (1 + d) % D, false);
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) sum[j][i][q] = 0.f;
+            int left = gs - s0 % gs;  // steps to the end of the current group (a split may start inside one)
+            bool fresh = true;
+            auto gstep = [&](int s, int p) {
+                if (fresh) step(s, p, true);
+                else step(s, p, false);
+                fresh = --left == 0;
+                if (fresh || s == nk - 1) {  // the group's (or the split's) last step
+                    fold();
+                    load_scales(min((s0 + s + 1) / gs, ngroups - 1));
+                    left = gs;
+                }
+            };
+            int s = 0;
+            for (; s + D - 1 < nk; s += D) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) gstep(s + d, d);
+            }
+#pragma unroll
+            for (int d = 0; d < D - 1; ++d)
+                if (s + d < nk) gstep(s + d, d);
+        } else {
+            step(0, 0, true);
+            int s = 1;
+            for (; s + D - 1 < nk; s += D) {
+#pragma unroll
+                for (int d = 0; d < D; ++d) step(s + d, (1 + d) % D, false);
+            }
+#pragma unroll
+            for (int d = 0; d < D - 1; ++d)
+                if (s + d < nk) step(s + d, (1 + d) % D, false);
         }
-#pragma unroll
-        for (int d = 0; d < D - 1; ++d)
-            if (s + d < nk) step(s + d, (1 + d) % D, false);
 
         // y = (((a3 256 + a2) 256 + a1) 256 + a0) 2^(e_m - 29) scale + bias; a
         // store instruction writes 32 consecutive outputs of two rows
@@ -336,7 +397,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int n = min(n0 + 32 * j + r, N - 1);
-            sc[j] = scale[n] * unit;
+            sc[j] = GROUPED ? unit : scale[n] * unit;
             bi[j] = bias && !split ? bias[n] : 0.f;
         }
         float4 rm[TM][4];  // rows past M hold whatever the buffer holds: their outputs are not stored
@@ -360,10 +421,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
                     TY* dst = yr + (int64_t)(8 * g + e) * ldy;
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
-                        float f = (float)acc[j][i][3][q];
-                        f = fmaf(f, 256.f, (float)acc[j][i][2][q]);
-                        f = fmaf(f, 256.f, (float)acc[j][i][1][q]);
-                        f = fmaf(f, 256.f, (float)acc[j][i][0][q]);
+                        float f;
+                        if constexpr (GROUPED) {
+                            f = sum[j][i][q];
+                        } else {
+                            f = (float)acc[j][i][3][q];
+                            f = fmaf(f, 256.f, (float)acc[j][i][2][q]);
+                            f = fmaf(f, 256.f, (float)acc[j][i][1][q]);
+                            f = fmaf(f, 256.f, (float)acc[j][i][0][q]);
+                        }
                         const float v = fmaf(f * rmq, sc[j], bi[j]);
                         if (full || (m0 + 32 * i + 8 * g + 4 * h + e < M && n0 + 32 * j + r < N)) {
                             if constexpr (sizeof(TY) == 4) dst[32 * j] = v;
@@ -385,7 +451,8 @@ int run_digits(const LinearArgs& a, const uint8_t* xt, const float* rs, TY* y, i
     const int64_t grid = PERSIST ? std::min<int64_t>(tiles, 256 * OCC) : tiles;
     hipLaunchKernelGGL((gemm_digits_kernel<WMW, TM, TN, D, OCC, PERSIST, FMT, TY>), dim3((unsigned)grid, 1, (unsigned)S),
                        dim3(256), 0, a.stream, xt, rs, a.w, a.ldw, a.scale, a.bias, y, ldy, (int)a.M, (int)a.N,
-                       (int)a.K);
+                       (int)a.K, a.scale16, FMT == kW4G ? (int)((a.K + a.group - 1) / a.group) : 0,
+                       FMT == kW4G ? a.group / 64 : 1);
     return launch_status();
 }
 
@@ -421,7 +488,9 @@ size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 template <int FMT, typename TY>
 int dispatch_digits(const LinearArgs& a, DigitTile tile, const uint8_t* xt, const float* rs, TY* y, int64_t ldy,
                     int64_t S) {
-    switch (tile) {
+    // group-wise: the fp32 sums beside the integer ones fit the small tile
+    if constexpr (FMT == kW4G) return run_digits<1, 1, 1, 3, 2, false, FMT, TY>(a, xt, rs, y, ldy, S);
+    else switch (tile) {
         case kTile64x256: return run_digits<2, 1, 4, 2, 1, false, FMT, TY>(a, xt, rs, y, ldy, S);
         case kTile64x128: return run_digits<2, 1, 2, 2, 2, true, FMT, TY>(a, xt, rs, y, ldy, S);
         default: return run_digits<1, 1, 1, 4, 2, false, FMT, TY>(a, xt, rs, y, ldy, S);
@@ -443,7 +512,7 @@ int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu) 
 
 template <int FMT>
 int run_digits_linear(const LinearArgs& a, uint8_t* xt, float* rs, float* part, int64_t S, bool gelu) {
-    int rc = launch_split_digits<FMT == kW4>(a, xt, rs, gelu);
+    int rc = launch_split_digits<FMT != kW8>(a, xt, rs, gelu);
     if (rc != TIQ_OK) return rc;
     const DigitTile tile = S > 1 ? kTile32x128 : digits_tile(a.M, a.N, a.K);
     if (S > 1) {
@@ -467,7 +536,9 @@ size_t digits_split_workspace(int64_t M, int64_t N, int64_t K) {
 }
 
 bool digits_supported(const LinearArgs& a) {
-    if (a.x_dtype != TIQ_F32 || (a.fmt != kW8 && a.fmt != kW4) || a.kw) return false;
+    if (a.x_dtype != TIQ_F32 || (a.fmt != kW8 && a.fmt != kW4 && a.fmt != kW4G) || a.kw) return false;
+    // group-wise: whole k64 steps a group, rows of whole nibble pairs
+    if (a.fmt == kW4G && (a.group % 64 != 0 || !aligned(a.scale16, 2))) return false;
     // int32 sums: K 2^14 < 2^31
     if (a.K % 64 != 0 || a.K > 65536) return false;
     if (!aligned(a.x, 16) || a.ldx % 4 != 0 || !aligned(a.w, 16) || a.ldw % 16 != 0) return false;
@@ -491,6 +562,7 @@ int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu) {
     if (a.N % 8 != 0 || a.ldy % unit != 0 || !aligned(a.y, 16) || (a.bias && !aligned(a.bias, 16))) S = 1;
     S = std::min<int64_t>(S, (int64_t)((ws_bytes - need) / (size_t)(a.M * a.N * 4)));
     S = std::max<int64_t>(S, 1);
+    if (a.fmt == kW4G) return run_digits_linear<kW4G>(a, xt, rs, part, S, gelu);
     return a.fmt == kW4 ? run_digits_linear<kW4>(a, xt, rs, part, S, gelu)
                         : run_digits_linear<kW8>(a, xt, rs, part, S, gelu);
 }

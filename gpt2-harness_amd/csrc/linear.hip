@@ -57,13 +57,27 @@ namespace {
 // vector-ALU GEMV (below it the GEMM wastes most of each tile).
 constexpr int64_t kGemmMinRows = 128;
 
-// fp32 rows against reference-layout int4 codes take the matrix cores through
-// digit planes (split over K where the tiles are few) from 32 rows, or
-// from 16 on matrices of 2048 rows or more: below 128 rows there is no
-// batched kernel for int4, and the LDS-staged GEMV, four activation rows a
-// tile, grows with M (GPT-2 small shapes at M = 64: 18-57 us against 10-13 us
-// through the planes; int8 has the batched kernel up to 64 rows).
-bool w4_planes_rows(int64_t M, int64_t N) { return M >= 32 || (M >= 16 && N >= 2048); }
+// Rows below kGemmMinRows from which fp32 rows against int4 codes (either
+// layout) have a workspace for digit planes: there is no batched kernel for
+// int4, and the LDS-staged GEMV, four activation rows a tile, grows with M
+// (graph-timed us, GEMV / planes: 768 x 3072 M = 16 18 / 10; 1280 x 5120 M = 8 17
+// / 12; 6400 x 1600 M = 16 29 / 17; but 768 x 768 M = 16 7.3 / 10.3).
+bool w4_planes_rows(int64_t M, int64_t K, int64_t N) {
+    const int64_t work = M * N * K;
+    return M >= 32 || (M >= 16 && (N >= 2048 || work >= 100000000)) || (M >= 8 && N >= 2048 && work >= 25000000);
+}
+
+// bf16 rows below kGemmMinRows that the MFMA GEMM takes when neither the
+// 16-row GEMV nor the batched kernel does (int8 past 64 rows or K past their
+// reach; int4): the alternative is the decode GEMV, four activation rows a
+// tile (us, GEMV / GEMM: int8 1600 x 4800 M = 100 166 / 17, 6400 x 1600 M = 24
+// 35 / 14; int4 768 x 2304 M = 8 12.0 / 9.7, 1024 x 4096 M = 64 85 / 11). Up to 16 rows on
+// matrices under 2048 rows the GEMV's direct kernel is ahead (3072 x 768 M = 16
+// 6.8 / 12) until the product is large (6400 x 1600 M = 16 30 / 16).
+bool bf16_gemm_rows(int64_t M, int64_t K, int64_t N) {
+    const int64_t work = M * N * K;
+    return M >= kGemmMinRows || M > 64 || (M > 16 || N >= 2048 ? work >= 14000000 : work >= 100000000);
+}
 
 LinearArgs make_args(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w, int64_t ldw,
                      const float* scale, const uint16_t* scale16, int group, const float* bias, int64_t N, void* y,
@@ -127,12 +141,18 @@ __global__ void split_bf16x3_kernel(const float* __restrict__ x, int64_t ldx, in
 
 size_t split_workspace(int64_t M, int64_t K) { return (size_t)(M * 3 * K * 2 + 255) / 256 * 256; }
 
-// Rows at and above which fp32 activations take the int8 matrix cores (digit
-// planes): int8 has the batched kernel up to 64 rows; from 65 the decode GEMV,
-// four activation rows a tile, was the only other one below kGemmMinRows (77
-// rows, 768 x 3072: 56 us against 11 us). int4 as w4_planes_rows.
-bool digits_rows(WFormat fmt, int64_t M, int64_t N) {
-    return M >= kGemmMinRows || (fmt == kW8 ? M > 64 : fmt == kW4 && w4_planes_rows(M, N));
+// fp32 rows that take the int8 matrix cores as digit planes, given a workspace.
+// int8 has the batched kernel up to 64 rows, which holds a wavefront's whole
+// share of K and reads every activation plane for each 32-row tile: past 32
+// rows of a long K the planes win (us, batched / planes: 1600 x 4800 M = 64 21 /
+// 15, 6400 x 1600 M = 32 32 / 20; 768 x 3072 M = 64 7.5 / 10.7); from 65 rows the
+// only other kernel is the decode GEMV (77 rows, 768 x 3072: 56 / 11). int4 as
+// w4_planes_rows, group-wise also only from the size at which its GEMV falls
+// behind (768 x 768: M = 32 10.9 / 14.2, M = 48 16.4 / 14.4).
+bool digits_rows(WFormat fmt, int64_t M, int64_t K, int64_t N) {
+    if (M >= kGemmMinRows) return true;
+    if (fmt == kW8) return M > 64 || (M > 32 && K >= 1536) || (M == 32 && K >= 3072);
+    return w4_planes_rows(M, K, N) && (fmt == kW4 || M * N * K >= 24000000);
 }
 
 // fp32 activations through the matrix cores: int8 and reference-layout int4
@@ -143,7 +163,7 @@ bool digits_rows(WFormat fmt, int64_t M, int64_t N) {
 int run_linear_split(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu_in = false) {
     if (a.x_dtype != TIQ_F32 || a.fmt == kF32 || a.K % 4 != 0) return TIQ_EUNSUPPORTED;
     const bool few = a.M < kGemmMinRows;  // below the documented row count: the workspace is optional
-    if (!digits_rows(a.fmt, a.M, a.N)) return TIQ_EUNSUPPORTED;
+    if (!digits_rows(a.fmt, a.M, a.K, a.N)) return TIQ_EUNSUPPORTED;
     if (!aligned(a.x, 16) || a.ldx % 4 != 0 || a.M * 3 * a.K > 0x7fffffffLL) return TIQ_EUNSUPPORTED;
     if (digits_supported(a)) {
         // from kGemmMinRows the documented size covers the planes
@@ -176,8 +196,13 @@ int run_linear(const LinearArgs& a) {
     if (rc != TIQ_OK || a.M == 0 || a.N == 0) return rc;
     if (rows16_preferred(a)) return launch_rows16(a);
     if (skinny_supported(a)) return launch_skinny(a);
-    if (a.M >= kGemmMinRows && gemm_supported(a)) return launch_gemm(a);
+    if (bf16_gemm_rows(a.M, a.K, a.N) && gemm_supported(a)) return launch_gemm(a);
     return launch_gemv(a);
+}
+
+// bf16 rows of the workspace entry points that split a GEMM over K when planned
+bool bf16_split_rows(const LinearArgs& a) {
+    return a.x_dtype == TIQ_BF16 && bf16_gemm_rows(a.M, a.K, a.N) && !rows16_preferred(a) && !skinny_supported(a);
 }
 
 }  // namespace
@@ -185,7 +210,7 @@ int run_linear(const LinearArgs& a) {
 
 using namespace tiq;
 
-extern "C" int tiq_version(void) { return 128; }
+extern "C" int tiq_version(void) { return 130; }
 
 extern "C" const char* tiq_status_string(int status) {
     switch (status) {
@@ -248,7 +273,7 @@ extern "C" int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K
     if (rc != TIQ_OK || M == 0 || N == 0) return rc;
     rc = run_linear_split(a, workspace, workspace_bytes);
     if (rc != TIQ_EUNSUPPORTED) return rc;
-    if (a.x_dtype == TIQ_BF16 && M >= kGemmMinRows) {  // bf16 rows: split-K when planned
+    if (bf16_split_rows(a)) {
         rc = launch_staged_gemm_split(a, workspace, workspace_bytes);
         if (rc != TIQ_EUNSUPPORTED) return rc;
     }
@@ -257,10 +282,23 @@ extern "C" int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K
 
 extern "C" size_t tiq_gemm_w8_workspace(int x_dtype, int64_t M, int64_t K, int64_t N) {
     if ((x_dtype != TIQ_F32 && x_dtype != TIQ_BF16) || K <= 0 || K % 64 != 0 || N <= 0) return 0;
-    if (M < kGemmMinRows && !(x_dtype == TIQ_F32 && w4_planes_rows(M, N))) return 0;
+    if (!(x_dtype == TIQ_F32 ? M >= kGemmMinRows || w4_planes_rows(M, K, N) : bf16_gemm_rows(M, K, N))) return 0;
     if (x_dtype == TIQ_F32)
         return std::max(split_workspace(M, K), digits_workspace(M, K)) +
                std::max(staged_split_workspace(M, N, 3 * K), digits_split_workspace(M, N, K));
+    return staged_split_workspace(M, N, K);
+}
+
+extern "C" size_t tiq_linear_workspace(int w_format, int x_dtype, int64_t M, int64_t K, int64_t N) {
+    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT4 && w_format != TIQ_WF_INT4_GROUPWISE) return 0;
+    if (M <= 4 || K <= 0 || N <= 0 || K % 64 != 0) return 0;
+    if (x_dtype == TIQ_F32)
+        return digits_rows((WFormat)w_format, M, K, N) ? tiq_gemm_w8_workspace(TIQ_F32, M, K, N) : 0;
+    if (x_dtype != TIQ_BF16 || !bf16_gemm_rows(M, K, N)) return 0;
+    // int8 rows of the 16-row GEMV and the batched kernel need none; nor does a
+    // product that launch_staged_gemm_split leaves whole
+    if (w_format == TIQ_WF_INT8 && (M <= 16 || (M <= 64 && K <= 3072))) return 0;
+    if (w_format != TIQ_WF_INT4_GROUPWISE && ((M + 127) / 128) * ((N + 127) / 128) >= 48 && K / 64 <= 32) return 0;
     return staged_split_workspace(M, N, K);
 }
 
@@ -401,7 +439,7 @@ extern "C" int tiq_linear_w4_ws(const void* x, int x_dtype, int64_t M, int64_t K
     if (workspace && !aligned(workspace, 16)) return TIQ_EALIGN;
     rc = run_linear_split(a, workspace, workspace_bytes);
     if (rc != TIQ_EUNSUPPORTED) return rc;
-    if (x_dtype == TIQ_BF16 && M >= kGemmMinRows) {  // bf16 rows: split over K when planned
+    if (bf16_split_rows(a)) {
         rc = launch_staged_gemm_split(a, workspace, workspace_bytes);
         if (rc != TIQ_EUNSUPPORTED) return rc;
     }
@@ -419,7 +457,7 @@ extern "C" int tiq_linear_w4g_ws(const void* x, int x_dtype, int64_t M, int64_t 
     if (workspace && !aligned(workspace, 16)) return TIQ_EALIGN;
     rc = run_linear_split(a, workspace, workspace_bytes);
     if (rc != TIQ_EUNSUPPORTED) return rc;
-    if (x_dtype == TIQ_BF16 && M >= kGemmMinRows) {  // bf16 rows: split over K when planned
+    if (bf16_split_rows(a)) {
         rc = launch_staged_w4g(a, workspace, workspace_bytes);
         if (rc != TIQ_EUNSUPPORTED) return rc;
         rc = launch_gemm_w4g_split(a, workspace, workspace_bytes);

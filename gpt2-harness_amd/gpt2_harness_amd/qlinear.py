@@ -23,6 +23,7 @@ import torch.nn as nn
 from . import _lib
 
 FMT_W8, FMT_W4, FMT_W4G = "int8", "int4", "int4_groupwise"
+_WF = {FMT_W8: _lib.WF_INT8, FMT_W4: _lib.WF_INT4, FMT_W4G: _lib.WF_INT4G}
 
 
 class QuantLinear(nn.Module):
@@ -107,7 +108,7 @@ class QuantLinear(nn.Module):
         y = torch.empty((M, N), dtype=torch.float32, device=x.device)
         ws_bytes = int(L.tiq_gemm_w8_workspace(_lib.dtype_code(torch.float32), M, K, N))
         ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-        wf = {FMT_W8: _lib.WF_INT8, FMT_W4: _lib.WF_INT4}.get(self.fmt, _lib.WF_INT4G)
+        wf = _WF[self.fmt]
         s32 = None if self.fmt == FMT_W4G else self.scale.data_ptr()
         s16 = self.scale.data_ptr() if self.fmt == FMT_W4G else None
         rc = L.tiq_linear_gelu_in_ws(x2.data_ptr(), M, K, K, self.codes.data_ptr(), wf, s32, s16, self.group_size,
@@ -139,27 +140,21 @@ def linear_into(m: QuantLinear, x2: torch.Tensor, y: torch.Tensor) -> None:
     xd, yd = _lib.dtype_code(x2.dtype), _lib.dtype_code(y.dtype)
     st = _lib.stream_of(x2)
     b = _lib.ptr(m.bias)
+    # fp32 activations over many rows (a prefill) take the int8 matrix cores as
+    # digit planes, and a product with few output tiles is split over K; the
+    # library sizes the workspace (0: none)
+    ws_bytes = L.tiq_linear_workspace(_WF[m.fmt], xd, M, K, N)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device) if ws_bytes else None
+    wp = None if ws is None else ws.data_ptr()
     if m.fmt == FMT_W8:
-        # fp32 activations over many rows (a prefill) take the int8 matrix cores
-        # as digit planes, and a product with few output tiles is split over K;
-        # the library sizes the workspace (0: none)
-        ws_bytes = max(int(L.tiq_linear_w8_workspace(xd, M, K)), int(L.tiq_gemm_w8_workspace(xd, M, K, N)))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device) if ws_bytes else None
         rc = L.tiq_linear_w8_ws(x2.data_ptr(), xd, M, K, x2.stride(0), m.codes.data_ptr(), m.scale.data_ptr(), b, N,
-                                y.data_ptr(), yd, y.stride(0), None if ws is None else ws.data_ptr(), ws_bytes, st)
+                                y.data_ptr(), yd, y.stride(0), wp, ws_bytes, st)
+    elif m.fmt == FMT_W4:
+        rc = L.tiq_linear_w4_ws(x2.data_ptr(), xd, M, K, x2.stride(0), m.codes.data_ptr(), m.scale.data_ptr(), b, N,
+                                y.data_ptr(), yd, y.stride(0), wp, ws_bytes, st)
     else:
-        # int4 formats: fp32 activations over many rows take the matrix cores
-        # too (group-wise as three exact bf16 planes); with bf16 rows a product
-        # with few output tiles splits over K (workspace 0: none)
-        ws_bytes = max(int(L.tiq_linear_w8_workspace(xd, M, K)), int(L.tiq_gemm_w8_workspace(xd, M, K, N)))
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device) if ws_bytes else None
-        wp = None if ws is None else ws.data_ptr()
-        if m.fmt == FMT_W4:
-            rc = L.tiq_linear_w4_ws(x2.data_ptr(), xd, M, K, x2.stride(0), m.codes.data_ptr(), m.scale.data_ptr(), b,
-                                    N, y.data_ptr(), yd, y.stride(0), wp, ws_bytes, st)
-        else:
-            rc = L.tiq_linear_w4g_ws(x2.data_ptr(), xd, M, K, x2.stride(0), m.codes.data_ptr(), m.scale.data_ptr(),
-                                     m.group_size, b, N, y.data_ptr(), yd, y.stride(0), wp, ws_bytes, st)
+        rc = L.tiq_linear_w4g_ws(x2.data_ptr(), xd, M, K, x2.stride(0), m.codes.data_ptr(), m.scale.data_ptr(),
+                                 m.group_size, b, N, y.data_ptr(), yd, y.stride(0), wp, ws_bytes, st)
     _lib.check(rc, f"quantized linear ({m.fmt}, M={M}, K={K}, N={N})")
 
 

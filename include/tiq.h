@@ -164,8 +164,8 @@ size_t tiq_linear_w8_workspace(int x_dtype, int64_t M, int64_t K);
  * two (31 bits below the row's largest element; written to the workspace) and
  * the product runs on the int8 matrix cores with exact integer sums: more
  * accurate than an fp32 GEMM. A row holding an infinity or NaN gives NaN
- * outputs. 65 <= M <= 127 runs so too given a workspace of
- * tiq_gemm_w8_workspace(TIQ_F32, M, K, N) bytes. Other cases behave as
+ * outputs. 65 <= M <= 127, and M >= 32 with a long K, run so too given a
+ * workspace of tiq_gemm_w8_workspace(TIQ_F32, M, K, N) bytes. Other cases behave as
  * tiq_linear_w8. TIQ_EWORKSPACE when M >= 128 and the workspace is smaller
  * than tiq_linear_w8_workspace() or not 16-byte aligned. */
 int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,
@@ -177,10 +177,17 @@ int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_t l
  * bf16 activations tiq_linear_w4_ws / tiq_linear_w4g_ws) run a product with
  * few output tiles split over K (fp32 partial slices, summed in a fixed order
  * by a second kernel), plus, for fp32 activations, their planes. 0 when
- * none is needed. Nonzero from M >= 128, and for fp32 activations also from
- * the fewer rows at which tiq_linear_w4_ws takes the planes (M >= 32, or
- * M >= 16 with N >= 2048; tiq_linear_w8_ws takes them from M = 65). */
+ * none is needed. Nonzero from M >= 128, and from the fewer rows at which the
+ * workspace entry points use it: fp32 activations M >= 32, or M >= 16 with
+ * N >= 2048 or a large product, or M >= 8 with both; bf16 activations the rows
+ * that take the GEMM and plan a split. */
 size_t tiq_gemm_w8_workspace(int x_dtype, int64_t M, int64_t K, int64_t N);
+/* Workspace bytes with which the workspace entry point of a weight format
+ * (tiq_linear_w8_ws, tiq_linear_w4_ws, tiq_linear_w4g_ws) runs this product
+ * at its best, 0 where it uses none: one query for the module slot
+ * (model.py:254,319,352,355). w_format TIQ_WF_INT8, TIQ_WF_INT4 or
+ * TIQ_WF_INT4_GROUPWISE. */
+size_t tiq_linear_workspace(int w_format, int x_dtype, int64_t M, int64_t K, int64_t N);
 /* tiq_gemm_w8 with a caller workspace (see tiq_gemm_w8_workspace): the
  * prefill product of the reference's Linears (model.py:254,319,352,355 at
  * M = B * T) on the matrix cores; without enough workspace it runs unsplit,
@@ -233,18 +240,16 @@ int tiq_linear_w4g(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx
 
 /* tiq_linear_w4 / tiq_linear_w4g with a caller workspace of
  * tiq_linear_w8_workspace(x_dtype, M, K) bytes: with fp32 x and M >= 128 the
- * product runs on the matrix cores, for reference-layout int4 as
- * tiq_linear_w8_ws does for int8, for the group-wise format with the
- * activations split exactly into three bf16 planes (every product exact, fp32
- * accumulation, each group's partial sum scaled) -- the prefill of a model quantized to int4 (model.py:254,
+ * product runs on the int8 matrix cores as tiq_linear_w8_ws does for int8 (the
+ * group-wise format: exact sums a group, each scaled and added in fp32; groups
+ * of a multiple of 64 columns) -- the prefill of a model quantized to int4 (model.py:254,
  * 319,352,355 at M = B*T). With bf16 x, M >= 128 and a workspace of
  * tiq_gemm_w8_workspace(TIQ_BF16, M, K, N) bytes both split a product with few
  * output tiles over K (group-wise: whole groups a split), the fp32 slices
- * summed in a fixed order. Reference-layout int4 (tiq_linear_w4_ws) with fp32
- * x takes the planes from fewer rows too -- M >= 32, or M >= 16 with
- * N >= 2048 -- given a workspace of tiq_gemm_w8_workspace(TIQ_F32, M, K, N)
- * bytes (planes, then the fp32 slices of a product split over K); with a
- * smaller one such a call computes what tiq_linear_w4 computes. Where the
+ * summed in a fixed order. Fewer fp32 rows take the planes too where
+ * tiq_gemm_w8_workspace(TIQ_F32, M, K, N) gives a size for them (planes, then
+ * the fp32 slices of a product split over K); with a smaller workspace such a
+ * call computes what tiq_linear_w4 / tiq_linear_w4g compute. Where the
  * GEMM does not take the shape (K % 64, group % 64), and for bf16 x or
  * M < 128 without a workspace, they compute what tiq_linear_w4 /
  * tiq_linear_w4g compute. With fp32 x, M >= 128 and a

@@ -74,6 +74,42 @@ def test_digit_planes(dev, K, N, M, bits):
     assert torch.equal(yb, y.bfloat16())
 
 
+# group-wise int4: groups of one k64 step to the whole row, ragged last groups,
+# splits that start inside a group; the bound gains a rounding of the running
+# sum a group
+@pytest.mark.parametrize("K,N,M,group", [(64, 128, 128, 64), (1600, 1212, 128, 128), (768, 772, 140, 192),
+                                         (3072, 768, 65, 128), (3072, 264, 200, 1024), (1600, 2049, 300, 128),
+                                         (6400, 96, 70, 320), (2048, 2304, 17, 64), (6400, 1600, 129, 6400)])
+def test_digit_planes_groupwise(dev, K, N, M, group):
+    gen = torch.Generator(device=dev).manual_seed(K + N + M)
+    lin = torch.nn.Linear(K, N, device=dev)
+    lin.weight.data = torch.randn(N, K, generator=gen, device=dev) * 0.02
+    mod = g.quantize_linear(lin, 4, group_size=group)[0]
+    x = torch.randn(M, K, generator=gen, device=dev)
+    x[:, ::97] *= 20.0
+    y = torch.full((M, N), float("nan"), device=dev)
+    L = _lib.lib()
+    n_ws = int(L.tiq_gemm_w8_workspace(_lib.F32, M, K, N))
+    ws = torch.empty(max(n_ws, 16), dtype=torch.uint8, device=dev)
+    for out in (y, yb := torch.empty(M, N, device=dev, dtype=torch.bfloat16)):
+        _lib.check(L.tiq_linear_w4g_ws(x.data_ptr(), _lib.F32, M, K, K, mod.codes.data_ptr(), mod.scale.data_ptr(),
+                                       group, _lib.ptr(mod.bias), N, out.data_ptr(), _lib.dtype_code(out.dtype), N,
+                                       ws.data_ptr(), n_ws, torch.cuda.current_stream().cuda_stream), "linear")
+    torch.cuda.synchronize()
+    q = g.unpack_int4(mod.codes, N * K).view(N, K)
+    s = mod.scale.double().repeat_interleave(group, dim=1)[:, :K]
+    w = q.double() * s
+    ref = x.double() @ w.t() + mod.bias.double()
+    top = x.abs().amax(1, keepdim=True).double()
+    u, groups = 2.0**-24, -(-K // group)
+    one = w.abs().sum(1)
+    bound = (top * 2.0**-30 * one * 2 + 3 * u * top * 2.0**-29 * 257 * K * 2**14 * s.amax(1)
+             + (groups + 1) * u * (x.double().abs() @ w.abs().t()) + 8 * u * (ref.abs() + mod.bias.double().abs()))
+    err = (y.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+    assert torch.equal(yb, y.bfloat16())
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 def test_digit_planes_strided(dev, bits):
     K, N, M = 768, 772, 140
