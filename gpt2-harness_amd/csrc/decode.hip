@@ -786,7 +786,8 @@ extern "C" int tiq_decode_qkv_attention(const uint16_t* x_planes, int64_t batch,
                                         int64_t t_max, const int64_t* pos, float* y, int64_t ldy,
                                         uint16_t* planes_out, void* workspace, size_t workspace_bytes,
                                         void* stream) {
-    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED) return TIQ_EUNSUPPORTED;
+    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED && w_format != TIQ_WF_INT4_TILED)
+        return TIQ_EUNSUPPORTED;
     if (batch < 0 || n_embd <= 0 || n_head <= 0 || n_kv_head <= 0 || n_head % n_kv_head) return TIQ_EINVAL;
     if (batch == 0) return TIQ_OK;
     if (!x_planes || !w || !scale || !k_cache || !v_cache || !pos || !y) return TIQ_EINVAL;
@@ -800,7 +801,7 @@ extern "C" int tiq_decode_qkv_attention(const uint16_t* x_planes, int64_t batch,
     if (need == 0) return TIQ_EUNSUPPORTED;  // K beyond the product's splits
     if (!workspace || workspace_bytes < need) return TIQ_EWORKSPACE;
     if (!aligned(workspace, 16)) return TIQ_EALIGN;
-    const WFormat fmt = w_format == TIQ_WF_INT8_TILED ? kW8T : kW8;
+    const WFormat fmt = (WFormat)w_format;
     LinearArgs a{};
     a.x_dtype = TIQ_F32;
     a.M = batch;

@@ -73,25 +73,6 @@ __device__ __forceinline__ void staged_tile_of(int i, int& tm, int& tn, int tile
     tn = in / gm;
 }
 
-// Nibbles as bf16 times 16: d holds 8 biased nibbles (column 2j in the low
-// nibble of byte j, code n - 8); e (even columns) and o (odd columns) get
-// each nibble in the high half of a byte with its top bit flipped, which as
-// a signed byte is 16 (n - 8). A byte becomes a float in one instruction
-// (sub-dword operand select with sign extension), and 16 (n - 8) is exact in
-// bf16; the factor 16 is taken out in the epilogue (an exact power of two:
-// every partial sum is 16 times the unscaled one, rounded the same way).
-__device__ __forceinline__ void nibbles_x16(uint32_t d, uint32_t& e, uint32_t& o) {
-    e = ((d << 4) & 0xf0f0f0f0u) ^ 0x80808080u;
-    o = (d & 0xf0f0f0f0u) ^ 0x80808080u;
-}
-
-// byte k of e and o -> two bf16 in one dword (even column low)
-__device__ __forceinline__ uint32_t bf16x2_of_x16(uint32_t e, uint32_t o, int k) {
-    const float lo = (float)(int8_t)(e >> (8 * k));
-    const float hi = (float)(int8_t)(o >> (8 * k));
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-
 // FMT: kW8 (int8 codes) or kW4 (the reference's nibbles), per-row scale.
 // Nibble rows are staged 8 bytes a thread per k64 step into the same bf16
 // LDS layout as int8 rows.

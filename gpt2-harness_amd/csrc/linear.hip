@@ -210,7 +210,7 @@ bool bf16_split_rows(const LinearArgs& a) {
 
 using namespace tiq;
 
-extern "C" int tiq_version(void) { return 130; }
+extern "C" int tiq_version(void) { return 131; }
 
 extern "C" const char* tiq_status_string(int status) {
     switch (status) {
@@ -475,7 +475,8 @@ extern "C" int tiq_linear_w4g(const void* x, int x_dtype, int64_t M, int64_t K, 
 
 extern "C" size_t tiq_decode_linear_workspace(int w_format, int64_t M, int64_t K, int64_t N) {
     if (w_format == TIQ_WF_F32_TILED) return 0;  // planes in only: nothing staged
-    if ((w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED && w_format != TIQ_WF_F32) ||
+    if ((w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED && w_format != TIQ_WF_INT4_TILED &&
+         w_format != TIQ_WF_F32) ||
         M < kSkinnyMinRows || M > 64 || K <= 0 ||
         K % 32 != 0 || N <= 0)
         return 0;
@@ -485,6 +486,10 @@ extern "C" size_t tiq_decode_linear_workspace(int w_format, int64_t M, int64_t K
 extern "C" int tiq_tile_int8(const int8_t* w, int64_t N, int64_t K, int64_t ldw, int8_t* tiles, void* stream) {
     return launch_tile_int8(reinterpret_cast<const uint8_t*>(w), N, K, ldw, reinterpret_cast<uint8_t*>(tiles),
                             as_stream(stream));
+}
+
+extern "C" int tiq_tile_int4(const uint8_t* w, int64_t N, int64_t K, uint8_t* tiles, void* stream) {
+    return launch_tile_int4(w, N, K, tiles, as_stream(stream));
 }
 
 extern "C" size_t tiq_tile_f32_bytes(int64_t N, int64_t K) { return tile_f32_bytes(N, K); }
@@ -554,8 +559,8 @@ extern "C" int tiq_decode_linear(const float* x, int64_t ldx, const uint16_t* x_
                                  int activation, const float* residual, int64_t ld_residual,
                                  const float* next_ln_weight, const float* next_ln_bias, float next_ln_eps,
                                  uint16_t* planes_out, void* workspace, size_t workspace_bytes, void* stream) {
-    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED && w_format != TIQ_WF_F32 &&
-        w_format != TIQ_WF_F32_TILED)
+    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED && w_format != TIQ_WF_INT4_TILED &&
+        w_format != TIQ_WF_F32 && w_format != TIQ_WF_F32_TILED)
         return TIQ_EUNSUPPORTED;
     if (activation != TIQ_ACT_NONE && activation != TIQ_ACT_GELU_TANH) return TIQ_EINVAL;
     if ((ln_weight == nullptr) != (ln_bias == nullptr)) return TIQ_EINVAL;

@@ -35,13 +35,36 @@ typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 8;
 // Units (32 K each) a wavefront holds in registers: all of its share of K.
 // int8: 25 units (K <= 8 * 25 * 32 = 6400); fp32 weights (4x the bytes): 8.
-// int8 codes, row-major or in operand tiles
+// integer codes: int8, row-major or in operand tiles, or nibbles in operand tiles
 template <int WF>
-constexpr bool is_w8() { return WF == kW8 || WF == kW8T; }
+constexpr bool is_w8() { return WF == kW8 || WF == kW8T || WF == kW4T; }
+// the registers of one unit's codes (16 columns a lane), and its 8 columns e
+// (0: the first 8, 1: the last) as an MFMA operand: exact in bf16, nibbles as
+// 16 (n - 8) -- the sums are scaled by code_unit, an exact power of two
+template <int WF>
+struct CodeReg { typedef u32x4 type; };
+template <>
+struct CodeReg<kW4T> { typedef u32x2 type; };
+template <int WF>
+constexpr float code_unit() { return WF == kW4T ? 0.0625f : 1.f; }
+__device__ __forceinline__ bf16x8 code_frag(const u32x4& d, int e) {
+    const uint32_t s0 = e == 0 ? d.x : d.z, s1 = e == 0 ? d.y : d.w;
+    const u32x4 wq = {bf16x2_of_bytes_perm(s0, 0), bf16x2_of_bytes_perm(s0, 16), bf16x2_of_bytes_perm(s1, 0),
+                      bf16x2_of_bytes_perm(s1, 16)};
+    return __builtin_bit_cast(bf16x8, wq);
+}
+__device__ __forceinline__ bf16x8 code_frag(const u32x2& d, int e) {
+    uint32_t ev, od;
+    nibbles_x16(e == 0 ? d.x : d.y, ev, od);
+    const u32x4 wq = {bf16x2_of_x16(ev, od, 0), bf16x2_of_x16(ev, od, 1), bf16x2_of_x16(ev, od, 2),
+                      bf16x2_of_x16(ev, od, 3)};
+    return __builtin_bit_cast(bf16x8, wq);
+}
 template <int WF>
 constexpr int max_units() { return is_w8<WF>() ? 25 : 8; }
 // activation units in flight per wavefront (ring): 4, 3 with fp32 weights
@@ -71,12 +94,6 @@ __device__ __forceinline__ void split3(const float (&v)[8], bf16x8& p0, bf16x8& 
     p0 = __builtin_bit_cast(bf16x8, a);
     p1 = __builtin_bit_cast(bf16x8, b);
     p2 = __builtin_bit_cast(bf16x8, c);
-}
-
-__device__ __forceinline__ uint32_t bf16x2_of_bytes(uint32_t d, int sh) {
-    const float lo = (float)((int32_t)(d << (24 - sh)) >> 24);
-    const float hi = (float)((int32_t)(d << (16 - sh)) >> 24);
-    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 
 template <typename TY>
@@ -331,7 +348,9 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
     const float* res, int64_t ldr, float* __restrict__ part, uint16_t* __restrict__ x3o) {
     // y may alias res (x = x + f(x) in place): neither is __restrict__
     constexpr bool W8 = is_w8<WF>();
-    constexpr int WB = W8 ? 16 : 64;  // weight bytes a lane loads per unit
+    constexpr int WB = WF == kW4T ? 8 : W8 ? 16 : 64;  // weight bytes a lane loads per unit
+    constexpr int WR = W8 ? 1 : 4;                     // their registers
+    typedef typename CodeReg<WF>::type WReg;
     constexpr bool PL = XM == kXPlanes;
     constexpr int kXp = ring_units<WF>();
     __shared__ float red[kWaves][32][33];      // partial output tiles, rows padded
@@ -354,7 +373,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
     const uint16_t* x3t = reinterpret_cast<const uint16_t*>(x) + (int64_t)blockIdx.y * (K / 32) * 6 * 64 * 8 + lane * 8;
     // row-major: row n0 + r, + 2 WB u per unit; tiles: this row tile's 1 KB
     // blocks (N % 32 == 0, the host checks), + 1024 u per unit
-    const uint8_t* wr = WF == kW8T ? w + (int64_t)blockIdx.x * U * 1024 + lane * 16
+    const uint8_t* wr = WF == kW8T || WF == kW4T
+                            ? w + ((int64_t)blockIdx.x * U * 64 + lane) * WB
                                    : w + (int64_t)min(n0 + r, N - 1) * ldw + WB * h;
 
     const int cnt = u1 - u0;  // <= kUnits (the host checks K)
@@ -362,18 +382,18 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
     // every weight slice of the wavefront is requested first, so the whole
     // matrix is in flight at once (behind the LayerNorm statistics);
     // activations (L2 hits) follow through a ring of kXp unit registers
-    u32x4 wreg[kUnits][WB / 16];
+    WReg wreg[kUnits][WR];
 #pragma unroll
     for (int c = 0; c < kUnits; ++c)
         if (c < cnt) {
-            if constexpr (WF == kW8T) {
-                // 1 KB of consecutive memory per load instruction, read once:
+            if constexpr (WF == kW8T || WF == kW4T) {
+                // 1 KB (nibbles: 512 bytes) of consecutive memory per load instruction, read once:
                 // nontemporal (1.5-1.9 us less per launch on a 7.7-10 MB
                 // matrix than row-major codes with the default policy)
-                wreg[c][0] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wr + (int64_t)(u0 + c) * 1024));
+                wreg[c][0] = __builtin_nontemporal_load(reinterpret_cast<const WReg*>(wr + (int64_t)(u0 + c) * 64 * WB));
             } else {
 #pragma unroll
-                for (int q = 0; q < WB / 16; ++q)
+                for (int q = 0; q < WR; ++q)
                     wreg[c][q] = *reinterpret_cast<const u32x4*>(wr + 2 * WB * (u0 + c) + 16 * q);
             }
         }
@@ -458,7 +478,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
 
     // compute one unit: activations v (16 fp32 of row r, K = 32 u + 16 h + 0..15)
     // and the weight registers of the same K
-    auto unit = [&](int u, const float (&xv)[16], const u32x4 (&wv)[WB / 16]) {
+    auto unit = [&](int u, const float (&xv)[16], const WReg (&wv)[WR]) {
         const int k0 = 32 * u + 16 * h;
         float v[16];
 #pragma unroll
@@ -482,11 +502,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
             bf16x8 x0, x1, x2;
             split3(ve, x0, x1, x2);
             if constexpr (W8) {
-                const u32x4 d = wv[0];
-                const uint32_t s0 = e == 0 ? d.x : d.z, s1 = e == 0 ? d.y : d.w;
-                const u32x4 wq = {bf16x2_of_bytes(s0, 0), bf16x2_of_bytes(s0, 16), bf16x2_of_bytes(s1, 0),
-                                  bf16x2_of_bytes(s1, 16)};
-                const bf16x8 wf = __builtin_bit_cast(bf16x8, wq);
+                const bf16x8 wf = code_frag(wv[0], e);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, x0, acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, x1, acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, x2, acc, 0, 0, 0);
@@ -506,7 +522,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
         }
     };
     // plane mode: the 6 operand registers of a unit come straight from x3
-    auto unit_pl = [&](const u32x4 (&xv)[3][2], const u32x4 (&wv)[WB / 16]) {
+    auto unit_pl = [&](const u32x4 (&xv)[3][2], const WReg (&wv)[WR]) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             bf16x8 xq[3];
@@ -517,11 +533,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
                 xq[q] = __builtin_bit_cast(bf16x8, t);
             }
             if constexpr (W8) {
-                const u32x4 d = wv[0];
-                const uint32_t s0 = e == 0 ? d.x : d.z, s1 = e == 0 ? d.y : d.w;
-                const u32x4 wq = {bf16x2_of_bytes(s0, 0), bf16x2_of_bytes(s0, 16), bf16x2_of_bytes(s1, 0),
-                                  bf16x2_of_bytes(s1, 16)};
-                const bf16x8 wf = __builtin_bit_cast(bf16x8, wq);
+                const bf16x8 wf = code_frag(wv[0], e);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xq[0], acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xq[1], acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xq[2], acc, 0, 0, 0);
@@ -563,16 +575,12 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
         xv[0] = *reinterpret_cast<const u32x4*>(xbr + 32 * u);
         xv[1] = *reinterpret_cast<const u32x4*>(xbr + 32 * u + 8);
     };
-    auto unit_bf = [&](const u32x4 (&xv)[2], const u32x4 (&wv)[WB / 16]) {
+    auto unit_bf = [&](const u32x4 (&xv)[2], const WReg (&wv)[WR]) {
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const u32x4 t = xrow_ok ? xv[e] : u32x4{0u, 0u, 0u, 0u};
-            const u32x4 d = wv[0];
-            const uint32_t s0 = e == 0 ? d.x : d.z, s1 = e == 0 ? d.y : d.w;
-            const u32x4 wq = {bf16x2_of_bytes(s0, 0), bf16x2_of_bytes(s0, 16), bf16x2_of_bytes(s1, 0),
-                              bf16x2_of_bytes(s1, 16)};
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, wq),
-                                                          __builtin_bit_cast(bf16x8, t), acc, 0, 0, 0);
+                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(code_frag(wv[0], e), __builtin_bit_cast(bf16x8, t), acc, 0, 0,
+                                                          0);
         }
     };
 
@@ -639,6 +647,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
             float t = 0.f;
 #pragma unroll
             for (int w = 0; w < kWaves; ++w) t += red[w][m][2 * c + i];
+            t *= code_unit<WF>();
             v[i] = t * (i ? pe_scale.y : pe_scale.x) + (i ? pe_bias.y : pe_bias.x);
         }
         apply_act<2>(v, act);
@@ -669,7 +678,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
         float v = 0.f;
 #pragma unroll
         for (int i = 0; i < kWaves; ++i) v += red[i][m][nn];
-        vsum[t] = v;
+        vsum[t] = v * code_unit<WF>();
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -706,7 +715,8 @@ template <int WF, int RT, int MU>
 __global__ __launch_bounds__(kWaves * 64, 1) void split_product_kernel(const uint16_t* __restrict__ x3, int M, int K,
                                                                       const uint8_t* __restrict__ w, int64_t ldw,
                                                                       int N, float* __restrict__ part) {
-    static_assert(WF == kW8 || WF == kW8T, "int8 codes");
+    static_assert(is_w8<WF>(), "integer codes");
+    typedef typename CodeReg<WF>::type WReg;
     __shared__ float red[kWaves][RT * 32][33];  // partial tiles, rows padded
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 31, h = lane >> 5;
@@ -730,15 +740,15 @@ __global__ __launch_bounds__(kWaves * 64, 1) void split_product_kernel(const uin
                 for (int e = 0; e < 2; ++e)
                     xv[c][q][e] = *reinterpret_cast<const u32x4*>(x3t + (((int64_t)(u0 + c) * 3 + q) * 2 + e) * 64 * 8);
         }
-    u32x4 wreg[MU][RT];
+    WReg wreg[MU][RT];
 #pragma unroll
     for (int c = 0; c < MU; ++c)
         if (c < cnt) {
 #pragma unroll
             for (int j = 0; j < RT; ++j) {
-                if constexpr (WF == kW8T) {  // 1 KB of consecutive codes per instruction, read once
-                    wreg[c][j] = __builtin_nontemporal_load(
-                        reinterpret_cast<const u32x4*>(w + ((int64_t)(t0 + j) * U + u0 + c) * 1024 + lane * 16));
+                if constexpr (WF == kW8T || WF == kW4T) {  // 1 KB (512 bytes) of consecutive codes per instruction, read once
+                    wreg[c][j] = __builtin_nontemporal_load(reinterpret_cast<const WReg*>(
+                        w + (((int64_t)(t0 + j) * U + u0 + c) * 64 + lane) * sizeof(WReg)));
                 } else {  // lane (r, h): 16 codes of row 32 (t0 + j) + r (clamped for a partial tile)
                     wreg[c][j] = *reinterpret_cast<const u32x4*>(w + (int64_t)min(32 * (t0 + j) + r, N - 1) * ldw +
                                                                  32 * (u0 + c) + 16 * h);
@@ -764,11 +774,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void split_product_kernel(const uin
                 }
 #pragma unroll
                 for (int j = 0; j < RT; ++j) {
-                    const u32x4 d = wreg[c][j];
-                    const uint32_t s0 = e == 0 ? d.x : d.z, s1 = e == 0 ? d.y : d.w;
-                    const u32x4 wq = {bf16x2_of_bytes(s0, 0), bf16x2_of_bytes(s0, 16), bf16x2_of_bytes(s1, 0),
-                                      bf16x2_of_bytes(s1, 16)};
-                    const bf16x8 wf = __builtin_bit_cast(bf16x8, wq);
+                    const bf16x8 wf = code_frag(wreg[c][j], e);
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xq[0], acc[j], 0, 0, 0);
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xq[1], acc[j], 0, 0, 0);
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, xq[2], acc[j], 0, 0, 0);
@@ -789,6 +795,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void split_product_kernel(const uin
         float v = 0.f;
 #pragma unroll
         for (int i = 0; i < kWaves; ++i) v += red[i][32 * j + m][nn];
+        v *= code_unit<WF>();
         const int gm = m0 + m, gn = 32 * (t0 + j) + nn;
         if (gm < M && gn < N) part[((int64_t)blockIdx.z * M + gm) * N + gn] = v;
     }
@@ -1086,11 +1093,11 @@ static int run_decode_f32_tiles(const LinearArgs& a, const uint16_t* x_planes, c
 int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float* next_ln_w,
                       const float* next_ln_b, float next_eps, uint16_t* planes_out) {
     if (a.fmt == kF32T) return run_decode_f32_tiles(a, x_planes, next_ln_w, planes_out);
-    if (a.fmt != kW8 && a.fmt != kW8T && a.fmt != kF32) return TIQ_EUNSUPPORTED;
+    if (a.fmt != kW8 && a.fmt != kW8T && a.fmt != kW4T && a.fmt != kF32) return TIQ_EUNSUPPORTED;
     if (a.M < kSkinnyMinRows || a.M > 64 || a.K <= 0 || a.K % 32 != 0 || a.N <= 0 || a.N > 0x7fffffff)
         return TIQ_EUNSUPPORTED;
-    if (a.fmt == kW8T && a.N % 32 != 0) return TIQ_EUNSUPPORTED;  // whole row tiles
-    const bool w8 = a.fmt == kW8 || a.fmt == kW8T;
+    if ((a.fmt == kW8T || a.fmt == kW4T) && a.N % 32 != 0) return TIQ_EUNSUPPORTED;  // whole row tiles
+    const bool w8 = a.fmt != kF32;
     if ((next_ln_w == nullptr) != (next_ln_b == nullptr) || (next_ln_w && !planes_out)) return TIQ_EINVAL;
     if (!a.y && !planes_out) return TIQ_EINVAL;
     // a row the reduction cannot take (N % 8, N > 8192) without planes out:
@@ -1159,6 +1166,7 @@ int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float
     float* part = reduce ? reinterpret_cast<float*>(ws) : nullptr;
     if (!part) plan.RT = 0;
     if (a.fmt == kW8) return run_decode_t<kW8>(a, x3, next_ln_w, next_ln_b, next_eps, planes_out, part, plan);
+    if (a.fmt == kW4T) return run_decode_t<kW4T>(a, x3, next_ln_w, next_ln_b, next_eps, planes_out, part, plan);
     if (a.fmt == kW8T) return run_decode_t<kW8T>(a, x3, next_ln_w, next_ln_b, next_eps, planes_out, part, plan);
     return run_decode_t<kF32>(a, x3, next_ln_w, next_ln_b, next_eps, planes_out, part, plan);
 }
@@ -1182,14 +1190,17 @@ size_t decode_slices_bytes(int64_t M, int64_t K, int64_t N) {
 }
 
 int launch_decode_slices(const LinearArgs& a, const uint16_t* x_planes, float* part) {
-    if (a.fmt != kW8 && a.fmt != kW8T) return TIQ_EUNSUPPORTED;
+    if (a.fmt != kW8 && a.fmt != kW8T && a.fmt != kW4T) return TIQ_EUNSUPPORTED;
     if (a.M < 1 || a.M > 64 || a.K <= 0 || a.K % 32 != 0 || a.N <= 0 || a.N > 0x7fffffff) return TIQ_EUNSUPPORTED;
-    if (a.fmt == kW8T && a.N % 32 != 0) return TIQ_EUNSUPPORTED;  // whole row tiles
+    if ((a.fmt == kW8T || a.fmt == kW4T) && a.N % 32 != 0) return TIQ_EUNSUPPORTED;  // whole row tiles
     if (!x_planes || !part || !a.w) return TIQ_EINVAL;
     if (a.fmt == kW8 && a.ldw < a.K) return TIQ_EINVAL;
     if (!aligned(a.w, 16) || a.ldw % 16 != 0 || !aligned(x_planes, 16) || !aligned(part, 16)) return TIQ_EALIGN;
     const SplitPlan plan = slices_plan(a.M, a.K, a.N);
     if (!slices_fit(a.K, plan)) return TIQ_EUNSUPPORTED;
+    if (a.fmt == kW4T)
+        return plan.RT == 2 ? launch_split_product<kW4T, 2>(a, x_planes, part, plan.S)
+                            : launch_split_product<kW4T, 1>(a, x_planes, part, plan.S);
     if (a.fmt == kW8T)
         return plan.RT == 2 ? launch_split_product<kW8T, 2>(a, x_planes, part, plan.S)
                             : launch_split_product<kW8T, 1>(a, x_planes, part, plan.S);
@@ -1217,6 +1228,31 @@ int launch_tile_int8(const uint8_t* w, int64_t N, int64_t K, int64_t ldw, uint8_
     if (!aligned(w, 16) || !aligned(tiles, 16) || ldw % 16 != 0) return TIQ_EALIGN;
     const int64_t nchunks = N * K / 16;
     hipLaunchKernelGGL(tile_int8_kernel, dim3((unsigned)((nchunks + 255) / 256)), dim3(256), 0, stream, w, ldw, K / 32,
+                       nchunks, tiles);
+    return launch_status();
+}
+
+// One thread per 8 bytes (16 nibbles) of a tile: block b = (t, u), lane l = 32 h
+// + r takes row 32 t + r, columns 32 u + 16 h .. + 15 (row stride K / 2 bytes).
+__global__ __launch_bounds__(256) void tile_int4_kernel(const uint8_t* __restrict__ w, int64_t U, int64_t nchunks,
+                                                        uint8_t* __restrict__ tiles) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nchunks) return;
+    const int64_t b = i >> 6, t = b / U, u = b - t * U;
+    const int l = (int)(i & 63), r = l & 31, h = l >> 5;
+    const uint2 v = *reinterpret_cast<const uint2*>(w + (32 * t + r) * U * 16 + 16 * u + 8 * h);
+    reinterpret_cast<uint2*>(tiles)[i] = v;
+}
+
+int launch_tile_int4(const uint8_t* w, int64_t N, int64_t K, uint8_t* tiles, hipStream_t stream) {
+    if (N < 0 || K < 0) return TIQ_EINVAL;
+    if (N == 0 || K == 0) return TIQ_OK;
+    if (!w || !tiles) return TIQ_EINVAL;
+    if (N % 32 != 0 || K % 32 != 0) return TIQ_EUNSUPPORTED;
+    if (!aligned(w, 16) || !aligned(tiles, 16)) return TIQ_EALIGN;
+    const int64_t nchunks = N * K / 16;
+    if ((nchunks + 255) / 256 > INT32_MAX) return TIQ_EUNSUPPORTED;
+    hipLaunchKernelGGL(tile_int4_kernel, dim3((unsigned)((nchunks + 255) / 256)), dim3(256), 0, stream, w, K / 32,
                        nchunks, tiles);
     return launch_status();
 }

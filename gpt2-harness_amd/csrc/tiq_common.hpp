@@ -158,6 +158,25 @@ __device__ __forceinline__ uint32_t bf16x2_of_bytes_perm(uint32_t d, int sh) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 
+// Nibbles as bf16 times 16: d holds 8 biased nibbles (column 2j in the low
+// nibble of byte j, code n - 8); e (even columns) and o (odd columns) get
+// each nibble in the high half of a byte with its top bit flipped, which as
+// a signed byte is 16 (n - 8). A byte becomes a float in one instruction
+// (sub-dword operand select with sign extension), and 16 (n - 8) is exact in
+// bf16; the factor 16 is taken out in the epilogue (an exact power of two:
+// every partial sum is 16 times the unscaled one, rounded the same way).
+__device__ __forceinline__ void nibbles_x16(uint32_t d, uint32_t& e, uint32_t& o) {
+    e = ((d << 4) & 0xf0f0f0f0u) ^ 0x80808080u;
+    o = (d & 0xf0f0f0f0u) ^ 0x80808080u;
+}
+
+// byte k of e and o -> two bf16 in one dword (even column low)
+__device__ __forceinline__ uint32_t bf16x2_of_x16(uint32_t e, uint32_t o, int k) {
+    const float lo = (float)(int8_t)(e >> (8 * k));
+    const float hi = (float)(int8_t)(o >> (8 * k));
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
+}
+
 template <int I>
 __device__ __forceinline__ float sbyte_f32(uint32_t d) {
     return (float)((int32_t)(d << (24 - 8 * I)) >> 24);

@@ -12,6 +12,7 @@ enum WFormat : int {
     kW4G = 2,  // group-wise nibbles, row n at byte n * ((K + 1) / 2), fp16 group scales
     kF32 = 3,  // fp32 weights (an unquantized Linear such as the tied lm_head), no scale
     kW8T = 4,  // int8 codes in 32 x 32 operand tiles (tiq_tile_int8; batched decode only)
+    kW4T = 6,  // reference nibbles in 32 x 32 operand tiles (tiq_tile_int4; batched decode only)
     kF32T = 5, // fp32 weights in 32 x 32 operand tiles (tiq_tile_f32; the batched decode head)
 };
 
@@ -97,7 +98,7 @@ int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float
 // consumer that finishes them itself (skinny.hip): slice z of `part` (M x N,
 // at part + z M N) holds K units [z U / S, (z + 1) U / S) of x W^T with no
 // scale or bias, S = decode_slices_count(M, K, N) <= kMaxSlices. int8
-// weights (kW8, kW8T), 1..64 rows, K % 32 == 0 (K <= 4096 with an even
+// weights (kW8, kW8T) or nibble tiles (kW4T), 1..64 rows, K % 32 == 0 (K <= 4096 with an even
 // count of 32-row tiles, else K <= 8192), the operand planes of a previous
 // decode linear in.
 constexpr int64_t kMaxSlices = 4;
@@ -114,6 +115,8 @@ size_t decode_linear_workspace(int64_t M, int64_t K, int64_t N);
 size_t decode_planes_bytes(int64_t M, int64_t K);
 // int8 codes (N, K) -> the operand tiles the decode product reads with kW8T.
 int launch_tile_int8(const uint8_t* w, int64_t N, int64_t K, int64_t ldw, uint8_t* tiles, hipStream_t stream);
+// reference-layout nibbles (N, K) -> the operand tiles it reads with kW4T.
+int launch_tile_int4(const uint8_t* w, int64_t N, int64_t K, uint8_t* tiles, hipStream_t stream);
 
 // The register-staged GEMM (gemm_staged.hip; int8 and reference-layout int4
 // weights): whether it takes these arguments, its tile choice (0: 256 x 256,

@@ -56,6 +56,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "tiq_decode_linear_workspace": ([_i32, _i64, _i64, _i64], _sz),
     "tiq_decode_planes_bytes": ([_i64, _i64], _sz),
     "tiq_tile_int8": ([_vp, _i64, _i64, _i64, _vp, _vp], _i32),
+    "tiq_tile_int4": ([_vp, _i64, _i64, _vp, _vp], _i32),
     "tiq_tile_f32_bytes": ([_i64, _i64], _sz),
     "tiq_tile_f32": ([_vp, _i64, _i64, _i64, _vp, _vp], _i32),
     "tiq_decode_linear": ([_vp, _i64, _vp, _i64, _i64, _vp, _i32, _vp, _vp, _i64, _vp, _i64, _vp, _vp, _f32, _i32,
@@ -87,7 +88,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
                                      _vp, _vp, _sz, _vp], _i32),
 }
 
-WF_INT8, WF_INT4, WF_INT4G, WF_F32, WF_INT8_TILED, WF_F32_TILED = 0, 1, 2, 3, 4, 5
+WF_INT8, WF_INT4, WF_INT4G, WF_F32, WF_INT8_TILED, WF_F32_TILED, WF_INT4_TILED = 0, 1, 2, 3, 4, 5, 6
 ACT_NONE, ACT_GELU_TANH = 0, 1
 #: status codes of tiq.h
 OK, EINVAL, EBITS, EALIGN, EUNSUPPORTED, EWORKSPACE, ESCRATCH = 0, -1, -2, -3, -4, -5, -6

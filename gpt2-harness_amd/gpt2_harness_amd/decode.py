@@ -173,6 +173,7 @@ class GraphDecoder(_DecoderBase):
 
 
 _WF = {FMT_W8: _lib.WF_INT8, FMT_W4: _lib.WF_INT4, FMT_W4G: _lib.WF_INT4G}
+_TILED = {_lib.WF_INT8: _lib.WF_INT8_TILED, _lib.WF_INT4: _lib.WF_INT4_TILED, _lib.WF_F32: _lib.WF_F32_TILED}
 
 
 def fused_supported(model) -> str | None:
@@ -240,12 +241,14 @@ class FusedDecoder(_DecoderBase):
         ws = max(ws, int(self.L.tiq_linear_fused_workspace(_lib.F32, head_fmt, B, C, cfg.vocab_size)))
         self.lin_ws = torch.empty(max(ws, 1), dtype=torch.uint8, device=dev)
         self.lin_ws_bytes = ws
-        # Batched rows (5..64) with int8 block Linears: each Linear splits its K
+        # Batched rows (5..64) with int8 or int4 block Linears: each Linear splits its K
         # range over workgroups and hands the next one its LayerNorm'd operand
         # planes (tiq_decode_linear), so no separate LayerNorm / split launches
         lins = [l for b in model.h for l in (b.attn.c_attn, b.attn.c_proj, b.mlp.c_fc, b.mlp.c_proj)]
         head_ok = self.head_q is None or self.head_q.fmt == FMT_W8
-        self.chain = 5 <= B <= 64 and head_ok and all(l.fmt == FMT_W8 for l in lins)
+        # (int4 codes only in operand tiles, so whole ones)
+        self.chain = 5 <= B <= 64 and head_ok and all(
+            l.fmt == FMT_W8 or (l.fmt == FMT_W4 and l.out_features % 32 == 0 and l.in_features % 32 == 0) for l in lins)
         self.rows_prefill = all(l.fmt == FMT_W8 for l in lins)
         # One sequence with the tied fp32 head: the decode step's head and
         # argmax read an int8 (or bf16) copy of the head and recompute from
@@ -292,16 +295,20 @@ class FusedDecoder(_DecoderBase):
             self.p_hid = torch.empty(ph, dtype=torch.uint8, device=dev)   # GELU(c_fc) planes
             self.p_att = torch.empty(pc, dtype=torch.uint8, device=dev)   # attention output planes
             # the block Linears' codes once more, in the operand tiles the
-            # batched products read as 1 KB consecutive loads (the row-major
-            # codes stay for prefill): 1x the int8 weight bytes again
+            # batched products read as consecutive loads (the row-major
+            # codes stay for prefill): 1x the weight bytes again
             self.tiles = {}
             for lin in lins:
                 if lin.out_features % 32 or lin.in_features % 32:
                     continue  # whole 32 x 32 tiles only; these keep the row-major codes
                 t = torch.empty_like(lin.codes)
-                _lib.check(L.tiq_tile_int8(lin.codes.data_ptr(), lin.out_features, lin.in_features,
-                                           lin.codes.stride(0), t.data_ptr(),
-                                           torch.cuda.current_stream(dev).cuda_stream), "tile int8 codes")
+                st = torch.cuda.current_stream(dev).cuda_stream
+                if lin.fmt == FMT_W4:
+                    _lib.check(L.tiq_tile_int4(lin.codes.data_ptr(), lin.out_features, lin.in_features, t.data_ptr(),
+                                               st), "tile int4 codes")
+                else:
+                    _lib.check(L.tiq_tile_int8(lin.codes.data_ptr(), lin.out_features, lin.in_features,
+                                               lin.codes.stride(0), t.data_ptr(), st), "tile int8 codes")
                 self.tiles[id(lin)] = t
             # the fp32 head (the tied embedding) in 4 KB operand tiles, which
             # the decode linear streams with one workgroup per CU (the
@@ -316,7 +323,7 @@ class FusedDecoder(_DecoderBase):
     @property
     def extra_weight_bytes(self) -> int:
         """Device bytes of the weight copies this decoder holds beyond the
-        model's own (the batched step's operand tiles of the int8 block codes
+        model's own (the batched step's operand tiles of the block codes
         and of the fp32 tied head; for one sequence with the fp32 tied head
         its int8 copy and two floats a row, or its bf16 copy and one float a
         row, for the screened argmax; 0 for two to four sequences, which read
@@ -434,7 +441,7 @@ class FusedDecoder(_DecoderBase):
         w = lin.codes if isinstance(lin, QuantLinear) else self.head_w
         tiles = getattr(self, "tiles", {}).get(id(lin))
         if tiles is not None:
-            w, wf = tiles, (_lib.WF_F32_TILED if wf == _lib.WF_F32 else _lib.WF_INT8_TILED)
+            w, wf = tiles, _TILED[_lib.WF_F32 if wf == _lib.WF_F32 else _WF[lin.fmt]]
         scale = lin.scale.data_ptr() if isinstance(lin, QuantLinear) else None
         bias = _lib.ptr(lin.bias) if isinstance(lin, QuantLinear) else None
         rc = self.L.tiq_decode_linear(
@@ -454,7 +461,7 @@ class FusedDecoder(_DecoderBase):
         w, wf = lin.codes, _lib.WF_INT8
         tiles = self.tiles.get(id(lin))
         if tiles is not None:
-            w, wf = tiles, _lib.WF_INT8_TILED
+            w, wf = tiles, _TILED[_WF[lin.fmt]]
         rc = self.L.tiq_decode_qkv_attention(
             self.p_ln1.data_ptr(), self.B, lin.in_features, w.data_ptr(), wf, lin.scale.data_ptr(),
             _lib.ptr(lin.bias), self.H, self.Hkv, self.hd, self.k[i].data_ptr(), self.v[i].data_ptr(), self.T,

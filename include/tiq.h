@@ -51,6 +51,8 @@ enum tiq_weight_format {
     TIQ_WF_INT8_TILED = 4,
     /* fp32 weights rearranged by tiq_tile_f32 (tiq_decode_linear from planes only) */
     TIQ_WF_F32_TILED = 5,
+    /* reference-layout int4 codes rearranged by tiq_tile_int4 (as TIQ_WF_INT8_TILED) */
+    TIQ_WF_INT4_TILED = 6,
 };
 
 /* Activations fused after a linear. */
@@ -317,7 +319,8 @@ int tiq_linear_fused_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_
 
 /* Batched decode-step linear (5 <= M <= 64 fp32 activation rows; int8
  * weights with per-row scale -- row-major (TIQ_WF_INT8) or in the operand
- * tiles of tiq_tile_int8 (TIQ_WF_INT8_TILED, N % 32 == 0) -- or fp32
+ * tiles of tiq_tile_int8 (TIQ_WF_INT8_TILED, N % 32 == 0) --, int4 codes in
+ * the tiles of tiq_tile_int4 (TIQ_WF_INT4_TILED, N % 32 == 0), or fp32
  * weights) whose K range is split over
  * workgroups: the matrix-core products write fp32 partial sums to the
  * workspace, a second kernel sums them in a fixed order and applies
@@ -351,6 +354,17 @@ size_t tiq_decode_planes_bytes(int64_t M, int64_t K);
  * (TIQ_WF_INT8): the products are the same, in the same order. No
  * counterpart in the reference (a device layout of this library). */
 int tiq_tile_int8(const int8_t* w, int64_t N, int64_t K, int64_t ldw, int8_t* tiles, void* stream);
+
+/* The reference-layout int4 codes of an (N, K) weight (row n at byte n * K / 2)
+ * rearranged for tiq_decode_linear and tiq_decode_qkv_attention with w_format
+ * TIQ_WF_INT4_TILED: N * K / 2 bytes in 512-byte blocks, block t * (K / 32) + u
+ * holding rows 32 t .. 32 t + 31 and columns 32 u .. 32 u + 31, bytes 8 l .. 8 l
+ * + 7 of it the nibbles of row 32 t + l % 32, columns 32 u + 16 (l / 32) .. + 15.
+ * Needs N % 32 == 0, K % 32 == 0 and 16-byte aligned pointers. Products, order
+ * and the other arguments are those of the int8 formats (a code is exact in
+ * bf16 either way). No counterpart in the reference (a device layout of this
+ * library). */
+int tiq_tile_int4(const uint8_t* w, int64_t N, int64_t K, uint8_t* tiles, void* stream);
 
 /* The fp32 weights of an (N, K) unquantized Linear (the tied lm_head,
  * model.py:585; leading dimension ldw floats, 16-byte aligned rows)
@@ -424,7 +438,8 @@ int tiq_decode_attention_planes(const float* qkv, int64_t ld_qkv, int64_t batch,
  * in one call (model.py:254 c_attn at T = 1, then as tiq_decode_attention_planes):
  * x_planes are the operand planes of LayerNorm 1's output (planes_out of a
  * previous tiq_decode_linear with next_ln = ln_1, K = n_embd); w the int8
- * codes of c_attn (TIQ_WF_INT8, rows of n_embd bytes, or TIQ_WF_INT8_TILED),
+ * codes of c_attn (TIQ_WF_INT8, rows of n_embd bytes, or TIQ_WF_INT8_TILED), or
+ * its int4 codes (TIQ_WF_INT4_TILED),
  * scale / bias (bias may be NULL) its per-output fp32 factors, N = (n_head +
  * 2 n_kv_head) * head_dim outputs. The product runs split over K into fp32
  * partial slices in the workspace, and the attention kernel sums them for
