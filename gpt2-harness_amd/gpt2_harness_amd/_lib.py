@@ -133,7 +133,9 @@ def check(status: int, what: str) -> None:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current HIP stream of the tensor's device (the raw handle: building
+    torch's Stream object costs as much as a small launch)."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -185,9 +185,8 @@ def _fused_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, first: i
 
     y = torch.empty(B, T, H * hd, device=q.device, dtype=torch.float32)
     rc = _lib.lib().tiq_prefill_attention(
-        q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2),
-        v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), B, H, T, first, hd, y.data_ptr(), y.stride(0), hd,
-        y.stride(1), _lib.stream_of(q))
+        q.data_ptr(), *q.stride()[:3], k.data_ptr(), *k.stride()[:3], v.data_ptr(), *v.stride()[:3], B, H, T, first, hd,
+        y.data_ptr(), T * H * hd, hd, H * hd, _lib.stream_of(q))
     if rc in (_lib.EALIGN, _lib.EUNSUPPORTED):
         return None  # strides or sizes the kernel does not take: the torch ops below
     _lib.check(rc, "prefill attention")
