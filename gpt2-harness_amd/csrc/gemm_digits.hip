@@ -79,12 +79,19 @@ __device__ __forceinline__ void store_digits(const float (&v)[16], float mul, ui
     for (int q = 0; q < kDigits; ++q) *reinterpret_cast<u32x4*>(dst + 1024 * q) = pl[q];
 }
 
-template <int IT, bool NIB>
+// LN: the digits of LayerNorm(x) (two-pass mean and biased variance as torch;
+// the row already sits in registers, so the LayerNorm's own pass -- a read and a
+// write of x, 9 us at 4096 x 1600 -- costs two exchanges more here).
+template <int IT, bool NIB, bool LN>
 __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float* __restrict__ x, int64_t ldx, int M,
                                                                      int K, uint8_t* __restrict__ xt,
-                                                                     float* __restrict__ rs, bool gelu) {
+                                                                     float* __restrict__ rs, bool gelu,
+                                                                     const float* __restrict__ ln_w,
+                                                                     const float* __restrict__ ln_b, float ln_eps) {
+    static_assert(!LN || IT > 0, "LayerNorm needs the row in registers");
     constexpr int WV = kSplitThreads / 64, CT = kSplitThreads / 8;  // 16-column chunks a pass
     __shared__ uint32_t am[WV][8];
+    __shared__ float ls[2][WV][8];
     const int tid = threadIdx.x, r8 = tid & 7, c0 = tid >> 3;
     const int m = blockIdx.x * 8 + r8;
     const int NC = K / 16, U = K / 32;
@@ -126,6 +133,50 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
     if constexpr (IT > 0) {
 #pragma unroll
         for (int it = 0; it < IT; ++it) load(min(c0 + CT * it, NC - 1), v[it]);  // past the row: its last chunk again
+        if constexpr (LN) {
+            // a row is the 64 threads of equal tid % 8: eight lanes of each wavefront
+            auto row_sum = [&](float s, int slot) {
+#pragma unroll
+                for (int off = 32; off >= 8; off >>= 1) s += __shfl_xor(s, off, 64);
+                if ((tid & 63) < 8) ls[slot][tid >> 6][r8] = s;
+                __syncthreads();
+                float t = 0.f;
+#pragma unroll
+                for (int w = 0; w < WV; ++w) t += ls[slot][w][r8];
+                return t;
+            };
+            float s = 0.f;
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                float t = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) t += v[it][i];
+                s += c0 + CT * it < NC ? t : 0.f;
+            }
+            const float mu = row_sum(s, 0) / (float)K;
+            float d = 0.f;
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                float t = 0.f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) t = fmaf(v[it][i] - mu, v[it][i] - mu, t);
+                d += c0 + CT * it < NC ? t : 0.f;
+            }
+            const float rstd = 1.0f / sqrtf(row_sum(d, 1) / (float)K + ln_eps);
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                const int c = 16 * min(c0 + CT * it, NC - 1);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 gw = *reinterpret_cast<const float4*>(ln_w + c + 4 * q);
+                    const float4 gb = *reinterpret_cast<const float4*>(ln_b + c + 4 * q);
+                    v[it][4 * q + 0] = fmaf((v[it][4 * q + 0] - mu) * rstd, gw.x, gb.x);
+                    v[it][4 * q + 1] = fmaf((v[it][4 * q + 1] - mu) * rstd, gw.y, gb.y);
+                    v[it][4 * q + 2] = fmaf((v[it][4 * q + 2] - mu) * rstd, gw.z, gb.z);
+                    v[it][4 * q + 3] = fmaf((v[it][4 * q + 3] - mu) * rstd, gw.w, gb.w);
+                }
+            }
+        }
 #pragma unroll
         for (int it = 0; it < IT; ++it)
 #pragma unroll
@@ -184,11 +235,25 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
 // fp32 sums -- the lanes of a result register share no column, so a scale is
 // one load a lane and column tile; the next group starts from zero.
 // gridDim.z > 1: split over K, workgroup z writes fp32 slice z of y (no bias).
+// Out (fp32 output, unsplit): a residual added last, or a c_attn whose key and
+// value columns go to the cache (a 32-column tile lies within one head, so its
+// base address is one scalar) instead of to rows that a copy would read again.
+// 32 x 128 rows of width 1600: attention with its cache 281 -> 256 us, the two
+// 10 us copies gone; four windows of 128 through GPT-2 small with both LayerNorms,
+// residuals and GELU inside the products 1515 -> 1374 us.
+struct DigitsOut {
+    const float* res;
+    int64_t ldr;
+    float *k, *v;
+    int64_t sb, sh, st;
+    uint32_t T, magic;  // magic = ceil(2^32 / T): m / T = (m magic) >> 32 for m T < 2^32; 0: T = 1
+};
+
 template <int WMW, int TM, int TN, int D, int OCC, bool PERSIST, int FMT, typename TY>
 __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
     const uint8_t* __restrict__ xt, const float* __restrict__ rs, const uint8_t* __restrict__ w, int64_t ldw,
     const float* __restrict__ scale, const float* __restrict__ bias, TY* __restrict__ y, int64_t ldy, int M, int N,
-    int K, const uint16_t* __restrict__ scale16, int ngroups, int gs) {
+    int K, const uint16_t* __restrict__ scale16, int ngroups, int gs, DigitsOut out) {
     constexpr bool GROUPED = FMT == kW4G;
     static_assert(D >= 2, "register sets");
     constexpr int WNW = 4 / WMW;
@@ -406,12 +471,67 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 rm[i][g] = *reinterpret_cast<const float4*>(rs + min(m0 / 32 + i, T - 1) * 32 + 8 * g + 4 * h);
+        auto digit_sum = [&](int i, int j, int q) -> float {
+            if constexpr (GROUPED) {
+                return sum[j][i][q];
+            } else {
+                float f = (float)acc[j][i][3][q];
+                f = fmaf(f, 256.f, (float)acc[j][i][2][q]);
+                f = fmaf(f, 256.f, (float)acc[j][i][1][q]);
+                return fmaf(f, 256.f, (float)acc[j][i][0][q]);
+            }
+        };
         tile += gridDim.x;
         const bool more = PERSIST && tile < total;
         if (more) begin_tile(tile);
 #pragma unroll
         for (int i = 0; i < TM; ++i) {
             TY* yr = y + ((int64_t)blockIdx.z * M + m0 + 32 * i + 4 * h) * ldy + n0 + r;
+            if constexpr (sizeof(TY) == 4) {
+                if (out.res || out.k) {
+                    // groups of four rows of a column tile, a group's residuals
+                    // requested RD groups before its stores
+                    constexpr int RD = PERSIST ? 0 : 3, NG = 4 * TN;  // persistent: the next tile's loads hold the registers
+                    float rv[RD + 1][4];
+                    auto request = [&](int t) {
+                        const int n = min(n0 + 32 * (t >> 2) + r, N - 1);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            rv[t % (RD + 1)][e] =
+                                out.res[(int64_t)min(m0 + 32 * i + 8 * (t & 3) + 4 * h + e, M - 1) * out.ldr + n];
+                    };
+                    if (out.res) {
+#pragma unroll
+                        for (int t = 0; t < RD; ++t) request(t);
+                    }
+                    const int C = N / 3;
+#pragma unroll
+                    for (int t = 0; t < NG; ++t) {
+                        const int j = t >> 2, g = t & 3;
+                        if (out.res && t + RD < NG) request(t + RD);
+                        const int n = n0 + 32 * j;  // scalar, as is the tile's place
+                        const int part = n / C, col = n - part * C;
+                        const bool cached = out.k && part > 0;
+                        TY* base = cached ? (part == 1 ? out.k : out.v) + (col >> 6) * out.sh + (col & 63) + r : y + n + r;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int q = 4 * g + e, m = m0 + 32 * i + 8 * g + 4 * h + e;
+                            const float4 g4 = rm[i][g];
+                            const float rmq = e == 0 ? g4.x : e == 1 ? g4.y : e == 2 ? g4.z : g4.w;
+                            const float v = fmaf(digit_sum(i, j, q) * rmq, sc[j], bi[j]);
+                            if (m < M && n + r < N) {
+                                if (cached) {
+                                    const uint32_t b = out.magic ? __umulhi((uint32_t)m, out.magic) : (uint32_t)m;
+                                    base[(int64_t)b * out.sb + (int64_t)((uint32_t)m - b * out.T) * out.st] = v;
+                                } else {
+                                    base[(int64_t)m * ldy] = out.res ? v + rv[t % (RD + 1)][e] : v;
+                                }
+                            }
+                        }
+                    }
+                    continue;
+                }
+            }
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
 #pragma unroll
@@ -421,16 +541,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
                     TY* dst = yr + (int64_t)(8 * g + e) * ldy;
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
-                        float f;
-                        if constexpr (GROUPED) {
-                            f = sum[j][i][q];
-                        } else {
-                            f = (float)acc[j][i][3][q];
-                            f = fmaf(f, 256.f, (float)acc[j][i][2][q]);
-                            f = fmaf(f, 256.f, (float)acc[j][i][1][q]);
-                            f = fmaf(f, 256.f, (float)acc[j][i][0][q]);
-                        }
-                        const float v = fmaf(f * rmq, sc[j], bi[j]);
+                        const float v = fmaf(digit_sum(i, j, q) * rmq, sc[j], bi[j]);
                         if (full || (m0 + 32 * i + 8 * g + 4 * h + e < M && n0 + 32 * j + r < N)) {
                             if constexpr (sizeof(TY) == 4) dst[32 * j] = v;
                             else dst[32 * j] = f32_to_bf16_bits(v);
@@ -445,14 +556,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
 }
 
 template <int WMW, int TM, int TN, int D, int OCC, bool PERSIST, int FMT, typename TY>
-int run_digits(const LinearArgs& a, const uint8_t* xt, const float* rs, TY* y, int64_t ldy, int64_t S) {
+int run_digits(const LinearArgs& a, const uint8_t* xt, const float* rs, TY* y, int64_t ldy, int64_t S,
+               const DigitsOut& out) {
     constexpr int BM = 32 * TM * WMW, BN = 32 * TN * (4 / WMW);
     const int64_t tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
     const int64_t grid = PERSIST ? std::min<int64_t>(tiles, 256 * OCC) : tiles;
     hipLaunchKernelGGL((gemm_digits_kernel<WMW, TM, TN, D, OCC, PERSIST, FMT, TY>), dim3((unsigned)grid, 1, (unsigned)S),
                        dim3(256), 0, a.stream, xt, rs, a.w, a.ldw, a.scale, a.bias, y, ldy, (int)a.M, (int)a.N,
                        (int)a.K, a.scale16, FMT == kW4G ? (int)((a.K + a.group - 1) / a.group) : 0,
-                       FMT == kW4G ? a.group / 64 : 1);
+                       FMT == kW4G ? a.group / 64 : 1, out);
     return launch_status();
 }
 
@@ -487,40 +599,46 @@ size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 template <int FMT, typename TY>
 int dispatch_digits(const LinearArgs& a, DigitTile tile, const uint8_t* xt, const float* rs, TY* y, int64_t ldy,
-                    int64_t S) {
+                    int64_t S, const DigitsOut& out = {}) {
     // group-wise: the fp32 sums beside the integer ones fit the small tile
-    if constexpr (FMT == kW4G) return run_digits<1, 1, 1, 3, 2, false, FMT, TY>(a, xt, rs, y, ldy, S);
+    if constexpr (FMT == kW4G) return run_digits<1, 1, 1, 3, 2, false, FMT, TY>(a, xt, rs, y, ldy, S, out);
     else switch (tile) {
-        case kTile64x256: return run_digits<2, 1, 4, 2, 1, false, FMT, TY>(a, xt, rs, y, ldy, S);
-        case kTile64x128: return run_digits<2, 1, 2, 2, 2, true, FMT, TY>(a, xt, rs, y, ldy, S);
-        default: return run_digits<1, 1, 1, 4, 2, false, FMT, TY>(a, xt, rs, y, ldy, S);
+        case kTile64x256: return run_digits<2, 1, 4, 2, 1, false, FMT, TY>(a, xt, rs, y, ldy, S, out);
+        case kTile64x128: return run_digits<2, 1, 2, 2, 2, true, FMT, TY>(a, xt, rs, y, ldy, S, out);
+        default: return run_digits<1, 1, 1, 4, 2, false, FMT, TY>(a, xt, rs, y, ldy, S, out);
     }
 }
 
 template <bool NIB>
-int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu) {
-    const dim3 grid((unsigned)((a.M + 7) / 8)), block(kSplitThreads);
-    const float* x = static_cast<const float*>(a.x);
-    const int M = (int)a.M, K = (int)a.K;
-    if (K <= 1024) hipLaunchKernelGGL((split_digits_kernel<1, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
-    else if (K <= 2048) hipLaunchKernelGGL((split_digits_kernel<2, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
-    else if (K <= 4096) hipLaunchKernelGGL((split_digits_kernel<4, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
-    else if (K <= 7168) hipLaunchKernelGGL((split_digits_kernel<7, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
-    else hipLaunchKernelGGL((split_digits_kernel<0, NIB>), grid, block, 0, a.stream, x, a.ldx, M, K, xt, rs, gelu);
-    return launch_status();
+int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu, const PrefillFusion& f) {
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((a.M + 7) / 8)), dim3(kSplitThreads), 0, a.stream,
+                           static_cast<const float*>(a.x), a.ldx, (int)a.M, (int)a.K, xt, rs, gelu, f.ln_w, f.ln_b,
+                           f.ln_eps);
+        return launch_status();
+    };
+    if (f.ln_w) return a.K <= 1024 ? launch(split_digits_kernel<1, NIB, true>) : launch(split_digits_kernel<2, NIB, true>);
+    if (a.K <= 1024) return launch(split_digits_kernel<1, NIB, false>);
+    if (a.K <= 2048) return launch(split_digits_kernel<2, NIB, false>);
+    if (a.K <= 4096) return launch(split_digits_kernel<4, NIB, false>);
+    if (a.K <= 7168) return launch(split_digits_kernel<7, NIB, false>);
+    return launch(split_digits_kernel<0, NIB, false>);
 }
 
 template <int FMT>
-int run_digits_linear(const LinearArgs& a, uint8_t* xt, float* rs, float* part, int64_t S, bool gelu) {
-    int rc = launch_split_digits<FMT != kW8>(a, xt, rs, gelu);
+int run_digits_linear(const LinearArgs& a, uint8_t* xt, float* rs, float* part, int64_t S, bool gelu,
+                      const PrefillFusion& f) {
+    int rc = launch_split_digits<FMT != kW8>(a, xt, rs, gelu, f);
     if (rc != TIQ_OK) return rc;
     const DigitTile tile = S > 1 ? kTile32x128 : digits_tile(a.M, a.N, a.K);
     if (S > 1) {
         rc = dispatch_digits<FMT, float>(a, tile, xt, rs, part, a.N, S);
-        return rc != TIQ_OK ? rc : launch_splitk_reduce(a, part, S, nullptr);
+        return rc != TIQ_OK ? rc : launch_splitk_reduce(a, part, S, nullptr, f.res, f.ldr);
     }
-    if (a.y_dtype == TIQ_F32) return dispatch_digits<FMT, float>(a, tile, xt, rs, static_cast<float*>(a.y), a.ldy, 1);
-    return dispatch_digits<FMT, uint16_t>(a, tile, xt, rs, static_cast<uint16_t*>(a.y), a.ldy, 1);
+    if (a.y_dtype != TIQ_F32) return dispatch_digits<FMT, uint16_t>(a, tile, xt, rs, static_cast<uint16_t*>(a.y), a.ldy, 1);
+    DigitsOut out = {f.res, f.ldr, f.k, f.v, f.sb, f.sh, f.st, (uint32_t)f.T, 0};
+    if (f.T > 1) out.magic = (uint32_t)(((1ull << 32) + f.T - 1) / f.T);
+    return dispatch_digits<FMT, float>(a, tile, xt, rs, static_cast<float*>(a.y), a.ldy, 1, out);
 }
 
 }  // namespace
@@ -547,8 +665,12 @@ bool digits_supported(const LinearArgs& a) {
     return ((a.M + 31) / 32) * ((a.N + 127) / 128) <= 0x7fffffffLL && a.M <= 0x7fffffff - 64;
 }
 
-int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu) {
+int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu, const PrefillFusion& f) {
     if (!digits_supported(a)) return TIQ_EUNSUPPORTED;
+    if (f.ln_w && (a.K > kDigitsLnMaxK || !aligned(f.ln_w, 16) || !aligned(f.ln_b, 16))) return TIQ_EUNSUPPORTED;
+    // rows of a sequence by multiplication: m T < 2^32; a product that is split
+    // for want of tiles leaves its key and value columns to the caller
+    if (f.k && (a.N % 192 != 0 || a.M * f.T > 0xffffffffLL || digits_splits(a.M, a.N, a.K) > 1)) return TIQ_EUNSUPPORTED;
     const size_t need = digits_workspace(a.M, a.K);
     if (!ws || ws_bytes < need || !aligned(ws, 16)) return TIQ_EWORKSPACE;
     uint8_t* xt = static_cast<uint8_t*>(ws);
@@ -560,11 +682,12 @@ int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu) {
     const int unit = a.y_dtype == TIQ_F32 ? 4 : 8;
     int64_t S = digits_splits(a.M, a.N, a.K);
     if (a.N % 8 != 0 || a.ldy % unit != 0 || !aligned(a.y, 16) || (a.bias && !aligned(a.bias, 16))) S = 1;
+    if (f.res && (f.ldr % 4 != 0 || !aligned(f.res, 16))) S = 1;
     S = std::min<int64_t>(S, (int64_t)((ws_bytes - need) / (size_t)(a.M * a.N * 4)));
     S = std::max<int64_t>(S, 1);
-    if (a.fmt == kW4G) return run_digits_linear<kW4G>(a, xt, rs, part, S, gelu);
-    return a.fmt == kW4 ? run_digits_linear<kW4>(a, xt, rs, part, S, gelu)
-                        : run_digits_linear<kW8>(a, xt, rs, part, S, gelu);
+    if (a.fmt == kW4G) return run_digits_linear<kW4G>(a, xt, rs, part, S, gelu, f);
+    return a.fmt == kW4 ? run_digits_linear<kW4>(a, xt, rs, part, S, gelu, f)
+                        : run_digits_linear<kW8>(a, xt, rs, part, S, gelu, f);
 }
 
 }  // namespace tiq

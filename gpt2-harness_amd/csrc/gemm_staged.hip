@@ -78,12 +78,14 @@ int staged_choice(int64_t M, int64_t N, int64_t K, bool bf16_out) {
 
 // The end of a split-K product: y[m][n] = scale[n] * sum_z part[z][m][n] +
 // bias[n] (scale 1 when null: the group-wise slices are scaled already), the
-// S slices summed in a fixed order; 4 consecutive outputs a thread.
+// S slices summed in a fixed order; 4 consecutive outputs a thread; fp32
+// output: the residual res added last when given.
 template <typename TY>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ part, int S, int M, int N,
                                                             const float* __restrict__ scale,
                                                             const float* __restrict__ bias, TY* __restrict__ y,
-                                                            int64_t ldy) {
+                                                            int64_t ldy, const float* __restrict__ res,
+                                                            int64_t ldr) {
     const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= (int64_t)M * N) return;
     const int m = (int)(i / N), n = (int)(i % N);
@@ -112,7 +114,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restr
     const float o2 = fmaf(a.z, sc.z, bi.z), o3 = fmaf(a.w, sc.w, bi.w);
     TY* yr = y + (int64_t)m * ldy + n;
     if constexpr (sizeof(TY) == 4) {
-        *reinterpret_cast<float4*>(yr) = make_float4(o0, o1, o2, o3);
+        float4 rv = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (res) rv = *reinterpret_cast<const float4*>(res + (int64_t)m * ldr + n);
+        *reinterpret_cast<float4*>(yr) =
+            res ? make_float4(o0 + rv.x, o1 + rv.y, o2 + rv.z, o3 + rv.w) : make_float4(o0, o1, o2, o3);
     } else {
         uint2 o;
         o.x = pk_bf16(o0, o1);
@@ -215,15 +220,16 @@ int launch_staged_gemm_split(const LinearArgs& a, void* ws, size_t ws_bytes) {
     return launch_splitk_reduce(a, part, S, a.scale);
 }
 
-int launch_splitk_reduce(const LinearArgs& a, const float* part, int64_t S, const float* scale) {
+int launch_splitk_reduce(const LinearArgs& a, const float* part, int64_t S, const float* scale, const float* res,
+                         int64_t ldr) {
     const int64_t quads = a.M * a.N / 4;
     const dim3 grid((unsigned)((quads + 255) / 256));
     if (a.y_dtype == TIQ_F32)
         hipLaunchKernelGGL(splitk_reduce_kernel<float>, grid, dim3(256), 0, a.stream, part, (int)S, (int)a.M,
-                           (int)a.N, scale, a.bias, static_cast<float*>(a.y), a.ldy);
+                           (int)a.N, scale, a.bias, static_cast<float*>(a.y), a.ldy, res, ldr);
     else
         hipLaunchKernelGGL(splitk_reduce_kernel<uint16_t>, grid, dim3(256), 0, a.stream, part, (int)S, (int)a.M,
-                           (int)a.N, scale, a.bias, static_cast<uint16_t*>(a.y), a.ldy);
+                           (int)a.N, scale, a.bias, static_cast<uint16_t*>(a.y), a.ldy, nullptr, (int64_t)0);
     return launch_status();
 }
 

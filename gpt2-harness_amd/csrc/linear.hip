@@ -336,6 +336,40 @@ extern "C" int tiq_linear_gelu_in_ws(const float* x, int64_t M, int64_t K, int64
     return run_linear_split(a, workspace, workspace_bytes, true);
 }
 
+extern "C" int tiq_linear_prefill_ws(const float* x, int64_t M, int64_t K, int64_t ldx, const void* w, int w_format,
+                                     const float* scale, const uint16_t* scale_f16, int group, const float* bias,
+                                     int64_t N, float* y, int64_t ldy, const float* ln_weight, const float* ln_bias,
+                                     float ln_eps, int gelu_in, const float* residual, int64_t ld_residual,
+                                     float* k_out, float* v_out, int64_t kv_sb, int64_t kv_sh, int64_t kv_st,
+                                     int64_t T, void* workspace, size_t workspace_bytes, void* stream) {
+    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT4 && w_format != TIQ_WF_INT4_GROUPWISE) return TIQ_EINVAL;
+    if ((ln_weight == nullptr) != (ln_bias == nullptr) || (k_out == nullptr) != (v_out == nullptr)) return TIQ_EINVAL;
+    if ((ln_weight && gelu_in) || (residual && (k_out || ld_residual < N))) return TIQ_EINVAL;
+    if (k_out && (T <= 0 || M % T != 0 || N % 3 != 0 || ldy < N / 3 || kv_sb < 0 || kv_sh < 0 || kv_st < 0))
+        return TIQ_EINVAL;
+    const WFormat fmt = (WFormat)w_format;
+    const int64_t ldw = fmt == kW8 ? K : fmt == kW4 ? K / 2 : (K + 1) / 2;
+    LinearArgs a = make_args(x, TIQ_F32, M, K, ldx, static_cast<const uint8_t*>(w), ldw, scale, scale_f16, group,
+                             bias, N, y, TIQ_F32, k_out ? std::max(ldy, N) : ldy, stream, fmt);
+    int rc = check_linear(a);
+    if (rc != TIQ_OK || M == 0 || N == 0) return rc;
+    a.ldy = ldy;
+    if (!digits_rows(fmt, M, K, N)) return TIQ_EUNSUPPORTED;
+    PrefillFusion f;
+    f.ln_w = ln_weight;
+    f.ln_b = ln_bias;
+    f.ln_eps = ln_eps;
+    f.res = residual;
+    f.ldr = ld_residual;
+    f.k = k_out;
+    f.v = v_out;
+    f.sb = kv_sb;
+    f.sh = kv_sh;
+    f.st = kv_st;
+    f.T = k_out ? T : 0;
+    return launch_digits(a, workspace, workspace_bytes, gelu_in != 0, f);
+}
+
 extern "C" int tiq_gemv_w8(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const int8_t* q,
                            const float* scale, const float* bias, int64_t N, void* y, int y_dtype, int64_t ldy,
                            void* stream) {

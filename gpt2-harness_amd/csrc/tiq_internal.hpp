@@ -134,7 +134,10 @@ size_t staged_split_workspace(int64_t M, int64_t N, int64_t K);
 int launch_staged_gemm_split(const LinearArgs& a, void* ws, size_t ws_bytes);
 // y = scale * (sum of the S fp32 slices part[S][M][N], in slice order) + bias
 // (scale null: 1), with a's output, bias and stream; N % 4 == 0.
-int launch_splitk_reduce(const LinearArgs& a, const float* part, int64_t S, const float* scale);
+// res (M, N) with leading dimension ldr is added last when given (fp32 output;
+// 16-byte aligned rows).
+int launch_splitk_reduce(const LinearArgs& a, const float* part, int64_t S, const float* scale,
+                         const float* res = nullptr, int64_t ldr = 0);
 // Group-wise int4 with bf16 activations split over K (whole groups a split)
 // when the 128 x 128 tiles are too few to fill the GPU; the partial slices in
 // ws (staged_split_workspace bytes). TIQ_EUNSUPPORTED: no split planned.
@@ -151,9 +154,23 @@ int launch_staged_w4g(const LinearArgs& a, void* ws, size_t ws_bytes);
 // (digits_workspace bytes, then the fp32 slices of a product split over K,
 // digits_split_workspace bytes: with less it runs unsplit or in fewer splits).
 // gelu: the product takes gelu_tanh(x). Any M and N, K % 64 == 0.
+// fuse (fp32 output): what a prompt's block does around the product.
+struct PrefillFusion {
+    const float* ln_w = nullptr;  // LayerNorm of the rows of x before their split (K <= kDigitsLnMaxK)
+    const float* ln_b = nullptr;
+    float ln_eps = 1e-5f;
+    const float* res = nullptr;   // residual (M, N), added last
+    int64_t ldr = 0;
+    // columns N / 3 .. N - 1 (the keys, then the values of N / 192 heads of 64)
+    // go to k and v instead of y: row m = b T + t at b sb + head sh + t st
+    float* k = nullptr;
+    float* v = nullptr;
+    int64_t sb = 0, sh = 0, st = 0, T = 0;
+};
+constexpr int64_t kDigitsLnMaxK = 2048;
 size_t digits_workspace(int64_t M, int64_t K);
 size_t digits_split_workspace(int64_t M, int64_t N, int64_t K);
 bool digits_supported(const LinearArgs& a);
-int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu);
+int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu, const PrefillFusion& fuse = {});
 
 }  // namespace tiq

@@ -34,6 +34,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .config import GPTConfig
+from .qlinear import QuantLinear
 
 __all__ = ["GPT", "MLP", "Block", "CausalSelfAttention", "KVCache", "gelu_tanh"]
 
@@ -128,19 +129,48 @@ class KVCache:
     def values(self) -> list[torch.Tensor | None]:
         return [None if b is None else b[:, :, :n] for b, n in zip(self._v, self._len)]
 
-    def update(self, layer: int, k: torch.Tensor, v: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
-        """Append ``k, v`` ``(B, heads, T_new, head_dim)`` to ``layer``; return
-        views of the whole history ``(B, heads, length, head_dim)``."""
-        n, t = self._len[layer], k.shape[-2]
+    def _room(self, layer: int, t: int, dims: tuple[int, ...], like_k: torch.Tensor,
+              like_v: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """The layer's buffers, grown (a copy) if ``t`` more positions do not
+        fit; a first buffer is ``(*dims[:-1], capacity, dims[-1])``."""
+        n = self._len[layer]
         buf_k, buf_v = self._k[layer], self._v[layer]
         if buf_k is None or n + t > buf_k.shape[-2]:
             cap = max(16, 2 * (n + t))
-            grown_k = k.new_empty(*k.shape[:-2], cap, k.shape[-1])
-            grown_v = v.new_empty(*v.shape[:-2], cap, v.shape[-1])
+            grown_k = like_k.new_empty(*dims[:-1], cap, dims[-1])
+            grown_v = like_v.new_empty(*dims[:-1], cap, dims[-1])
             if buf_k is not None:
                 grown_k[:, :, :n] = buf_k[:, :, :n]
                 grown_v[:, :, :n] = buf_v[:, :, :n]
             self._k[layer], self._v[layer] = buf_k, buf_v = grown_k, grown_v
+        return buf_k, buf_v
+
+    def _append_slots(self, layer: int, batch: int, heads: int, t: int,
+                      like: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor] | None:
+        """The ``(batch, heads, t, 64)`` slots the next ``t`` positions of an fp32
+        GPU cache take, for a kernel that writes them (then :meth:`_advance`);
+        None where :meth:`update` has to copy: another type, device, shape or
+        layout, a tensor that autograd follows."""
+        buf = self._k[layer]
+        if buf is not None and (buf.dim() != 4 or buf.shape[:2] != (batch, heads) or buf.shape[3] != 64):
+            return None
+        bk, bv = self._room(layer, t, (batch, heads, 64), like, like)
+        n, s = self._len[layer], bk.stride()
+        if (bk.dtype != torch.float32 or bv.dtype != torch.float32 or bk.get_device() != like.get_device()
+                or bv.get_device() != like.get_device() or bk.requires_grad or bv.requires_grad
+                or bv.shape != bk.shape or bv.stride() != s or s[3] != 1 or min(s[:3]) < 64):
+            return None
+        return bk[:, :, n : n + t], bv[:, :, n : n + t]
+
+    def _advance(self, layer: int, t: int) -> tuple[torch.Tensor, torch.Tensor]:
+        n = self._len[layer] = self._len[layer] + t
+        return self._k[layer][:, :, :n], self._v[layer][:, :, :n]
+
+    def update(self, layer: int, k: torch.Tensor, v: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
+        """Append ``k, v`` ``(B, heads, T_new, head_dim)`` to ``layer``; return
+        views of the whole history ``(B, heads, length, head_dim)``."""
+        n, t = self._len[layer], k.shape[-2]
+        buf_k, buf_v = self._room(layer, t, (*k.shape[:-2], k.shape[-1]), k, v)
         buf_k[:, :, n : n + t] = k
         buf_v[:, :, n : n + t] = v
         self._len[layer] = n + t
@@ -193,6 +223,32 @@ def _fused_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, first: i
     return y
 
 
+def _as_is(module: nn.Module, cls: type) -> bool:
+    """A plain ``cls`` without hooks, whose call may be replaced by a kernel that
+    does the same."""
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and not module._backward_hooks and not module._backward_pre_hooks)
+
+
+def _prefill_rows(x: torch.Tensor) -> bool:
+    """Contiguous fp32 GPU rows that no gradient, tangent or global hook follows,
+    as :meth:`QuantLinear.forward_prefill` takes them."""
+    return (x.is_cuda and x.dtype is torch.float32 and x.dim() == 3 and x.numel() > 4 * x.shape[2]
+            and x.is_contiguous() and not (torch.is_grad_enabled() and x.requires_grad)
+            and torch.autograd.forward_ad._current_level < 0 and not nn.modules.module._has_any_global_hook())
+
+
+def _plain_ln(ln: nn.Module, x: torch.Tensor) -> bool:
+    """An nn.LayerNorm over the rows of ``x`` with fp32 parameters that no
+    gradient follows."""
+    if not _as_is(ln, nn.LayerNorm) or ln.normalized_shape != x.shape[2:]:
+        return False
+    w, b = ln.weight, ln.bias
+    return (w is not None and b is not None and w.dtype is torch.float32 and b.dtype is torch.float32
+            and w.get_device() == x.get_device() and b.get_device() == x.get_device() and w.is_contiguous()
+            and b.is_contiguous() and not (torch.is_grad_enabled() and (w.requires_grad or b.requires_grad)))
+
+
 class CausalSelfAttention(nn.Module):
     """Fused ``c_attn`` (q, k, v side by side), heads of 64 columns, causal
     attention over the cache, ``c_proj``."""
@@ -206,18 +262,43 @@ class CausalSelfAttention(nn.Module):
         self.c_proj = nn.Linear(config.n_embd, config.n_embd, bias=config.attn_bias)
 
     def forward(self, x: torch.Tensor, cache: KVCache | None = None) -> torch.Tensor:
+        return self.c_proj(self._heads(x, cache))
+
+    def _heads(self, x: torch.Tensor, cache: KVCache | None, ln: nn.LayerNorm | None = None) -> torch.Tensor | None:
+        """The attention of (the LayerNorm of) ``x`` before ``c_proj``, ``(B, T, C)``
+        rows. A quantized ``c_attn`` over a prompt applies ``ln`` itself and puts
+        keys and values straight into the cache, which saves their copies (two
+        of 10 us beside a 96 us product at 4096 rows of width 1600). With ``ln``:
+        None, nothing done, where the product does not apply it."""
         B, T, C = x.shape
         first = 0 if cache is None else cache.length(self.layer_idx)
+        qkv = None
+        if (ln is not None or (cache is not None and _prefill_rows(x))) and _as_is(self.c_attn, QuantLinear):
+            x2 = x.view(B * T, C)
+            if cache is not None and self.head_dim == 64 and self.c_attn.out_features == 3 * 64 * self.n_head:
+                slots = cache._append_slots(self.layer_idx, B, self.n_head, T, x)
+                q = None if slots is None else self.c_attn.forward_prefill(x2, ln=ln, kv=(*slots, T))
+                if q is not None:
+                    k, v = cache._advance(self.layer_idx, T)
+                    return self._attend(q.view(B, T, self.n_head, 64).transpose(1, 2), k, v, first)
+            if ln is not None:
+                qkv = self.c_attn.forward_prefill(x2, ln=ln)
+        if qkv is None:
+            if ln is not None:
+                return None
+            qkv = self.c_attn(x)
         # (B, T, 3C) -> (3, B, heads, T, hd): q, k, v heads in one permute
-        q, k, v = self.c_attn(x).view(B, T, 3, self.n_head, self.head_dim).permute(2, 0, 3, 1, 4).unbind(0)
+        q, k, v = qkv.view(B, T, 3, self.n_head, self.head_dim).permute(2, 0, 3, 1, 4).unbind(0)
         if cache is not None:
             k, v = cache.update(self.layer_idx, k, v)
+        return self._attend(q, k, v, first)
+
+    def _attend(self, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, first: int) -> torch.Tensor:
         p = self.config.dropout if self.training else 0.0
         y = _fused_attention(q, k, v, first, p)
-        if y is not None:
-            return self.c_proj(y)
-        y = _causal_softmax_attention(q, k, v, first, p)
-        return self.c_proj(y.transpose(1, 2).reshape(B, T, C))
+        if y is None:
+            y = _causal_softmax_attention(q, k, v, first, p).transpose(1, 2).flatten(2)
+        return y
 
 
 class MLP(nn.Module):
@@ -229,10 +310,19 @@ class MLP(nn.Module):
         self.c_proj = nn.Linear(4 * config.n_embd, config.n_embd, bias=config.mlp_bias)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        h = self.c_fc(x)
+        return self._project(self.c_fc(x))
+
+    def _project(self, h: torch.Tensor, residual: torch.Tensor | None = None) -> torch.Tensor:
+        """``c_proj(gelu_tanh(h))``, plus ``residual``."""
+        if _prefill_rows(h) and _as_is(self.c_proj, QuantLinear):
+            y = self.c_proj.forward_prefill(h.view(-1, h.shape[2]), gelu=True, residual=residual)
+            if y is not None:
+                return y.view(*h.shape[:2], -1)
         fused = getattr(self.c_proj, "forward_gelu_in", None)  # a quantized c_proj over a prefill's rows
         y = fused(h) if fused is not None else None
-        return y if y is not None else self.c_proj(gelu_tanh(h))
+        if y is None:
+            y = self.c_proj(gelu_tanh(h))
+        return y if residual is None else residual + y
 
 
 class Block(nn.Module):
@@ -251,8 +341,36 @@ class Block(nn.Module):
         return F.dropout(t, self.p_drop, training=True) if self.training and self.p_drop else t
 
     def forward(self, x: torch.Tensor, cache: KVCache | None = None) -> torch.Tensor:
+        y = self._prefill(x, cache)
+        if y is not None:
+            return y
         x = x + self._drop(self.attn(self.ln_1(x), cache))
         return x + self._drop(self.mlp(self.ln_2(x)))
+
+
+    def _prefill(self, x: torch.Tensor, cache: KVCache | None) -> torch.Tensor | None:
+        """The block over a prompt's rows with quantized Linears: both
+        LayerNorms inside the Linear that follows, both residual adds at the end
+        of the Linear before (four passes over x fewer; each step that a Linear
+        does not take runs as its own op). None, nothing done, where the block
+        has to run module by module: hooks, replaced modules, a gradient,
+        dropout, rows that ``c_attn`` does not take as digit planes."""
+        attn, mlp = self.attn, self.mlp
+        if not (_prefill_rows(x) and _as_is(attn.c_attn, QuantLinear) and _as_is(attn.c_proj, QuantLinear)
+                and _as_is(mlp.c_fc, QuantLinear) and _as_is(mlp.c_proj, QuantLinear)
+                and _as_is(attn, CausalSelfAttention) and _as_is(mlp, MLP)
+                and _plain_ln(self.ln_1, x) and _plain_ln(self.ln_2, x)
+                and not (self.training and (self.p_drop or attn.config.dropout))):
+            return None
+        B, T, C = x.shape
+        heads = attn._heads(x, cache, self.ln_1)
+        if heads is None:
+            return None
+        y = attn.c_proj.forward_prefill(heads.view(B * T, -1), residual=x)
+        x = x + attn.c_proj(heads) if y is None else y.view(B, T, C)
+        h = mlp.c_fc.forward_prefill(x.view(B * T, C), ln=self.ln_2)
+        h = mlp.c_fc(self.ln_2(x)) if h is None else h.view(B, T, -1)
+        return mlp._project(h, x)
 
 
 def _refuse_unsupported(config: GPTConfig) -> None:

@@ -126,6 +126,43 @@ class QuantLinear(nn.Module):
             _lib.check(rc, f"quantized linear over gelu_tanh ({self.fmt}, M={M}, K={K}, N={N})")
         return y.view(*lead, N)
 
+    def forward_prefill(self, x2: torch.Tensor, ln: nn.LayerNorm | None = None, gelu: bool = False,
+                        residual: torch.Tensor | None = None,
+                        kv: tuple[torch.Tensor, torch.Tensor, int] | None = None) -> torch.Tensor | None:
+        """``self(ln(x2))``, ``self(gelu_tanh(x2))`` or ``self(x2)`` plus
+        ``residual`` for contiguous fp32 GPU rows ``(M, K)``, in the two
+        launches of the plain product (``tiq_linear_prefill_ws``). ``kv`` = (keys,
+        values, T): this is a ``c_attn`` over M / T sequences whose keys and
+        values go to those ``(B, heads, T, 64)`` cache slots; the result is the
+        query columns. None (nothing launched) where the rows do not take the
+        matrix cores as digit planes; the caller then takes the separate steps."""
+        M, K = x2.shape
+        N, fmt = self.out_features, self.fmt
+        if M <= 4 or K != self.in_features or (residual is not None and residual.shape[-1] != N):
+            return None
+        L = _lib.lib()
+        ws_bytes = L.tiq_linear_workspace(_WF[fmt], _lib.F32, M, K, N)
+        if not ws_bytes:
+            return None
+        cols = N if kv is None else N // 3
+        y = x2.new_empty((M, cols))
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x2.device)
+        codes, scale, bias = self._buffers["codes"], self._buffers["scale"].data_ptr(), self._parameters["bias"]
+        grouped = fmt == FMT_W4G
+        lw, lb, eps = (None, None, 1e-5) if ln is None else (ln.weight.data_ptr(), ln.bias.data_ptr(), ln.eps)
+        k, v, strides, T = (None, None, (0, 0, 0), 0) if kv is None else (kv[0].data_ptr(), kv[1].data_ptr(),
+                                                                          kv[0].stride()[:3], kv[2])
+        rc = L.tiq_linear_prefill_ws(
+            x2.data_ptr(), M, K, K, codes.data_ptr(), _WF[fmt], None if grouped else scale, scale if grouped else None,
+            self.group_size, None if bias is None else bias.data_ptr(), N, y.data_ptr(), cols, lw, lb, eps, gelu,
+            None if residual is None else residual.data_ptr(), 0 if residual is None else N, k, v, *strides, T,
+            ws.data_ptr(), ws_bytes, _lib.stream_of(x2))
+        if rc == _lib.EUNSUPPORTED:
+            return None
+        if rc:
+            _lib.check(rc, f"quantized prefill linear ({fmt}, M={M}, K={K}, N={N})")
+        return y
+
     @property
     def weight(self) -> torch.Tensor:
         """The dequantized ``W_hat`` (fp32, ``(N, K)``), as the reference stores it."""

@@ -498,6 +498,27 @@ int tiq_linear_gelu_in_ws(const float* x, int64_t M, int64_t K, int64_t ldx, con
                           const float* scale, const uint16_t* scale_f16, int group, const float* bias, int64_t N,
                           float* y, int64_t ldy, void* workspace, size_t workspace_bytes, void* stream);
 
+/* A quantized Linear over a prompt's fp32 rows with what its block does around
+ * it (model.py:227-320,351-355,434-441 at M = B * T rows):
+ *     y = LayerNorm(x) or gelu_tanh(x) or x, times W^T, + bias, + residual.
+ * ln_weight / ln_bias (K each, 16-byte aligned, K <= 2048) or NULL; gelu_in is
+ * exclusive of them. residual (M, N) with leading dimension ld_residual, added
+ * last, or NULL; it may not overlap y. k_out / v_out (both or neither, exclusive
+ * of residual): the product is a c_attn, N = 3 C with C % 64 == 0, whose key and
+ * value columns go to the caches instead of y: row m = b T + t, head i, dim d at
+ * b kv_sb + i kv_sh + t kv_st + d (elements; M a multiple of T); y then holds the
+ * C query columns (ldy >= C). The workspace is tiq_linear_workspace's for
+ * fp32 rows. TIQ_EUNSUPPORTED, with nothing launched, where that size is 0 (the
+ * rows do not take the matrix cores as digit planes), for the layouts
+ * tiq_linear_w8_ws would not take on them, and for k_out with so few tiles that
+ * the product is split over K; TIQ_EWORKSPACE when the workspace is short. */
+int tiq_linear_prefill_ws(const float* x, int64_t M, int64_t K, int64_t ldx, const void* w, int w_format,
+                          const float* scale, const uint16_t* scale_f16, int group, const float* bias, int64_t N,
+                          float* y, int64_t ldy, const float* ln_weight, const float* ln_bias, float ln_eps,
+                          int gelu_in, const float* residual, int64_t ld_residual, float* k_out, float* v_out,
+                          int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int64_t T, void* workspace,
+                          size_t workspace_bytes, void* stream);
+
 /* x[b] = wte[tokens[b]] + wpe[*pos]  (model.py:561-564 for one position). */
 int tiq_embed_tokens(const int64_t* tokens, const int64_t* pos, const float* wte, int64_t vocab,
                      const float* wpe, int64_t n_positions, int64_t batch, int64_t n_embd, float* x,
