@@ -19,22 +19,20 @@ namespace {
 constexpr int kGroup = 128;  // two k64 steps
 constexpr int kBN = 128;
 
-// Tile height: 224 rows, or 128 where 128-row tiles cover M with fewer rows
-// than 224-row ones and all fit on the CUs at once (GPT-2-XL shapes: M = 256,
-// 256 rows of work instead of 448, 13-22% faster; M = 1024 with N = 1600,
-// 4-9% faster).
-int w4g_rows(int64_t M, int64_t N) {
-    const bool fewer_rows = (M + 127) / 128 * 128 < (M + 223) / 224 * 224;
-    return fewer_rows && ((M + 127) / 128) * ((N + kBN - 1) / kBN) <= 256 ? 128 : 224;
-}
+// 128 x 128 tiles, two workgroups a CU (the partial and the summed tiles fit 256
+// registers), whose loads and folds hide beside each other's MFMAs: ahead of one
+// 224 x 128 workgroup a CU at every GPT-2 shape and row count (us, 224 rows / 128:
+// 1600 x 4800 M = 4096 90 / 78, 1600 x 6400 M = 4096 119 / 104, 1024 x 4096 M =
+// 2048 42 / 23, 768 x 768 M = 1024 17 / 11).
+constexpr int kBM = 128;
 
 // One workgroup per tile (the group-wise kernel does not run persistent);
 // gridDim.z = S splits of whole groups, fp32 slices without bias when S > 1.
-template <int BM, typename TY>
+template <typename TY>
 int run_w4g(const LinearArgs& a, TY* y, int64_t ldy, const float* bias, int64_t S) {
-    const int64_t tiles = ((a.M + BM - 1) / BM) * ((a.N + kBN - 1) / kBN);
+    const int64_t tiles = ((a.M + kBM - 1) / kBM) * ((a.N + kBN - 1) / kBN);
     const int ngroups = (int)((a.K + kGroup - 1) / kGroup);
-    hipLaunchKernelGGL((gemm_staged<BM, kBN, 1, kW4G, TY>), dim3((unsigned)tiles, 1, (unsigned)S), dim3(256), 0,
+    hipLaunchKernelGGL((gemm_staged<kBM, kBN, 1, kW4G, TY, false, 2, 2>), dim3((unsigned)tiles, 1, (unsigned)S), dim3(256), 0,
                        a.stream, static_cast<const uint16_t*>(a.x), a.ldx, a.w, a.ldw, nullptr, bias, y, ldy,
                        (int)a.M, (int)a.N, (int)a.K, (int)a.K, a.scale16, ngroups, nullptr);
     return launch_status();
@@ -56,35 +54,39 @@ bool staged_w4g_supported(const LinearArgs& a) {
     return true;
 }
 
-// Splits of whole groups when the tiles fill less than a round of 256 CUs (at
-// most 8, at most one a group, within the workspace); 1: none, also for 96
-// tiles or more with at most 32 k64 steps, where the slices' trip through
-// memory costs more than the idle CUs (M = 256 and 1024 at K = 1600: 5-9%).
+// Splits of whole groups (at most 8, within the workspace): the one with the least
+// time by a model of the timings over GPT-2's shapes at M = 64 .. 4096: per k64
+// step 0.585 us with one workgroup on a CU, 0.95 with two; 3.9 us a launch; for
+// a split 3.8 us and 0.3 us a MB of slices for the sum. Its choices take 0.6% more
+// than the best splits altogether (us, unsplit / chosen: 6400 x 1600 M = 1024 63 /
+// 40, M = 512 63 / 27; 3072 x 768 M = 2048 33 / 26; 768 x 2304 M = 256 11.3 / none).
 int64_t staged_w4g_splits(int64_t M, int64_t N, int64_t K, size_t ws_bytes) {
-    const int bm = w4g_rows(M, N);
-    const int64_t tiles = ((M + bm - 1) / bm) * ((N + kBN - 1) / kBN);
-    if (tiles >= 96 && K / BK <= 32) return 1;
+    const int64_t tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
     const int64_t groups = (K + kGroup - 1) / kGroup;
-    int64_t S = std::min<int64_t>(std::min<int64_t>(256 / std::max<int64_t>(tiles, 1), groups), 8);
-    S = std::min<int64_t>(S, (int64_t)(ws_bytes / (size_t)(M * N * 4)));
-    return std::max<int64_t>(S, 1);
+    int64_t most = std::min<int64_t>(std::min<int64_t>(512 / std::max<int64_t>(tiles, 1), groups), 8);
+    most = std::min<int64_t>(most, (int64_t)(ws_bytes / (size_t)(M * N * 4)));
+    int64_t best = 1;
+    double best_t = 1e30;
+    for (int64_t S = 1; S <= most; ++S) {
+        const double steps = 2.0 * (double)((groups + S - 1) / S);
+        double t = steps * (tiles * S <= 256 ? 0.585 : 0.95);
+        if (S > 1) t += 3.8 + 0.3e-6 * (double)(S * M * N * 4);
+        if (t < best_t) best_t = t, best = S;
+    }
+    return best;
 }
 
 int launch_staged_w4g(const LinearArgs& a, void* ws, size_t ws_bytes) {
     if (!staged_w4g_supported(a)) return TIQ_EUNSUPPORTED;
     const int64_t S = (ws && aligned(ws, 16)) ? staged_w4g_splits(a.M, a.N, a.K, ws_bytes) : 1;
-    const bool short_m = w4g_rows(a.M, a.N) == 128;
     if (S > 1 && a.M * a.N * S <= 0x7fffffffLL) {
         float* part = static_cast<float*>(ws);
-        int rc = short_m ? run_w4g<128, float>(a, part, a.N, nullptr, S) : run_w4g<224, float>(a, part, a.N, nullptr, S);
+        const int rc = run_w4g<float>(a, part, a.N, nullptr, S);
         if (rc != TIQ_OK) return rc;
         return launch_splitk_reduce(a, part, S, nullptr);
     }
-    if (a.y_dtype == TIQ_F32)
-        return short_m ? run_w4g<128, float>(a, static_cast<float*>(a.y), a.ldy, a.bias, 1)
-                       : run_w4g<224, float>(a, static_cast<float*>(a.y), a.ldy, a.bias, 1);
-    return short_m ? run_w4g<128, uint16_t>(a, static_cast<uint16_t*>(a.y), a.ldy, a.bias, 1)
-                   : run_w4g<224, uint16_t>(a, static_cast<uint16_t*>(a.y), a.ldy, a.bias, 1);
+    if (a.y_dtype == TIQ_F32) return run_w4g<float>(a, static_cast<float*>(a.y), a.ldy, a.bias, 1);
+    return run_w4g<uint16_t>(a, static_cast<uint16_t*>(a.y), a.ldy, a.bias, 1);
 }
 
 }  // namespace tiq

@@ -93,8 +93,9 @@ __device__ __forceinline__ void staged_tile_of(int i, int& tm, int& tn, int tile
 // weights staged through LDS): a stage's loads are issued DEPTH - 1 steps
 // before its LDS store, for tiles whose k64 step is too short to cover a trip
 // to memory (few tiles a CU at M = 256 .. 1024).
-template <int BM, int BN, int WMW, int FMT, typename TY, bool STAMP = false, int DEPTH = 2>
-__global__ __launch_bounds__(256, 1) void gemm_staged(
+// OCC: workgroups a CU that the registers are held to.
+template <int BM, int BN, int WMW, int FMT, typename TY, bool STAMP = false, int DEPTH = 2, int OCC = 1>
+__global__ __launch_bounds__(256, OCC) void gemm_staged(
     const uint16_t* __restrict__ x, int64_t ldx, const uint8_t* __restrict__ w, int64_t ldw,
     const float* __restrict__ scale, const float* __restrict__ bias, TY* __restrict__ y, int64_t ldy, int M, int N,
     int K, int kw, const uint16_t* __restrict__ scale16, int ngroups, uint64_t* stamp) {
