@@ -911,6 +911,96 @@ __global__ __launch_bounds__(kWaves * 64, 1) void stream_f32_kernel(const uint16
     });
 }
 
+// stream_f32_kernel for K <= 8 PU 32: a wavefront meets the same PU units of the
+// activations in every tile, so it keeps their first two planes in registers and
+// the third in its part of LDS, and only weights are read per tile (with the planes
+// from L2 each time, 6 KB a unit passed the vector memory path beside 4 KB of
+// weights). The same products in the same order: the same bits. A slot is loaded
+// for the next tile as soon as it is consumed. K = 1024, 8 rows, 50257 weight rows
+// 45 -> 39 us (5.3 TB/s); at seven units a wavefront (K = 1600) there was nothing
+// to gain (78 -> 77 us), and such K stay with the ring.
+template <int PU>
+__global__ __launch_bounds__(kWaves * 64, 1) void stream_f32_held_kernel(const uint16_t* __restrict__ x3, int M, int K,
+                                                                        const uint8_t* __restrict__ wt, int N,
+                                                                        float* __restrict__ y, int64_t ldy) {
+    __shared__ float red[kWaves][32][33];
+    __shared__ __attribute__((aligned(16))) u32x4 low[kWaves][PU][2][64];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = lane & 31, h = lane >> 5;
+    const int U = K / 32, m0 = blockIdx.y * 32;
+    const int u0 = wave * U / kWaves, cnt = (wave + 1) * U / kWaves - u0;  // 1 .. PU (the host checks)
+    const int T = (N + 31) / 32, G = gridDim.x;
+    const uint8_t* wl = wt + (int64_t)u0 * 4096 + lane * 16;
+    u32x4 wring[PU][4];
+    auto issue = [&](int tile, auto unit) __attribute__((always_inline)) {
+        constexpr int c = decltype(unit)::value;
+        if (c < cnt && tile < T) {
+            const uint8_t* wb = wl + ((int64_t)tile * U + c) * 4096;
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                wring[c][q] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(wb + 1024 * q));
+        }
+    };
+    for_each_slot(std::make_integer_sequence<int, PU>{}, [&](auto c) __attribute__((always_inline)) { issue((int)blockIdx.x, c); });
+    u32x4 xh[PU][2][2];
+    {
+        const uint16_t* x3t = x3 + ((int64_t)blockIdx.y * U + u0) * 6 * 64 * 8 + lane * 8;
+        const bool xrow_ok = m0 + r < M;
+        const u32x4 z = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int c = 0; c < PU; ++c)
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                u32x4 t[3];
+#pragma unroll
+                for (int q = 0; q < 3; ++q)
+                    t[q] = *reinterpret_cast<const u32x4*>(x3t + (((int64_t)min(c, cnt - 1) * 3 + q) * 2 + e) * 64 * 8);
+                xh[c][0][e] = xrow_ok ? t[0] : z;
+                xh[c][1][e] = xrow_ok ? t[1] : z;
+                low[wave][c][e][lane] = xrow_ok ? t[2] : z;
+            }
+    }
+    for (int tile = blockIdx.x; tile < T; tile += G) {
+        floatx16 acc = {};
+        for_each_slot(std::make_integer_sequence<int, PU>{}, [&](auto unit) __attribute__((always_inline)) {
+            constexpr int c = decltype(unit)::value;
+            if (c < cnt) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const bf16x8 x0 = __builtin_bit_cast(bf16x8, xh[c][0][e]);
+                    const bf16x8 x1 = __builtin_bit_cast(bf16x8, xh[c][1][e]);
+                    const bf16x8 x2 = __builtin_bit_cast(bf16x8, low[wave][c][e][lane]);
+                    float wf[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) wf[i] = __uint_as_float(wring[c][2 * e + i / 4][i % 4]);
+                    bf16x8 w0, w1, w2;
+                    split3(wf, w0, w1, w2);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0, x0, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0, x1, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1, x0, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w0, x2, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w1, x1, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w2, x0, acc, 0, 0, 0);
+                }
+            }
+            issue(tile + G, unit);
+        });
+#pragma unroll
+        for (int q = 0; q < 16; ++q) red[wave][r][8 * (q >> 2) + 4 * h + (q & 3)] = acc[q];
+        __syncthreads();
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt) {  // 1024 outputs, two per thread, wavefront order
+            const int o = threadIdx.x + kWaves * 64 * tt;
+            const int m = o >> 5, nn = o & 31;
+            float v = 0.f;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) v += red[w][m][nn];
+            if (m0 + m < M && 32 * tile + nn < N) y[(int64_t)(m0 + m) * ldy + 32 * tile + nn] = v;
+        }
+        __syncthreads();  // red is free for the next tile
+    }
+}
+
 size_t round256(size_t b) { return (b + 255) / 256 * 256; }
 
 // Workspace: the split activation planes, row tiles x 32 x 3K bf16 in operand order.
@@ -1085,9 +1175,15 @@ static int run_decode_f32_tiles(const LinearArgs& a, const uint16_t* x_planes, c
     if (!aligned(a.w, 16) || !aligned(x_planes, 16)) return TIQ_EALIGN;
     const int64_t T = (a.N + 31) / 32;
     const dim3 grid((unsigned)std::min<int64_t>(T, 256), (unsigned)((a.M + 31) / 32));
-    hipLaunchKernelGGL(stream_f32_kernel, grid, dim3(kWaves * 64), 0, a.stream, x_planes, (int)a.M, (int)a.K, a.w,
-                       (int)a.N, static_cast<float*>(a.y), a.ldy);
-    return launch_status();
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), 0, a.stream, x_planes, (int)a.M, (int)a.K, a.w, (int)a.N,
+                           static_cast<float*>(a.y), a.ldy);
+        return launch_status();
+    };
+    const int64_t units = (a.K / 32 + kWaves - 1) / kWaves;  // a wavefront's
+    if (units <= 4) return launch(stream_f32_held_kernel<4>);
+    if (units <= 5) return launch(stream_f32_held_kernel<5>);
+    return launch(stream_f32_kernel);
 }
 
 int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float* next_ln_w,
