@@ -249,6 +249,28 @@ def _plain_ln(ln: nn.Module, x: torch.Tensor) -> bool:
             and b.is_contiguous() and not (torch.is_grad_enabled() and (w.requires_grad or b.requires_grad)))
 
 
+def _head_logits(head: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``head(x)``; a plain bias-free fp32 ``nn.Linear`` over more than 64 rows that no
+    gradient follows goes through ``tiq_linear_f32_ws``."""
+    if _prefill_rows(x) and _as_is(head, nn.Linear) and head.bias is None:
+        w = head.weight
+        B, T, C = x.shape
+        if (type(w) is nn.Parameter and w.dtype is torch.float32 and w.get_device() == x.get_device()
+                and w.is_contiguous() and w.shape[1] == C and not (torch.is_grad_enabled() and w.requires_grad)
+                and not torch.is_autocast_enabled("cuda")):
+            from . import _lib
+
+            L, M, N = _lib.lib(), B * T, w.shape[0]
+            ws_bytes = L.tiq_linear_f32_workspace(M, C, N)
+            if ws_bytes and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+                y = x.new_empty((B, T, N))
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+                _lib.check(L.tiq_linear_f32_ws(x.data_ptr(), M, C, C, w.data_ptr(), C, N, y.data_ptr(), N,
+                                               ws.data_ptr(), ws_bytes, _lib.stream_of(x)), "lm_head over a batch")
+                return y
+    return head(x)
+
+
 class CausalSelfAttention(nn.Module):
     """Fused ``c_attn`` (q, k, v side by side), heads of 64 columns, causal
     attention over the cache, ``c_proj``."""
@@ -467,7 +489,7 @@ class GPT(nn.Module):
             x = block(x, cache)
         if last_only:
             x = x[:, -1:]
-        logits = self.lm_head(self.ln_f(x))
+        logits = _head_logits(self.lm_head, self.ln_f(x))
         out: dict[str, Any] = {"logits": logits}
         if targets is not None:
             out["loss"] = F.cross_entropy(logits.flatten(0, 1), targets.reshape(-1), ignore_index=-100)

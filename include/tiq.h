@@ -519,6 +519,16 @@ int tiq_linear_prefill_ws(const float* x, int64_t M, int64_t K, int64_t ldx, con
                           int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int64_t T, void* workspace,
                           size_t workspace_bytes, void* stream);
 
+/* y = x w^T, fp32 rows against fp32 weights: the tied lm_head over every
+ * position of a batch (model.py:585) on the bf16 matrix cores, both operands as
+ * three bf16 planes, as accurate as an fp32 GEMM (an infinite operand gives NaN).
+ * x (M, K) and w (N, K) 16-byte aligned, ldx % 4 == 0, ldw % 4 == 0, K % 32 == 0,
+ * M >= 65, N >= 4096: TIQ_EUNSUPPORTED for other sizes, whose workspace is 0;
+ * y any alignment. The workspace holds the planes of x. */
+size_t tiq_linear_f32_workspace(int64_t M, int64_t K, int64_t N);
+int tiq_linear_f32_ws(const float* x, int64_t M, int64_t K, int64_t ldx, const float* w, int64_t ldw, int64_t N,
+                      float* y, int64_t ldy, void* workspace, size_t workspace_bytes, void* stream);
+
 /* x[b] = wte[tokens[b]] + wpe[*pos]  (model.py:561-564 for one position). */
 int tiq_embed_tokens(const int64_t* tokens, const int64_t* pos, const float* wte, int64_t vocab,
                      const float* wpe, int64_t n_positions, int64_t batch, int64_t n_embd, float* x,
