@@ -44,8 +44,9 @@ constexpr int kDigits = 4;
 // 16 l + j of it the digit of row 32 t + l % 32, column 32 u + 16 (l / 32) + j
 // (NIB: the even columns of the 16 first, then the odd ones -- the order in
 // which nibble weights unpack), so the product's loads and LDS accesses are
-// all contiguous. One workgroup per 8 rows: 8 rows' chunks of a block are 128
-// consecutive bytes, a whole cache line a store. rs[m] = 2^(e_m - 29), NaN for
+// all contiguous. One workgroup per R rows: 8 rows' chunks of a block are 128
+// consecutive bytes, a whole cache line a store (4 rows where that would leave
+// CUs idle). rs[m] = 2^(e_m - 29), NaN for
 // a row holding an infinity or NaN (every output of it is then NaN).
 // IT: 1024-column passes held in registers; 0: the row is read twice.
 constexpr int kSplitThreads = 512;
@@ -82,18 +83,19 @@ __device__ __forceinline__ void store_digits(const float (&v)[16], float mul, ui
 // LN: the digits of LayerNorm(x) (two-pass mean and biased variance as torch;
 // the row already sits in registers, so the LayerNorm's own pass -- a read and a
 // write of x, 9 us at 4096 x 1600 -- costs two exchanges more here).
-template <int IT, bool NIB, bool LN>
+template <int IT, int R, bool NIB, bool LN>
 __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float* __restrict__ x, int64_t ldx, int M,
                                                                      int K, uint8_t* __restrict__ xt,
                                                                      float* __restrict__ rs, bool gelu,
                                                                      const float* __restrict__ ln_w,
                                                                      const float* __restrict__ ln_b, float ln_eps) {
     static_assert(!LN || IT > 0, "LayerNorm needs the row in registers");
-    constexpr int WV = kSplitThreads / 64, CT = kSplitThreads / 8;  // 16-column chunks a pass
-    __shared__ uint32_t am[WV][8];
-    __shared__ float ls[2][WV][8];
-    const int tid = threadIdx.x, r8 = tid & 7, c0 = tid >> 3;
-    const int m = blockIdx.x * 8 + r8;
+    static_assert(R == 8 || R == 4, "whole quads of rows");
+    constexpr int WV = kSplitThreads / 64, CT = kSplitThreads / R;  // 16-column chunks a pass
+    __shared__ uint32_t am[WV][R];
+    __shared__ float ls[2][WV][R];
+    const int tid = threadIdx.x, row = tid % R, c0 = tid / R;
+    const int m = blockIdx.x * R + row;
     const int NC = K / 16, U = K / 32;
     // A quad of lanes reads 64 consecutive bytes of each of its four rows in
     // turn (16 segments a load instruction, not 64), then transposes: each lane
@@ -102,7 +104,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
     const float* xq[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        xq[i] = x + (int64_t)min((int)blockIdx.x * 8 + (r8 & 4) + i, M - 1) * ldx + 4 * j4;
+        xq[i] = x + (int64_t)min((int)blockIdx.x * R + (row & 4) + i, M - 1) * ldx + 4 * j4;
     const bool odd = j4 & 1, high = j4 & 2;
     auto load = [&](int c, float (&v)[16]) {
 #pragma unroll
@@ -134,15 +136,15 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
 #pragma unroll
         for (int it = 0; it < IT; ++it) load(min(c0 + CT * it, NC - 1), v[it]);  // past the row: its last chunk again
         if constexpr (LN) {
-            // a row is the 64 threads of equal tid % 8: eight lanes of each wavefront
+            // a row is the threads of equal tid % R: 64 / R lanes of each wavefront
             auto row_sum = [&](float s, int slot) {
 #pragma unroll
-                for (int off = 32; off >= 8; off >>= 1) s += __shfl_xor(s, off, 64);
-                if ((tid & 63) < 8) ls[slot][tid >> 6][r8] = s;
+                for (int off = 32; off >= R; off >>= 1) s += __shfl_xor(s, off, 64);
+                if ((tid & 63) < R) ls[slot][tid >> 6][row] = s;
                 __syncthreads();
                 float t = 0.f;
 #pragma unroll
-                for (int w = 0; w < WV; ++w) t += ls[slot][w][r8];
+                for (int w = 0; w < WV; ++w) t += ls[slot][w][row];
                 return t;
             };
             float s = 0.f;
@@ -189,11 +191,11 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
         }
     }
 #pragma unroll
-    for (int off = 32; off >= 8; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
-    if ((tid & 63) < 8) am[tid >> 6][r8] = mx;
+    for (int off = 32; off >= R; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
+    if ((tid & 63) < R) am[tid >> 6][row] = mx;
     __syncthreads();
 #pragma unroll
-    for (int w = 0; w < WV; ++w) mx = max(mx, am[w][r8]);
+    for (int w = 0; w < WV; ++w) mx = max(mx, am[w][row]);
     // rows below 2^-97 share its exponent: both powers of two stay normal
     const int e = max((int)(mx >> 23) - 127, -97);
     const bool finite = mx < 0x7f800000u;
@@ -609,20 +611,33 @@ int dispatch_digits(const LinearArgs& a, DigitTile tile, const uint8_t* xt, cons
     }
 }
 
+// Rows below which a split workgroup takes four rows of more than 1024 columns, not
+// eight: twice the workgroups and half a thread's chain where they do not fill the
+// chip (with the product, us, eight / four: 3072 x 768 M = 512 24.8 / 22.5, 6400 x
+// 1600 M = 128 27.9 / 24.4, M = 1024 68.3 / 66.1; level from M = 1536, where the
+// eight-row stores are whole cache lines).
+constexpr int64_t kSplitWideRows = 1280;
+
 template <bool NIB>
 int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu, const PrefillFusion& f) {
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)((a.M + 7) / 8)), dim3(kSplitThreads), 0, a.stream,
+    auto launch = [&](auto kernel, int rows) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)((a.M + rows - 1) / rows)), dim3(kSplitThreads), 0, a.stream,
                            static_cast<const float*>(a.x), a.ldx, (int)a.M, (int)a.K, xt, rs, gelu, f.ln_w, f.ln_b,
                            f.ln_eps);
         return launch_status();
     };
-    if (f.ln_w) return a.K <= 1024 ? launch(split_digits_kernel<1, NIB, true>) : launch(split_digits_kernel<2, NIB, true>);
-    if (a.K <= 1024) return launch(split_digits_kernel<1, NIB, false>);
-    if (a.K <= 2048) return launch(split_digits_kernel<2, NIB, false>);
-    if (a.K <= 4096) return launch(split_digits_kernel<4, NIB, false>);
-    if (a.K <= 7168) return launch(split_digits_kernel<7, NIB, false>);
-    return launch(split_digits_kernel<0, NIB, false>);
+    if (a.K > 1024 && a.K <= 8192 && a.M < kSplitWideRows) {
+        if (f.ln_w) return launch(split_digits_kernel<1, 4, NIB, true>, 4);
+        if (a.K <= 2048) return launch(split_digits_kernel<1, 4, NIB, false>, 4);
+        if (a.K <= 4096) return launch(split_digits_kernel<2, 4, NIB, false>, 4);
+        return launch(split_digits_kernel<4, 4, NIB, false>, 4);
+    }
+    if (f.ln_w) return a.K <= 1024 ? launch(split_digits_kernel<1, 8, NIB, true>, 8) : launch(split_digits_kernel<2, 8, NIB, true>, 8);
+    if (a.K <= 1024) return launch(split_digits_kernel<1, 8, NIB, false>, 8);
+    if (a.K <= 2048) return launch(split_digits_kernel<2, 8, NIB, false>, 8);
+    if (a.K <= 4096) return launch(split_digits_kernel<4, 8, NIB, false>, 8);
+    if (a.K <= 7168) return launch(split_digits_kernel<7, 8, NIB, false>, 8);
+    return launch(split_digits_kernel<0, 8, NIB, false>, 8);
 }
 
 template <int FMT>
