@@ -38,6 +38,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kDigits = 4;
+constexpr int kPairSteps = 4;  // k64 steps of a group whose digit sums join in int32: 256 (2^14 257) < 2^31
 
 // The digit planes in MFMA operand order: for row tile t (32 rows), unit u (32
 // columns) and digit d (0 lowest) a 1 KB block at ((t U + u) 4 + d) 1024, byte
@@ -232,10 +233,12 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
 // FMT kW8 (codes) or kW4 (the reference's nibbles, unpacked to 16 (n - 8) on
 // the LDS store: the 16 is taken out with the scale).
 // kW4G (group-wise nibbles, groups of gs k64 steps, an fp16 scale per row and
-// group): a group's four sums, exact integers below 2^29 as two combined pairs,
-// become one fp32 value a result, which times the group's scale is added to
-// fp32 sums -- the lanes of a result register share no column, so a scale is
-// one load a lane and column tile; the next group starts from zero.
+// group): a group's four sums become one fp32 value a result, which times the
+// group's scale is added to fp32 sums -- the lanes of a result register share no
+// column, so a scale is one load a lane and column tile; the next group starts
+// from zero. A digit and a code reach 2^7 each, so a sum reaches 2^14 a column:
+// two of them join in int32 (256 times one plus the other) up to 256 columns, in
+// fp32 for wider groups.
 // gridDim.z > 1: split over K, workgroup z writes fp32 slice z of y (no bias).
 // Out (fp32 output, unsplit): a residual added last, or a c_attn whose key and
 // value columns go to the cache (a 32-column tile lies within one head, so its
@@ -380,6 +383,13 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
         }
     };
 
+    // an output's four digit sums in fp32
+    auto joined = [&](const i32x16 (&a)[kDigits], int q) -> float {
+        float f = (float)a[3][q];
+        f = fmaf(f, 256.f, (float)a[2][q]);
+        f = fmaf(f, 256.f, (float)a[1][q]);
+        return fmaf(f, 256.f, (float)a[0][q]);
+    };
     // group-wise: fp32 sums, the current group's scales (fp16 bits as loaded)
     float sum[GROUPED ? TN : 1][GROUPED ? TM : 1][16];
     uint16_t sg[TN];
@@ -397,9 +407,15 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int q = 0; q < 16; ++q) {
-                        const float hi = (float)((acc[j][i][3][q] << 8) + acc[j][i][2][q]);
-                        const float lo = (float)((acc[j][i][1][q] << 8) + acc[j][i][0][q]);
-                        sum[j][i][q] = fmaf(fmaf(hi, 65536.f, lo), sc, sum[j][i][q]);
+                        float v;
+                        if (gs <= kPairSteps) {
+                            const float hi = (float)((acc[j][i][3][q] << 8) + acc[j][i][2][q]);
+                            const float lo = (float)((acc[j][i][1][q] << 8) + acc[j][i][0][q]);
+                            v = fmaf(hi, 65536.f, lo);
+                        } else {
+                            v = joined(acc[j][i], q);
+                        }
+                        sum[j][i][q] = fmaf(v, sc, sum[j][i][q]);
                     }
             }
         }
@@ -477,10 +493,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
             if constexpr (GROUPED) {
                 return sum[j][i][q];
             } else {
-                float f = (float)acc[j][i][3][q];
-                f = fmaf(f, 256.f, (float)acc[j][i][2][q]);
-                f = fmaf(f, 256.f, (float)acc[j][i][1][q]);
-                return fmaf(f, 256.f, (float)acc[j][i][0][q]);
+                return joined(acc[j][i], q);
             }
         };
         tile += gridDim.x;

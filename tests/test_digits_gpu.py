@@ -110,6 +110,32 @@ def test_digit_planes_groupwise(dev, K, N, M, group):
     assert torch.equal(yb, y.bfloat16())
 
 
+# Groups to either side of the 256 columns whose digit sums join in int32, with
+# nothing that cancels: constant rows whose digits are (lowest first) (-128, 103,
+# 102, 38), (0, 0, 0, 32) and (-128, 21, -82, 64), weights of one sign, so every
+# digit sum is as large as its group makes it. Bound: the inputs' 2^-30, a rounding
+# of the running sum a group and a split (at least six k64 steps each) and six more.
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("K,N,M,group", [(1024, 128, 128, 256), (960, 128, 129, 320), (1024, 1056, 130, 512),
+                                         (1024, 128, 128, 1024), (3072, 4096, 256, 3072), (3072, 136, 66, 1536),
+                                         (6400, 96, 70, 6400)])
+def test_digit_planes_wide_groups_of_one_sign(dev, K, N, M, group, sign):
+    lin = torch.nn.Linear(K, N, device=dev)
+    lin.weight.data = (torch.rand(N, K, device=dev) * 0.01 + 0.99) * sign
+    lin.weight.data[: N // 2] = sign  # every code at its extreme
+    lin.bias.data.zero_()
+    mod = g.quantize_linear(lin, 4, group_size=group)[0]
+    x = torch.tensor([1.2, 1.0, 1.99], device=dev)[torch.arange(M, device=dev) % 3].unsqueeze(1).repeat(1, K)
+    with torch.no_grad():
+        y = mod(x)
+    q = g.unpack_int4(mod.codes, N * K).view(N, K)
+    w = q.double() * mod.scale.double().repeat_interleave(group, dim=1)[:, :K]
+    ref = x.double() @ w.t()
+    bound = ref.abs() * (2.0**-29 + (-(-K // group) + K // 384 + 6) * 2.0**-24)
+    err = (y.double() - ref).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
 @pytest.mark.parametrize("bits", [8, 4])
 def test_digit_planes_strided(dev, bits):
     K, N, M = 768, 772, 140
