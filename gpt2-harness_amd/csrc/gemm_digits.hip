@@ -38,7 +38,10 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef int i32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kDigits = 4;
-constexpr int kPairSteps = 4;  // k64 steps of a group whose digit sums join in int32: 256 (2^14 257) < 2^31
+// kW4G with groups of more than kPairGroup columns, whose digit sums do not join in
+// int32 (256 columns: 256 (2^14 257) < 2^31); a kernel of its own, as a choice inside
+// the fold costs the narrow groups 15% (1600 x 4800 M = 1024 65 -> 76 us)
+constexpr int kW4GWide = 1000 + kW4G, kPairGroup = 256;
 
 // The digit planes in MFMA operand order: for row tile t (32 rows), unit u (32
 // columns) and digit d (0 lowest) a 1 KB block at ((t U + u) 4 + d) 1024, byte
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
 // column, so a scale is one load a lane and column tile; the next group starts
 // from zero. A digit and a code reach 2^7 each, so a sum reaches 2^14 a column:
 // two of them join in int32 (256 times one plus the other) up to 256 columns, in
-// fp32 for wider groups.
+// fp32 for wider groups (kW4GWide).
 // gridDim.z > 1: split over K, workgroup z writes fp32 slice z of y (no bias).
 // Out (fp32 output, unsplit): a residual added last, or a c_attn whose key and
 // value columns go to the cache (a 32-column tile lies within one head, so its
@@ -259,7 +262,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
     const uint8_t* __restrict__ xt, const float* __restrict__ rs, const uint8_t* __restrict__ w, int64_t ldw,
     const float* __restrict__ scale, const float* __restrict__ bias, TY* __restrict__ y, int64_t ldy, int M, int N,
     int K, const uint16_t* __restrict__ scale16, int ngroups, int gs, DigitsOut out) {
-    constexpr bool GROUPED = FMT == kW4G;
+    constexpr bool GROUPED = FMT == kW4G || FMT == kW4GWide;
     static_assert(D >= 2, "register sets");
     constexpr int WNW = 4 / WMW;
     constexpr int MT = TM * WMW, NTL = TN * WNW;  // row and column tiles of the workgroup
@@ -408,7 +411,7 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
 #pragma unroll
                     for (int q = 0; q < 16; ++q) {
                         float v;
-                        if (gs <= kPairSteps) {
+                        if constexpr (FMT == kW4G) {
                             const float hi = (float)((acc[j][i][3][q] << 8) + acc[j][i][2][q]);
                             const float lo = (float)((acc[j][i][1][q] << 8) + acc[j][i][0][q]);
                             v = fmaf(hi, 65536.f, lo);
@@ -578,8 +581,8 @@ int run_digits(const LinearArgs& a, const uint8_t* xt, const float* rs, TY* y, i
     const int64_t grid = PERSIST ? std::min<int64_t>(tiles, 256 * OCC) : tiles;
     hipLaunchKernelGGL((gemm_digits_kernel<WMW, TM, TN, D, OCC, PERSIST, FMT, TY>), dim3((unsigned)grid, 1, (unsigned)S),
                        dim3(256), 0, a.stream, xt, rs, a.w, a.ldw, a.scale, a.bias, y, ldy, (int)a.M, (int)a.N,
-                       (int)a.K, a.scale16, FMT == kW4G ? (int)((a.K + a.group - 1) / a.group) : 0,
-                       FMT == kW4G ? a.group / 64 : 1, out);
+                       (int)a.K, a.scale16, a.fmt == kW4G ? (int)((a.K + a.group - 1) / a.group) : 0,
+                       a.fmt == kW4G ? a.group / 64 : 1, out);
     return launch_status();
 }
 
@@ -616,7 +619,7 @@ template <int FMT, typename TY>
 int dispatch_digits(const LinearArgs& a, DigitTile tile, const uint8_t* xt, const float* rs, TY* y, int64_t ldy,
                     int64_t S, const DigitsOut& out = {}) {
     // group-wise: the fp32 sums beside the integer ones fit the small tile
-    if constexpr (FMT == kW4G) return run_digits<1, 1, 1, 3, 2, false, FMT, TY>(a, xt, rs, y, ldy, S, out);
+    if constexpr (FMT == kW4G || FMT == kW4GWide) return run_digits<1, 1, 1, 3, 2, false, FMT, TY>(a, xt, rs, y, ldy, S, out);
     else switch (tile) {
         case kTile64x256: return run_digits<2, 1, 4, 2, 1, false, FMT, TY>(a, xt, rs, y, ldy, S, out);
         case kTile64x128: return run_digits<2, 1, 2, 2, 2, true, FMT, TY>(a, xt, rs, y, ldy, S, out);
@@ -713,7 +716,9 @@ int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu, con
     if (f.res && (f.ldr % 4 != 0 || !aligned(f.res, 16))) S = 1;
     S = std::min<int64_t>(S, (int64_t)((ws_bytes - need) / (size_t)(a.M * a.N * 4)));
     S = std::max<int64_t>(S, 1);
-    if (a.fmt == kW4G) return run_digits_linear<kW4G>(a, xt, rs, part, S, gelu, f);
+    if (a.fmt == kW4G)
+        return a.group <= kPairGroup ? run_digits_linear<kW4G>(a, xt, rs, part, S, gelu, f)
+                                     : run_digits_linear<kW4GWide>(a, xt, rs, part, S, gelu, f);
     return a.fmt == kW4 ? run_digits_linear<kW4>(a, xt, rs, part, S, gelu, f)
                         : run_digits_linear<kW8>(a, xt, rs, part, S, gelu, f);
 }
