@@ -1072,3 +1072,43 @@ def test_prefill_attention_arguments(dev):
     assert L.tiq_prefill_attention(*args(64, 66)) == -3
     assert L.tiq_prefill_attention(*args(64, 64, f + 4)) == -3
     assert L.tiq_prefill_attention(*args(64)) == 0
+
+
+def test_gelu_tanh_special_values(dev):
+    """Infinities, NaN, signed zeros, cubes that overflow and the ends of the
+    range, in the pass and in the epilogues of the row kernels: what 0.5 x (1 +
+    tanh(u)) gives in fp32, signs of zeros included."""
+    top = torch.finfo(torch.float32).max
+    inf = float("inf")
+    x = torch.tensor([inf, -inf, float("nan"), 0.0, -0.0, top, -top, 1e20, -1e20, 1e13, -1e13, 20.0, -20.0, 12.7, 1e-38,
+                      -1e-38, 1e-45, -1e-45])
+    want = 0.5 * x * (1.0 + torch.tanh(math.sqrt(2.0 / math.pi) * (x + 0.044715 * x * x * x)))
+    # halving a subnormal rounds it away in the chain; the function's value there is x / 2
+    want[-4:] = torch.tensor([0.5e-38, -0.5e-38, 0.0, -0.0])
+
+    def same(y):
+        y = y.cpu()
+        assert torch.equal(y.isnan(), want.isnan())
+        assert torch.equal(torch.signbit(y)[~y.isnan()], torch.signbit(want)[~want.isnan()])
+        keep = want.isfinite()
+        assert torch.equal(y[~keep & ~want.isnan()], want[~keep & ~want.isnan()])
+        assert torch.allclose(y[keep], want[keep], rtol=1e-6, atol=2e-45)
+
+    L, n = _lib.lib(), x.numel()
+    st = torch.cuda.current_stream().cuda_stream
+    xd, y = x.to(dev), torch.empty(n, device=dev)
+    _lib.check(L.tiq_gelu_tanh(xd.data_ptr(), y.data_ptr(), n, st), "gelu")
+    same(y)
+    K, N = 64, 96  # rows of zeros: 0 + bias is what the activation sees
+    want[4] = 0.0
+    bias = torch.zeros(N)
+    bias[:n] = x
+    codes, scale = torch.ones(N, K, dtype=torch.int8, device=dev), torch.ones(N, device=dev)
+    bias = bias.to(dev)
+    for M in (1, 4, 12, 40):
+        rows, y = torch.zeros(M, K, device=dev), torch.empty(M, N, device=dev)
+        _lib.check(L.tiq_linear_fused(rows.data_ptr(), _lib.F32, M, K, K, codes.data_ptr(), _lib.WF_INT8,
+                                      scale.data_ptr(), None, 0, bias.data_ptr(), N, y.data_ptr(), _lib.F32, N, None,
+                                      None, 1e-5, _lib.ACT_GELU_TANH, None, 0, st), "linear with gelu")
+        for m in range(M):
+            same(y[m, :n])
