@@ -15,6 +15,22 @@
 // three bf16 planes with fp32 sums before and as digits now: K = 768 1.0e-7 /
 // 5.1e-8, K = 1600 5.2e-7 / 5.1e-8, K = 6400 1.0e-6 / 5.1e-8.
 //
+// (Exact products of sliced operands: Ozaki, Ogita, Oishi, Rump, Numerical Algorithms
+// 59, 2012; on integer matrix units: Ootomo, Ozaki, Yokota, IJHPCA 38, 2024.)
+//
+// Rows of wide range. Where a few elements stand far above the rest, the rest's
+// rounding (2^-30 of the largest) is what an output with zero codes in those few
+// columns has: N(0, 1) with one element T, such outputs, K = 768: T = 1e3 3.0e-7 of
+// their norm, 1e5 3.5e-5, where an fp32 chain has 5e-7 at any T. So a row whose
+// largest element is more than kFar^2 sqrt(K) times the square of the mean square
+// root of its other elements (of each pair of neighbours the larger; no zeros) keeps
+// its fp32 bits, a byte a plane in the
+// digits' place and size, and rs < 0 marks it: the product computes its outputs once
+// more, by fp32 sums (wide_rows). The line lies where the digits' error on such
+// outputs reaches the chain's, which grows with sqrt(K) (one large element among
+// N(0, 1): T = 1400 at K = 768); the mean square root weighs a row's many elements and
+// not its few: a hidden row after GELU, mostly small, stays on this side.
+//
 // Why four int8 planes: int8 MFMAs run at twice the bf16 rate, so four planes
 // cost two bf16 passes over the product instead of three, and the codes enter
 // the matrix cores as they are stored, with no widening beside the MFMAs.
@@ -26,6 +42,7 @@
 // 84 us of the 143 at 1600 x 4800), then the step's LDS traffic, which does not
 // hide wholly beside one wavefront's MFMAs a SIMD.
 #include <algorithm>
+#include <cmath>
 
 #include "tiq_internal.hpp"
 
@@ -50,10 +67,46 @@ constexpr int kW4GWide = 1000 + kW4G, kPairGroup = 256;
 // which nibble weights unpack), so the product's loads and LDS accesses are
 // all contiguous. One workgroup per R rows: 8 rows' chunks of a block are 128
 // consecutive bytes, a whole cache line a store (4 rows where that would leave
-// CUs idle). rs[m] = 2^(e_m - 29), NaN for
-// a row holding an infinity or NaN (every output of it is then NaN).
+// CUs idle). rs[m] = 2^(e_m - 29), -1 for a row held as its fp32 bits: one of wide
+// range or below 2^-97 or, with fewer than kInfRows rows, one that holds an infinity or
+// NaN. From kInfRows rows such a row has rs NaN (every output of it is then NaN).
 // IT: 1024-column passes held in registers; 0: the row is read twice.
 constexpr int kSplitThreads = 512;
+
+// Rows from which a row that holds an infinity or NaN gives NaN in every output, as a
+// split into planes does; fewer rows replace the GEMV, which gives inf there.
+constexpr int kInfRows = 128;
+// Rows of a row tile held as fp32 bits up to which dot products beat the MFMAs.
+constexpr int kFewWide = 4;
+
+constexpr float kFar = 7.0f;
+
+// 2^-64 times the square root of a float, from its bits, to a constant and 6% (half
+// the exponent); 0 for zero.
+__device__ __forceinline__ float rough_root(uint32_t b) { return __uint_as_float(b >> 1); }
+
+// op over the lanes of equal number modulo R (4 or 8), in every lane, by lane moves on
+// the VALU (shuffles pass through the LDS crossbar).
+template <int R, typename Op>
+__device__ __forceinline__ uint32_t across(uint32_t v, Op op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    v = op(a[0], a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    v = op(b[0], b[1]);
+    v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xf, 0xf, false));  // row_ror:8
+    if constexpr (R == 4) v = op(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xf, 0xf, false));
+    return v;
+}
+template <int R>
+__device__ __forceinline__ float sum_across(float v) {
+    return __uint_as_float(across<R>(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+        return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+    }));
+}
+template <int R>
+__device__ __forceinline__ uint32_t max_across(uint32_t v) {
+    return across<R>(v, [](uint32_t a, uint32_t b) { return max(a, b); });
+}
 
 __device__ __forceinline__ uint32_t digits_of(float v, float mul) {
     const int t = (int)__builtin_rintf(v * mul) + 0x00808080;
@@ -61,7 +114,7 @@ __device__ __forceinline__ uint32_t digits_of(float v, float mul) {
 }
 
 template <bool NIB>
-__device__ __forceinline__ void store_digits(const float (&v)[16], float mul, uint8_t* __restrict__ dst) {
+__device__ __forceinline__ void store_digits(const float (&v)[16], float mul, bool bits, uint8_t* __restrict__ dst) {
     u32x4 pl[kDigits];
 #pragma unroll
     for (int g = 0; g < 4; ++g) {  // four columns -> one dword of each plane
@@ -69,7 +122,8 @@ __device__ __forceinline__ void store_digits(const float (&v)[16], float mul, ui
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int p = 4 * g + i;
-            t[i] = digits_of(v[NIB ? (p < 8 ? 2 * p : 2 * (p - 8) + 1) : p], mul);
+            const float e = v[NIB ? (p < 8 ? 2 * p : 2 * (p - 8) + 1) : p];
+            t[i] = bits ? __float_as_uint(e) : digits_of(e, mul);
         }
         const uint32_t a = __builtin_amdgcn_perm(t[1], t[0], 0x05010400u);  // d0 d0 d1 d1 of t0, t1
         const uint32_t b = __builtin_amdgcn_perm(t[3], t[2], 0x05010400u);
@@ -90,13 +144,13 @@ __device__ __forceinline__ void store_digits(const float (&v)[16], float mul, ui
 template <int IT, int R, bool NIB, bool LN>
 __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float* __restrict__ x, int64_t ldx, int M,
                                                                      int K, uint8_t* __restrict__ xt,
-                                                                     float* __restrict__ rs, bool gelu,
+                                                                     float* __restrict__ rs, bool gelu, float line,
                                                                      const float* __restrict__ ln_w,
                                                                      const float* __restrict__ ln_b, float ln_eps) {
     static_assert(!LN || IT > 0, "LayerNorm needs the row in registers");
     static_assert(R == 8 || R == 4, "whole quads of rows");
     constexpr int WV = kSplitThreads / 64, CT = kSplitThreads / R;  // 16-column chunks a pass
-    __shared__ uint32_t am[WV][R];
+    __shared__ float4 stat[WV][R];
     __shared__ float ls[2][WV][R];
     const int tid = threadIdx.x, row = tid % R, c0 = tid / R;
     const int m = blockIdx.x * R + row;
@@ -135,6 +189,23 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
         }
     };
     uint32_t mx = 0;
+    // over pairs of neighbours: the sum of their larger elements' square roots, how
+    // many are not zero (each element by itself is twice the instructions: the GELU'd
+    // split of 4096 x 6400 47 -> 53 us, by pairs 52)
+    float root = 0.f, count = 0.f;
+    auto measure = [&](const float (&e)[16], bool mine) {
+        float s = 0.f;
+        uint32_t n = 0;
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+            const uint32_t b = max(abs_bits(e[i]), abs_bits(e[i + 1]));
+            mx = max(mx, b);
+            n += min(b, 1u);
+            s += rough_root(b);
+        }
+        root += mine ? s : 0.f;
+        count += mine ? (float)n : 0.f;
+    };
     float v[IT ? IT : 1][16];
     if constexpr (IT > 0) {
 #pragma unroll
@@ -142,8 +213,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
         if constexpr (LN) {
             // a row is the threads of equal tid % R: 64 / R lanes of each wavefront
             auto row_sum = [&](float s, int slot) {
-#pragma unroll
-                for (int off = 32; off >= R; off >>= 1) s += __shfl_xor(s, off, 64);
+                s = sum_across<R>(s);
                 if ((tid & 63) < R) ls[slot][tid >> 6][row] = s;
                 __syncthreads();
                 float t = 0.f;
@@ -184,39 +254,48 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
             }
         }
 #pragma unroll
-        for (int it = 0; it < IT; ++it)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) mx = max(mx, abs_bits(v[it][i]));
+        for (int it = 0; it < IT; ++it) measure(v[it], c0 + CT * it < NC);
     } else {
         for (int c = c0; c < NC; c += CT) {
             load(c, v[0]);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) mx = max(mx, abs_bits(v[0][i]));
+            measure(v[0], true);
         }
     }
-#pragma unroll
-    for (int off = 32; off >= R; off >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, off, 64));
-    if ((tid & 63) < R) am[tid >> 6][row] = mx;
+    mx = max_across<R>(mx);
+    root = sum_across<R>(root);
+    count = sum_across<R>(count);
+    if ((tid & 63) < R) stat[tid >> 6][row] = make_float4(__uint_as_float(mx), root, count, 0.f);
     __syncthreads();
+    root = count = 0.f;
 #pragma unroll
-    for (int w = 0; w < WV; ++w) mx = max(mx, am[w][row]);
-    // rows below 2^-97 share its exponent: both powers of two stay normal
-    const int e = max((int)(mx >> 23) - 127, -97);
+    for (int w = 0; w < WV; ++w) {
+        const float4 t = stat[w][row];
+        mx = max(mx, __float_as_uint(t.x));
+        root += t.y;
+        count += t.z;
+    }
     const bool finite = mx < 0x7f800000u;
+    // the other elements' mean square root against the largest's; rows below 2^-97
+    // would need powers of two that are not normal
+    const float top = rough_root(mx);
+    const int far = (count > 1.f) & (top * (count - 1.f) > line * (root - top));
+    const int tiny = (mx != 0) & (mx < (127u - 97) << 23);
+    const bool wide = (finite & (far | tiny)) | (!finite & (M < kInfRows));
+    const int e = max((int)(mx >> 23) - 127, -97);
     const float mul = finite ? __uint_as_float((uint32_t)(29 - e + 127) << 23) : 0.f;
     if (c0 == 0 && m < M)
-        rs[m] = finite ? __uint_as_float((uint32_t)(e - 29 + 127) << 23) : __uint_as_float(0x7fc00000u);
+        rs[m] = wide ? -1.f : finite ? __uint_as_float((uint32_t)(e - 29 + 127) << 23) : __uint_as_float(0x7fc00000u);
     uint8_t* base = xt + (int64_t)(m >> 5) * U * 4096 + (m & 31) * 16;
     if constexpr (IT > 0) {
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int c = c0 + CT * it;
-            if (c < NC && m < M) store_digits<NIB>(v[it], mul, base + (int64_t)(c >> 1) * 4096 + (c & 1) * 512);
+            if (c < NC && m < M) store_digits<NIB>(v[it], mul, wide, base + (int64_t)(c >> 1) * 4096 + (c & 1) * 512);
         }
     } else {
         for (int c = c0; c < NC; c += CT) {
             load(c, v[0]);  // every lane of a quad: rows past M too
-            if (m < M) store_digits<NIB>(v[0], mul, base + (int64_t)(c >> 1) * 4096 + (c & 1) * 512);
+            if (m < M) store_digits<NIB>(v[0], mul, wide, base + (int64_t)(c >> 1) * 4096 + (c & 1) * 512);
         }
     }
 }
@@ -424,7 +503,180 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
         }
     };
 
+    constexpr float unit = FMT == kW8 ? 1.f : 0.0625f;
+    // The outputs of a tile's rows that are held as fp32 bits, over what the digit
+    // sums gave (the same lanes' stores): few rows of a row tile by dot products, a
+    // wavefront along K for one column after the other; more of them by the fp32
+    // MFMAs over the whole row tile (the other rows' results are not stored). Rare rows,
+    // which cost: int8, M = 4096, none / one / every 128th / every row of them, 1600 x
+    // 6400 236 / 287 / 384 / 979 us, 6400 x 1600 213 / 362 / 522 / 1259 (three bf16 planes
+    // with fp32 sums, which this product replaced: 310 for any row).
+    auto wide_rows = [&](int tile) {
+        int rm, rn;
+        staged_tile_of(tile, rm, rn, tiles_m, tiles_n);
+        const int n0 = rn * 32 * NTL + wn * 32 * TN, m0 = (rm * MT + wm * TM) * 32;
+        const int u0 = 2 * s0, u1 = 2 * (s0 + nk);
+        // a unit's codes, in the order of the digits' bytes
+        auto codes = [&](const uint8_t* src) -> u32x4 {
+            if constexpr (FMT == kW8) {
+                return *reinterpret_cast<const u32x4*>(src);
+            } else {
+                const uint2 t = *reinterpret_cast<const uint2*>(src);
+                uint32_t e0, o0, e1, o1;
+                nibbles_x16(t.x, e0, o0);
+                nibbles_x16(t.y, e1, o1);
+                return u32x4{e0, e1, o0, o1};
+            }
+        };
+        auto code = [](const u32x4& c, int p) { return (float)(int8_t)(c[p >> 2] >> 8 * (p & 3)); };
+        // a unit's 16 values: byte p of the four planes
+        auto values = [&](const uint8_t* src, float (&v)[16]) {
+            u32x4 d[kDigits];
+#pragma unroll
+            for (int q = 0; q < kDigits; ++q) d[q] = *reinterpret_cast<const u32x4*>(src + 1024 * q);
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const uint32_t pick = e ? 0x07030602u : 0x05010400u;
+                    const uint32_t lo = __builtin_amdgcn_perm(d[1][g], d[0][g], pick);
+                    const uint32_t hi = __builtin_amdgcn_perm(d[3][g], d[2][g], pick);
+                    v[4 * g + 2 * e] = __uint_as_float(__builtin_amdgcn_perm(hi, lo, 0x05040100u));
+                    v[4 * g + 2 * e + 1] = __uint_as_float(__builtin_amdgcn_perm(hi, lo, 0x07060302u));
+                }
+        };
+        // column tile j's outputs: where row 0 of each lane's column lies, what follows
+        struct Column {
+            TY* base;
+            float scale, bias;
+            bool in, cached;
+        };
+        auto column = [&](int j) {
+            const int n = n0 + 32 * j + r, nc = min(n, N - 1);
+            Column c = {y + (int64_t)blockIdx.z * M * ldy + n, GROUPED ? unit : scale[nc] * unit,
+                        bias && !split ? bias[nc] : 0.f, n < N, false};
+            if constexpr (sizeof(TY) == 4) {
+                if (out.k && n0 + 32 * j >= N / 3) {  // whole tiles lie within one head
+                    const int col = (n0 + 32 * j) % (N / 3);
+                    c.base = (n0 + 32 * j < 2 * (N / 3) ? out.k : out.v) + (col >> 6) * out.sh + (col & 63) + r;
+                    c.cached = true;
+                }
+            }
+            return c;
+        };
+        auto put = [&](const Column& c, int m, float v) {
+            if (!c.in) return;
+            v = fmaf(v, c.scale, c.bias);
+            if constexpr (sizeof(TY) == 4) {
+                if (c.cached) {
+                    const uint32_t b = out.magic ? __umulhi((uint32_t)m, out.magic) : (uint32_t)m;
+                    c.base[(int64_t)b * out.sb + (int64_t)((uint32_t)m - b * out.T) * out.st] = v;
+                } else {
+                    c.base[(int64_t)m * ldy] =
+                        out.res ? v + out.res[(int64_t)m * out.ldr + (c.base - y)] : v;  // unsplit with a residual
+                }
+            } else {
+                c.base[(int64_t)m * ldy] = f32_to_bf16_bits(v);
+            }
+        };
+#pragma unroll 1
+        for (int i = 0; i < TM; ++i) {
+            const int mt = m0 + 32 * i;
+            uint32_t rows = (uint32_t)__ballot(mt + r < M && rs[min(mt + r, M - 1)] < 0.f);  // both halves alike
+            const uint8_t* xr = xt + (int64_t)min(mt >> 5, T - 1) * U * 4096;
+            if (__popc(rows) > kFewWide) {
+                floatx16 a[TN][2], whole[GROUPED ? TN : 1];
+                const floatx16 z = {};
+                const uint8_t* wr[TN];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) a[j][0] = a[j][1] = z, wr[j] = w + (int64_t)min(n0 + 32 * j + r, N - 1) * ldw + h * WB;
+                if constexpr (GROUPED) {
+                    static_assert(TN == 1, "group-wise: one column tile");
+                    whole[0] = z;
+                }
+                for (int u = u0; u < u1; u += 2) {  // whole k64 steps
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        float xv[16];
+                        u32x4 c[TN];
+                        values(xr + (int64_t)(u + e) * 4096 + lane * 16, xv);
+#pragma unroll
+                        for (int j = 0; j < TN; ++j) c[j] = codes(wr[j] + 2 * WB * (u + e));
+#pragma unroll
+                        for (int p = 0; p < 16; ++p)
+#pragma unroll
+                            for (int j = 0; j < TN; ++j)
+                                a[j][e] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[p], code(c[j], p), a[j][e], 0, 0, 0);
+                    }
+                    if constexpr (GROUPED) {
+                        if ((u + 2) % (2 * gs) == 0 || u + 2 == u1) {
+                            const float sg =
+                                f16_bits_to_f32(scale16[(int64_t)min(n0 + r, N - 1) * ngroups + u / (2 * gs)]);
+#pragma unroll
+                            for (int q = 0; q < 16; ++q)
+                                whole[0][q] = fmaf(a[0][0][q] + a[0][1][q], sg, whole[0][q]);
+                            a[0][0] = a[0][1] = z;
+                        }
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const Column c = column(j);
+#pragma unroll
+                    for (int q = 0; q < 16; ++q) {
+                        const int o = 8 * (q >> 2) + 4 * h + (q & 3);
+                        const float v = GROUPED ? whole[0][q] : a[j][0][q] + a[j][1][q];
+                        if (rows >> o & 1) put(c, mt + o, v);
+                    }
+                }
+                continue;
+            }
+            while (rows) {
+                const int o = __builtin_ctz(rows);
+                rows &= rows - 1;
+#pragma unroll 1
+                for (int j = 0; j < TN; ++j) {
+                    float keep = 0.f;
+                    for (int ub = u0; ub < u1; ub += 32) {  // 1024 columns of x, 16 a lane
+                        const int u = min(ub + (lane >> 1), u1 - 1);
+                        float xv[16];
+                        values(xr + (int64_t)u * 4096 + (lane & 1) * 512 + o * 16, xv);
+                        const bool in = ub + (lane >> 1) < u1;
+#pragma unroll
+                        for (int p = 0; p < 16; ++p) xv[p] = in ? xv[p] : 0.f;
+                        constexpr int kAhead = 8;  // columns in flight
+#pragma unroll 1
+                        for (int c = 0; c < 32; c += kAhead) {
+                            u32x4 cv[kAhead];
+                            float sg[GROUPED ? kAhead : 1];
+#pragma unroll
+                            for (int e = 0; e < kAhead; ++e) {
+                                const int64_t n = min(n0 + 32 * j + c + e, N - 1);
+                                cv[e] = codes(w + n * ldw + 2 * WB * u + (lane & 1) * WB);
+                                if constexpr (GROUPED) sg[e] = f16_bits_to_f32(scale16[n * ngroups + u / (2 * gs)]);
+                            }
+                            asm volatile("" ::: "memory");
+                            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                            for (int e = 0; e < kAhead; ++e) {
+                                float s[4] = {};
+#pragma unroll
+                                for (int p = 0; p < 16; ++p) s[p & 3] = fmaf(xv[p], code(cv[e], p), s[p & 3]);
+                                float v = (s[0] + s[1]) + (s[2] + s[3]);
+                                if constexpr (GROUPED) v *= sg[e];
+                                v = wave_sum_dpp(v);
+                                keep = r == c + e ? keep + v : keep;
+                            }
+                        }
+                    }
+                    if (h == (o >> 2 & 1)) put(column(j), mt + o, keep);  // the half whose lanes stored this row
+                }
+            }
+        }
+    };
+
     const int total = tiles_m * tiles_n;
+    bool wide = false;  // some row of this wavefront's tiles is held as fp32 bits
     begin_tile(blockIdx.x);
     // the workgroup's tiles: one, or every gridDim.x-th of a persistent grid,
     // where the next tile's first loads go out before the epilogue
@@ -476,7 +728,6 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
 
         // y = (((a3 256 + a2) 256 + a1) 256 + a0) 2^(e_m - 29) scale + bias; a
         // store instruction writes 32 consecutive outputs of two rows
-        constexpr float unit = FMT == kW8 ? 1.f : 0.0625f;
         const int n0 = tn * 32 * NTL + wn * 32 * TN, m0 = (tm * MT + wm * TM) * 32;
         const bool full = m0 + 32 * TM <= M && n0 + 32 * TN <= N;
         float sc[TN], bi[TN];
@@ -568,8 +819,19 @@ __global__ __launch_bounds__(256, OCC) void gemm_digits_kernel(
                 }
             }
         }
+        uint32_t signs = 0;  // (rows past M too: then wide_rows finds none)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                signs |= __float_as_uint(rm[i][g].x) | __float_as_uint(rm[i][g].y) | __float_as_uint(rm[i][g].z) |
+                         __float_as_uint(rm[i][g].w);
+        wide |= __any((int)signs < 0);
         if (!more) break;
         __syncthreads();  // every wavefront's last LDS reads are done
+    }
+    if (wide) {
+        for (int t = blockIdx.x; t < total; t += PERSIST ? (int)gridDim.x : total) wide_rows(t);
     }
 }
 
@@ -636,10 +898,11 @@ constexpr int64_t kSplitWideRows = 1280;
 
 template <bool NIB>
 int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu, const PrefillFusion& f) {
+    const float line = kFar * sqrtf(sqrtf((float)a.K));
     auto launch = [&](auto kernel, int rows) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)((a.M + rows - 1) / rows)), dim3(kSplitThreads), 0, a.stream,
-                           static_cast<const float*>(a.x), a.ldx, (int)a.M, (int)a.K, xt, rs, gelu, f.ln_w, f.ln_b,
-                           f.ln_eps);
+                           static_cast<const float*>(a.x), a.ldx, (int)a.M, (int)a.K, xt, rs, gelu, line, f.ln_w,
+                           f.ln_b, f.ln_eps);
         return launch_status();
     };
     if (a.K > 1024 && a.K <= 8192 && a.M < kSplitWideRows) {

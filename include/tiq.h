@@ -163,11 +163,16 @@ size_t tiq_linear_w8_workspace(int x_dtype, int64_t M, int64_t K);
  * (model.py:254,319,352,355), used by the prefill (M = B*T rows) of a model
  * that keeps fp32 activations. With fp32 x and M >= 128 each activation row
  * becomes a fixed-point row of four int8 digit planes under its own power of
- * two (31 bits below the row's largest element; written to the workspace) and
- * the product runs on the int8 matrix cores with exact integer sums: more
- * accurate than an fp32 GEMM. A row holding an infinity or NaN gives NaN
- * outputs. 65 <= M <= 127, and M >= 32 with a long K, run so too given a
- * workspace of tiq_gemm_w8_workspace(TIQ_F32, M, K, N) bytes. Other cases behave as
+ * two (every element to within 2^-30 of the row's largest; written to the
+ * workspace) and the product runs on the int8 matrix cores with exact integer
+ * sums: error at most 2^-30 max|x| sum|w| and a few roundings of the result,
+ * where an fp32 GEMM rounds every partial sum. That is the smaller error unless
+ * a few elements stand far above the rest (one element of 1400 among N(0, 1) at
+ * K = 768, sqrt(K) times that for other K) in columns whose codes are zero: such
+ * a row is kept as fp32 and its outputs are fp32 sums. A row holding an infinity
+ * or NaN gives NaN outputs from M = 128; below, what an fp32 sum gives. 65 <= M
+ * <= 127, and M >= 32 with a long K, run so too given a workspace of
+ * tiq_gemm_w8_workspace(TIQ_F32, M, K, N) bytes. Other cases behave as
  * tiq_linear_w8. TIQ_EWORKSPACE when M >= 128 and the workspace is smaller
  * than tiq_linear_w8_workspace() or not 16-byte aligned. */
 int tiq_linear_w8_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx,

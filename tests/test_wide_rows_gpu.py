@@ -1,0 +1,161 @@
+"""fp32 rows of wide range through the digit-plane products: rows in which one or a
+few elements stand so far above the rest that a fixed point under the largest
+would round the rest away, and (below 128 rows) rows that hold an infinity.
+
+Every weight has a column of zeros in half of its outputs, in the place of the
+rows' large element: those outputs are sums of the other elements alone. Bound:
+one rounding of a partial sum a product, each 2^-24 of it, their 2-norm over an
+output row sqrt(K) 2^-24 of the outputs' (six more for the scale, the chains' sum
+and the slices); for the other outputs the worst order, (K + 8) 2^-24 sum |x| |w|.
+"""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+import gpt2_harness_amd as g
+from gpt2_harness_amd import _lib
+from gpt2_harness_amd.model import gelu_tanh
+
+pytestmark = pytest.mark.gpu
+
+GROUPS = {"int8": None, "int4": None, "g128": 128, "g1024": 1024}
+COL = 37  # of the large element
+
+
+def _quantized(K, N, fmt, dev, bias=False):
+    """(module, its weight in 64 bits); column COL is zero in the odd outputs."""
+    gen = torch.Generator(device=dev).manual_seed(K + N)
+    lin = torch.nn.Linear(K, N, device=dev)
+    lin.weight.data = torch.randn(N, K, generator=gen, device=dev) * 0.02
+    lin.weight.data[1::2, COL] = 0.0
+    lin.bias.data = torch.randn(N, generator=gen, device=dev) * (0.1 if bias else 0.0)
+    mod = g.quantize_linear(lin, 8 if fmt == "int8" else 4, group_size=GROUPS[fmt])[0]
+    if fmt == "int8":
+        w = mod.codes.double() * mod.scale.double().unsqueeze(1)
+    else:
+        q = g.unpack_int4(mod.codes, N * K).view(N, K).double()
+        s = mod.scale.double()
+        w = q * (s.unsqueeze(1) if GROUPS[fmt] is None else s.repeat_interleave(GROUPS[fmt], dim=1)[:, :K])
+    assert bool((w[1::2, COL] == 0).all())
+    return mod, w
+
+
+def _rows(M, K, dev):
+    """(rows, the same without the large elements, the indexes of the wide rows)"""
+    gen = torch.Generator(device=dev).manual_seed(M + K)
+    base = torch.randn(M, K, generator=gen, device=dev)
+    x = base.clone()
+    # a few rows of the first row tile, many of the second, the last two
+    wide = sorted({0, 5, 31, *range(32, 42), 63, M - 2, M - 1})
+    for i, m in enumerate(wide):
+        x[m, COL] = (1.4e3, -4e3, 1e5, -1e7, 1e12, 1e30)[i % 6]
+    return x, base, wide
+
+
+def _check(y, x, w, wide):
+    K = x.shape[1]
+    ref = x.double() @ w.t()
+    err = y.double() - ref
+    bound = (K + 8) * 2.0**-24 * (x.double().abs() @ w.abs().t())
+    assert bool((err.abs() <= bound + 1e-30).all())
+    e, r = err[wide][:, 1::2].norm(dim=1), ref[wide][:, 1::2].norm(dim=1)
+    assert bool((e <= (math.sqrt(K) + 6) * 2.0**-24 * r).all()), (e / r).tolist()
+
+
+# Small, split, persistent and wide product tiles; ragged rows and columns; groups
+# that a split cuts
+@pytest.mark.parametrize("fmt", sorted(GROUPS))
+@pytest.mark.parametrize("K,N,M", [(64, 128, 65), (768, 3072, 77), (3072, 768, 65), (1600, 1212, 130), (1024, 37, 129),
+                                   (768, 2304, 1500), (3200, 1020, 4033), (7232, 128, 130)])
+@torch.no_grad()
+def test_wide_rows(dev, fmt, K, N, M):
+    mod, w = _quantized(K, N, fmt, dev)
+    x, base, wide = _rows(M, K, dev)
+    y = mod(x)
+    _check(y, x, w, wide)
+    plain = mod(base)  # the other rows do not notice
+    keep = [m for m in range(M) if m not in wide]
+    assert torch.equal(y[keep], plain[keep])
+    L = _lib.lib()
+    n_ws = int(L.tiq_gemm_w8_workspace(_lib.F32, M, K, N))
+    ws = torch.empty(max(n_ws, 16), dtype=torch.uint8, device=dev)
+    yb = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
+    tail = (_lib.ptr(mod.bias), N, yb.data_ptr(), _lib.BF16, N, ws.data_ptr(), n_ws,
+            torch.cuda.current_stream().cuda_stream)
+    head = (x.data_ptr(), _lib.F32, M, K, K, mod.codes.data_ptr(), mod.scale.data_ptr())
+    if GROUPS[fmt]:
+        rc = L.tiq_linear_w4g_ws(*head, GROUPS[fmt], *tail)
+    else:
+        rc = (L.tiq_linear_w8_ws if fmt == "int8" else L.tiq_linear_w4_ws)(*head, *tail)
+    _lib.check(rc, "linear")
+    assert torch.equal(yb, y.bfloat16())
+
+
+@pytest.mark.parametrize("fmt", sorted(GROUPS))
+@torch.no_grad()
+def test_wide_rows_in_a_block(dev, fmt):
+    """LayerNorm and GELU in, residual and cache writes out."""
+    C, B, T = 768, 3, 43
+    M = B * T
+    mod, w = _quantized(C, 3 * C, fmt, dev, bias=True)
+    x, _, wide = _rows(M, C, dev)
+    x[wide, COL] = x[wide, COL].clamp(-1e7, 1e7)
+    ln = torch.nn.LayerNorm(C, device=dev)
+    ref = torch.nn.functional.layer_norm(x.double(), (C,)) @ w.t() + mod.bias.double()
+    y = mod.forward_prefill(x, ln=ln)
+    e = (y.double() - ref)[wide][:, 1::2].norm(dim=1) / ref[wide][:, 1::2].norm(dim=1)
+    f = (mod(ln(x)).double() - ref)[wide][:, 1::2].norm(dim=1) / ref[wide][:, 1::2].norm(dim=1)
+    assert bool((e <= 1.25 * f + (math.sqrt(C) + 8) * 2.0**-24).all()), (e.tolist(), f.tolist())
+    plain = mod(x)
+    k, v = torch.zeros(2, B, C // 64, T + 3, 64, device=dev).unbind(0)
+    q = mod.forward_prefill(x, kv=(k[:, :, 1 : T + 1], v[:, :, 1 : T + 1], T))
+    parts = plain.view(B, T, 3, C // 64, 64).permute(2, 0, 3, 1, 4)
+    assert torch.equal(q.view(B, T, C // 64, 64).transpose(1, 2), parts[0])
+    assert torch.equal(k[:, :, 1 : T + 1], parts[1]) and torch.equal(v[:, :, 1 : T + 1], parts[2])
+    for z in (k, v):
+        assert not bool(z[:, :, 0].any()) and not bool(z[:, :, T + 1 :].any())
+    res = torch.randn(M, 3 * C, device=dev)
+    assert torch.equal(mod.forward_prefill(x, residual=res), res + plain)
+    x[wide, COL] = x[wide, COL].abs()
+    assert torch.equal(mod.forward_prefill(x, gelu=True, residual=res), res + mod(gelu_tanh(x)))
+
+
+# few large elements among zeros stay digits; subnormal rows and single elements
+@torch.no_grad()
+def test_sparse_and_tiny_rows(dev):
+    K, N = 768, 256
+    mod, w = _quantized(K, N, "int8", dev)
+    assert torch.allclose(mod(torch.eye(K, device=dev)).double(), w.t().contiguous(), rtol=2.0**-22, atol=0.0)
+    x = torch.randn(128, K, device=dev)
+    for m, p in ((3, -98), (40, -110), (127, -126)):
+        x[m] *= 2.0**p
+    y, ref = mod(x), x.double() @ w.t()
+    e = (y.double() - ref).norm(dim=1) / ref.norm(dim=1)
+    assert bool((e <= (math.sqrt(K) + 6) * 2.0**-24).all()), e.max().item()
+
+
+@pytest.mark.parametrize("fmt,K,N,M", [("int8", 768, 3072, 77), ("int8", 3072, 768, 65), ("g128", 768, 3072, 127),
+                                       ("g128", 3072, 768, 64)])
+@torch.no_grad()
+def test_infinities_below_128_rows(dev, fmt, K, N, M):
+    """As the row kernels give them: an infinity where the code is not zero."""
+    mod, w = _quantized(K, N, fmt, dev, bias=True)
+    x = torch.randn(M, K, device=dev)
+    plain = mod(x)
+    inf, nan = float("inf"), float("nan")
+    bad = {3: inf, 31: -inf, 40: nan, **{m: -inf for m in range(44, 50)}, M - 1: inf}
+    for m, v in bad.items():
+        x[m, COL] = v
+    y = mod(x)
+    for m, v in bad.items():
+        want = v * w[:, COL]
+        assert torch.equal(y[m].isnan(), want.isnan())
+        ok = ~want.isnan()
+        assert torch.equal(y[m][ok].double(), want[ok])
+    keep = [m for m in range(M) if m not in bad]
+    assert torch.equal(y[keep], plain[keep])
+    few = mod(x[30:34].contiguous())  # the row kernel
+    assert torch.equal(few[1].isnan(), y[31].isnan()) and torch.equal(few[1].isinf(), y[31].isinf())
