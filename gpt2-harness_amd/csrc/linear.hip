@@ -517,6 +517,13 @@ extern "C" size_t tiq_decode_linear_workspace(int w_format, int64_t M, int64_t K
     return decode_linear_workspace(M, K, N);
 }
 
+extern "C" int tiq_decode_linear_takes(int w_format, int64_t M, int64_t K, int64_t N, int planes_out, int finish) {
+    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT8_TILED && w_format != TIQ_WF_INT4_TILED &&
+        w_format != TIQ_WF_F32 && w_format != TIQ_WF_F32_TILED)
+        return 0;
+    return decode_linear_takes((WFormat)w_format, M, K, N, planes_out != 0, finish != 0);
+}
+
 extern "C" int tiq_tile_int8(const int8_t* w, int64_t N, int64_t K, int64_t ldw, int8_t* tiles, void* stream) {
     return launch_tile_int8(reinterpret_cast<const uint8_t*>(w), N, K, ldw, reinterpret_cast<uint8_t*>(tiles),
                             as_stream(stream));

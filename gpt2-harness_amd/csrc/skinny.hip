@@ -1186,6 +1186,45 @@ static int run_decode_f32_tiles(const LinearArgs& a, const uint16_t* x_planes, c
     return launch(stream_f32_kernel);
 }
 
+// How a decode linear runs: its split, whether the product kernel writes the planes
+// itself, whether the reduction kernel follows. finish: a LayerNorm or residual after
+// the product. False: a wavefront's share of K does not fit its weight registers.
+struct DecodeShape {
+    SplitPlan plan;
+    bool product_planes, reduce;
+};
+
+static bool decode_shape(bool w8, int64_t M, int64_t K, int64_t N, bool planes_out, bool finish, DecodeShape& s) {
+    // a row the reduction cannot take (N % 8, N > 8192) without planes out:
+    // one split, the product kernel's own epilogue
+    const bool red_ok = N % 8 == 0 && N <= kRedMaxCols;
+    // LayerNorm'd planes or a residual after the product: the reduction kernel
+    // runs whatever the split, so int8 products split to fill the GPU
+    const bool must_reduce = planes_out && (finish || N % 32 != 0);
+    s.plan = {(red_ok || planes_out) ? decode_splits(M, K, N) : 1, 0};
+    if (w8 && must_reduce && red_ok) {
+        const SplitPlan p = reduce_plan(M, K, N);
+        const int64_t per_wave = ((K / 32 + p.S - 1) / p.S + kWaves - 1) / kWaves;
+        if (per_wave <= split_max_units(p.RT) && ((N + 31) / 32) % p.RT == 0) s.plan = p;
+    }
+    // planes without a LayerNorm or residual from one split: the product
+    // kernel writes them itself (its 32 columns are one unit of the next
+    // linear's K), no reduction launch
+    s.product_planes = planes_out && !finish && s.plan.S == 1 && N % 32 == 0;
+    s.reduce = !s.product_planes && (s.plan.S > 1 || planes_out);
+    const int64_t units = ((K / 32 + s.plan.S - 1) / s.plan.S + kWaves - 1) / kWaves;
+    return s.plan.RT > 0 || units <= (w8 ? max_units<kW8>() : max_units<kF32>());
+}
+
+bool decode_linear_takes(WFormat fmt, int64_t M, int64_t K, int64_t N, bool planes_out, bool finish) {
+    if (M < kSkinnyMinRows || M > 64 || K <= 0 || K % 32 != 0 || N <= 0 || N > 0x7fffffff - 31) return false;
+    if (fmt == kF32T) return !planes_out && !finish && K / 32 >= kWaves;
+    if ((fmt == kW8T || fmt == kW4T) && N % 32 != 0) return false;
+    DecodeShape s;
+    if (!decode_shape(fmt != kF32, M, K, N, planes_out, finish, s)) return false;
+    return !s.reduce || (N % 8 == 0 && N <= kRedMaxCols && (!planes_out || N % 32 == 0));
+}
+
 int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float* next_ln_w,
                       const float* next_ln_b, float next_eps, uint16_t* planes_out) {
     if (a.fmt == kF32T) return run_decode_f32_tiles(a, x_planes, next_ln_w, planes_out);
@@ -1196,27 +1235,10 @@ int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float
     const bool w8 = a.fmt != kF32;
     if ((next_ln_w == nullptr) != (next_ln_b == nullptr) || (next_ln_w && !planes_out)) return TIQ_EINVAL;
     if (!a.y && !planes_out) return TIQ_EINVAL;
-    // a row the reduction cannot take (N % 8, N > 8192) without planes out:
-    // one split, the product kernel's own epilogue
-    const bool red_ok = a.N % 8 == 0 && a.N <= kRedMaxCols;
-    // LayerNorm'd planes or a residual after the product: the reduction kernel
-    // runs whatever the split, so int8 products split to fill the GPU
-    const bool must_reduce = planes_out && (next_ln_w || a.fuse.res || a.N % 32 != 0);
-    SplitPlan plan{(red_ok || planes_out) ? decode_splits(a.M, a.K, a.N) : 1, 0};
-    if (w8 && must_reduce && red_ok) {
-        const SplitPlan p = reduce_plan(a.M, a.K, a.N);
-        const int64_t per_wave = ((a.K / 32 + p.S - 1) / p.S + kWaves - 1) / kWaves;
-        if (per_wave <= split_max_units(p.RT) && ((a.N + 31) / 32) % p.RT == 0) plan = p;
-    }
-    const int64_t S = plan.S;
-    // planes without a LayerNorm or residual from one split: the product
-    // kernel writes them itself (its 32 columns are one unit of the next
-    // linear's K), no reduction launch
-    const bool product_planes = planes_out && !next_ln_w && !a.fuse.res && S == 1 && a.N % 32 == 0;
-    const bool reduce = !product_planes && (S > 1 || planes_out);
-    // every wavefront's share of K fits its weight registers
-    const int64_t units = ((a.K / 32 + S - 1) / S + kWaves - 1) / kWaves;
-    if (plan.RT == 0 && units > (w8 ? max_units<kW8>() : max_units<kF32>())) return TIQ_EUNSUPPORTED;
+    DecodeShape shape;
+    if (!decode_shape(w8, a.M, a.K, a.N, planes_out, next_ln_w || a.fuse.res, shape)) return TIQ_EUNSUPPORTED;
+    SplitPlan plan = shape.plan;
+    const bool product_planes = shape.product_planes, reduce = shape.reduce;
     if (!aligned(a.w, 16) || a.ldw % 16 != 0) return TIQ_EALIGN;
     if (x_planes ? !aligned(x_planes, 16)
                  : (!a.x || !aligned(a.x, 16) || a.ldx % 4 != 0 ||

@@ -91,6 +91,7 @@ size_t skinny_workspace(int64_t M, int64_t K);
 // epilogue and optionally writes the next linear's LayerNorm'd operand planes
 // (planes_out, K' = N). The input is fp32 rows (a.x, with a.fuse.ln_w) or the
 // planes of a previous call (x_planes).
+bool decode_linear_takes(WFormat fmt, int64_t M, int64_t K, int64_t N, bool planes_out, bool finish);
 int run_decode_linear(const LinearArgs& a, const uint16_t* x_planes, const float* next_ln_w,
                       const float* next_ln_b, float next_eps, uint16_t* planes_out);
 

@@ -54,6 +54,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
     "tiq_linear_workspace": ([_i32, _i32, _i64, _i64, _i64], _sz),
     "tiq_gemm_w8_ws": ([_vp, _i32, _i64, _i64, _i64, _vp, _vp, _vp, _i64, _vp, _i32, _i64, _vp, _sz, _vp], _i32),
     "tiq_decode_linear_workspace": ([_i32, _i64, _i64, _i64], _sz),
+    "tiq_decode_linear_takes": ([_i32, _i64, _i64, _i64, _i32, _i32], _i32),
     "tiq_decode_planes_bytes": ([_i64, _i64], _sz),
     "tiq_tile_int8": ([_vp, _i64, _i64, _i64, _vp, _vp], _i32),
     "tiq_tile_int4": ([_vp, _i64, _i64, _vp, _vp], _i32),

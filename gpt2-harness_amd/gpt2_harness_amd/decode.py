@@ -202,6 +202,21 @@ def _layer_norm(ln, x: torch.Tensor) -> torch.Tensor:
     return ln(x)
 
 
+def _chain_takes(L, batch: int, block) -> bool:
+    """Whether the batched chain's products take a block's Linears: int8, or int4 in
+    whole operand tiles, at widths within the products' registers and the
+    reduction's 8192 columns (not c_fc from 3072 inputs on, whose K is split)."""
+    roles = ((block.attn.c_attn, 0, 0), (block.attn.c_proj, 1, 1), (block.mlp.c_fc, 1, 0), (block.mlp.c_proj, 1, 1))
+    for lin, planes_out, finish in roles:
+        whole = lin.out_features % 32 == 0 and lin.in_features % 32 == 0
+        if lin.fmt != FMT_W8 and (lin.fmt != FMT_W4 or not whole):
+            return False
+        wf = _TILED[_WF[lin.fmt]] if whole else _lib.WF_INT8
+        if not L.tiq_decode_linear_takes(wf, batch, lin.in_features, lin.out_features, planes_out, finish):
+            return False
+    return True
+
+
 class FusedDecoder(_DecoderBase):
     """Decode step built from the library's fused decode kernels.
 
@@ -246,9 +261,7 @@ class FusedDecoder(_DecoderBase):
         # planes (tiq_decode_linear), so no separate LayerNorm / split launches
         lins = [l for b in model.h for l in (b.attn.c_attn, b.attn.c_proj, b.mlp.c_fc, b.mlp.c_proj)]
         head_ok = self.head_q is None or self.head_q.fmt == FMT_W8
-        # (int4 codes only in operand tiles, so whole ones)
-        self.chain = 5 <= B <= 64 and head_ok and all(
-            l.fmt == FMT_W8 or (l.fmt == FMT_W4 and l.out_features % 32 == 0 and l.in_features % 32 == 0) for l in lins)
+        self.chain = 5 <= B <= 64 and head_ok and all(_chain_takes(self.L, B, b) for b in model.h)
         self.rows_prefill = all(l.fmt == FMT_W8 for l in lins)
         # One sequence with the tied fp32 head: the decode step's head and
         # argmax read an int8 (or bf16) copy of the head and recompute from

@@ -345,6 +345,11 @@ int tiq_linear_fused_ws(const void* x, int x_dtype, int64_t M, int64_t K, int64_
  *   bytes, 16-byte aligned; clobbered.
  * No counterpart in the reference (its decode runs one torch op per step). */
 size_t tiq_decode_linear_workspace(int w_format, int64_t M, int64_t K, int64_t N);
+
+/* 1 where tiq_decode_linear takes this shape (aligned operands and a workspace
+ * provided), else 0. planes_out: operand planes are asked for; finish: with a
+ * residual or the next LayerNorm before them. */
+int tiq_decode_linear_takes(int w_format, int64_t M, int64_t K, int64_t N, int planes_out, int finish);
 size_t tiq_decode_planes_bytes(int64_t M, int64_t K);
 
 /* The int8 codes of an (N, K) weight (leading dimension ldw bytes, 16-byte

@@ -303,3 +303,26 @@ def test_greedy_agreement_reports_first_divergence():
     assert b["first_divergence"] == {"step": 5, "sequence": 2, "oracle_top2_margin": float(gaps[5, 2]),
                                      "steps_all_equal": 5}
     assert abs(b["min_top2_margin"] - 0.001) < 1e-6
+
+
+def test_decode_linear_takes_the_reductions_reach():
+    """The batched decode chain's query about its own limits: planes of a c_fc whose
+    K is split (from 3072) pass the reduction, 8192 columns; 64 rows; whole tiles."""
+    L = _lib.load()
+    int4, int8, f32, f32t = _lib.WF_INT4_TILED, _lib.WF_INT8_TILED, _lib.WF_F32, _lib.WF_F32_TILED
+    for wf in (int4, int8):
+        assert L.tiq_decode_linear_takes(wf, 8, 3040, 4 * 3040, 1, 0)
+        assert not L.tiq_decode_linear_takes(wf, 8, 3072, 4 * 3072, 1, 0)
+        assert L.tiq_decode_linear_takes(wf, 8, 3072, 8192, 1, 0)
+        assert L.tiq_decode_linear_takes(wf, 8, 12288, 3072, 1, 1)
+        assert not L.tiq_decode_linear_takes(wf, 8, 1024, 8224, 1, 1)
+        assert L.tiq_decode_linear_takes(wf, 8, 6400, 50272, 0, 0)
+        assert not L.tiq_decode_linear_takes(wf, 8, 6432, 50272, 0, 0)
+        assert not L.tiq_decode_linear_takes(wf, 8, 768, 776, 0, 0)
+        assert not L.tiq_decode_linear_takes(wf, 65, 768, 768, 0, 0)
+    assert L.tiq_decode_linear_takes(_lib.WF_INT8, 8, 768, 776, 0, 0)
+    assert not L.tiq_decode_linear_takes(_lib.WF_INT4, 8, 768, 768, 0, 0)
+    assert L.tiq_decode_linear_takes(f32t, 8, 8192, 50257, 0, 0)
+    assert not L.tiq_decode_linear_takes(f32t, 8, 224, 50257, 0, 0)
+    assert L.tiq_decode_linear_takes(f32, 8, 2048, 50257, 0, 0)
+    assert not L.tiq_decode_linear_takes(f32, 8, 2080, 50257, 0, 0)

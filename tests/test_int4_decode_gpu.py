@@ -115,3 +115,16 @@ def test_int4_batched_decoder(dev, batch, bits, granularity):
     with torch.no_grad():
         logits = qm(want[:, :-1])["logits"][:, -1]
     assert torch.allclose(dec.logits, logits, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_widths_past_the_chain(dev, bits):
+    """A block whose c_fc the chain does not take (3072 inputs) keeps one fused
+    product a Linear."""
+    torch.manual_seed(0)
+    cfg = g.GPTConfig(vocab_size=320, n_positions=32, n_layer=1, n_head=48, n_embd=3072)
+    qm, _ = g.quantize_model(g.GPT(cfg).to(dev).eval(), bits)
+    idx = torch.randint(0, cfg.vocab_size, (6, 4), device=dev)
+    dec = g.FusedDecoder(qm, 6, 16)
+    assert not dec.chain
+    assert torch.equal(dec.run(idx, 6), g.generate(qm, idx, 6))
