@@ -162,6 +162,49 @@ def test_attention_falls_back_to_copies(dev):
     assert torch.equal(y, ref) and full.length(0) == 128
 
 
+class _Recording(KVCache):
+    def update(self, layer, k, v):
+        self.seen = getattr(self, "seen", 0) + k.shape[-2]
+        return super().update(layer, k, v)
+
+
+class _Duck:
+    """The members a forward pass uses, and no others."""
+
+    def __init__(self):
+        self.inner, self.seen = KVCache(1), 0
+
+    @property
+    def seq_len(self):
+        return self.inner.seq_len
+
+    def length(self, layer):
+        return self.inner.length(layer)
+
+    def update(self, layer, k, v):
+        self.seen += k.shape[-2]
+        return self.inner.update(layer, k, v)
+
+
+@torch.no_grad()
+def test_caches_with_an_update_of_their_own(dev):
+    blk = _block("int8", dev)
+    x = _rows(128, 768, dev).view(1, 128, 768)
+    plain = KVCache(1)
+    want = blk(x, plain)
+    patched, seen = KVCache(1), []
+    update = patched.update
+    patched.update = lambda layer, k, v: (seen.append(k.shape[-2]), update(layer, k, v))[1]
+    for cache in (_Recording(1), _Duck(), patched):
+        y = blk(x, cache)
+        inner = getattr(cache, "inner", cache)
+        assert (sum(seen) if cache is patched else cache.seen) == 128 and cache.length(0) == 128
+        assert torch.equal(inner.keys[0], plain.keys[0]) and torch.equal(inner.values[0], plain.values[0])
+        assert torch.equal(y, want)
+        assert torch.equal(CausalSelfAttention.forward(blk.attn, x, type(cache)() if cache.__class__ is _Duck
+                                                       else type(cache)(1)), blk.attn(x))
+
+
 def test_arguments(dev):
     lin = _linear(768, 2304, "int8", dev)
     L, M, K, N = _lib.lib(), 128, 768, 2304
