@@ -68,9 +68,9 @@ __global__ __launch_bounds__(256) void split_planes_kernel(const float* __restri
                                   (32 * h + (m & 31)) * 16) = p[q];
 }
 
-__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const uint8_t* __restrict__ x3, const float* __restrict__ w,
-                                                          int64_t ldw, float* __restrict__ y, int64_t ldy, int M,
-                                                          int N, int K) {
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const uint8_t* __restrict__ x3, const float* __restrict__ x,
+                                                          int64_t ldx, const float* __restrict__ w, int64_t ldw,
+                                                          float* __restrict__ y, int64_t ldy, int M, int N, int K) {
     __shared__ __attribute__((aligned(1024))) uint8_t smem[2][kFX * 1024];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -157,13 +157,44 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const uint8_t* __restr
     // 32 consecutive outputs of two rows a store, written once and read by a later kernel
     const int m0 = tm * kFM + 4 * h;
     if (n0 + r >= N) return;
+    float odd[kFT] = {};  // NaN where an output is not finite
 #pragma unroll
     for (int i = 0; i < kFT; ++i)
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             const int m = m0 + 32 * i + 8 * (q >> 2) + (q & 3);
-            if (m < M) __builtin_nontemporal_store(acc[i][q], y + (int64_t)m * ldy + n0 + r);
+            if (m < M) {
+                __builtin_nontemporal_store(acc[i][q], y + (int64_t)m * ldy + n0 + r);
+                odd[i] = fmaf(acc[i][q], 0.f, odd[i]);
+            }
         }
+    if ((odd[0] + odd[1]) + (odd[2] + odd[3]) == 0.f) return;
+    // An operand that is infinite or rounds to infinity in bf16 (from 3.39e38) has a
+    // NaN plane, and so has every output of it: those as plain fp32 sums, which give
+    // infinities and NaN their meaning. The chain ends where it is NaN.
+    uint64_t todo = 0;
+#pragma unroll
+    for (int i = 0; i < kFT; ++i)
+#pragma unroll
+        for (int q = 0; q < 16; ++q)
+            todo |= (uint64_t)(acc[i][q] != acc[i][q]) << (16 * i + q);
+    const float4* wn = reinterpret_cast<const float4*>(w + (int64_t)(n0 + r) * ldw);
+    while (todo) {
+        const int o = __builtin_ctzll(todo);
+        todo &= todo - 1;
+        const int m = m0 + 32 * (o >> 4) + 8 * (o >> 2 & 3) + (o & 3);
+        if (m >= M) continue;
+        const float4* xm = reinterpret_cast<const float4*>(x + (int64_t)m * ldx);
+        float s = 0.f;
+        for (int k = 0; k < K / 4 && s == s; ++k) {
+            const float4 a = xm[k], b = wn[k];
+            s = fmaf(a.x, b.x, s);
+            s = fmaf(a.y, b.y, s);
+            s = fmaf(a.z, b.z, s);
+            s = fmaf(a.w, b.w, s);
+        }
+        y[(int64_t)m * ldy + n0 + r] = s;
+    }
 }
 
 // From 65 rows: at 64 the platform's GEMM has a tile of its own (width 1024 70 us
@@ -198,7 +229,7 @@ extern "C" int tiq_linear_f32_ws(const float* x, int64_t M, int64_t K, int64_t l
     const int rc = launch_status();
     if (rc != TIQ_OK) return rc;
     const int64_t tiles = ((M + kFM - 1) / kFM) * ((N + kFN - 1) / kFN);
-    hipLaunchKernelGGL(gemm_f32_kernel, dim3((unsigned)tiles), dim3(256), 0, as_stream(stream), x3, w, ldw, y, ldy,
-                       (int)M, (int)N, (int)K);
+    hipLaunchKernelGGL(gemm_f32_kernel, dim3((unsigned)tiles), dim3(256), 0, as_stream(stream), x3, x, ldx, w, ldw,
+                       y, ldy, (int)M, (int)N, (int)K);
     return launch_status();
 }

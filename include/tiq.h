@@ -531,7 +531,8 @@ int tiq_linear_prefill_ws(const float* x, int64_t M, int64_t K, int64_t ldx, con
 
 /* y = x w^T, fp32 rows against fp32 weights: the tied lm_head over every
  * position of a batch (model.py:585) on the bf16 matrix cores, both operands as
- * three bf16 planes, as accurate as an fp32 GEMM (an infinite operand gives NaN).
+ * three bf16 planes, as accurate as an fp32 GEMM (an output whose planes give NaN,
+ * as those of an infinite operand do, is computed as an fp32 sum).
  * x (M, K) and w (N, K) 16-byte aligned, ldx % 4 == 0, ldw % 4 == 0, K % 32 == 0,
  * M >= 65, N >= 4096: TIQ_EUNSUPPORTED for other sizes, whose workspace is 0;
  * y any alignment. The workspace holds the planes of x. */

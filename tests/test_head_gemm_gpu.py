@@ -45,6 +45,34 @@ def test_head_over_a_batch(dev, M, K, N):
     assert err.norm() <= 1.125 * ((x @ w.t()).double() - ref).norm() + 1e-30
 
 
+@pytest.mark.parametrize("M,K,N", [(65, 96, 4097), (130, 768, 4224)])
+def test_head_of_infinities(dev, M, K, N):
+    """Infinities, NaN and values that round to infinity in bf16 mean in x and w what
+    they mean in an fp32 sum; other outputs do not notice."""
+    gen = torch.Generator(device=dev).manual_seed(M)
+    x = torch.randn(M, K, generator=gen, device=dev)
+    w = torch.randn(N, K, generator=gen, device=dev) * 0.02
+    w[5::7, 3] = 0.0  # inf times zero
+    plain, y = torch.empty(M, N, device=dev), torch.empty(M, N, device=dev)
+    assert _call(x, w, plain) == _lib.OK
+    inf, top = float("inf"), torch.finfo(torch.float32).max
+    for m, v in ((0, inf), (7, -inf), (33, float("nan")), (40, top), (41, 3.393e38), (M - 1, -3.4e38)):
+        x[m, 3] = v
+    for n, v in ((2, -inf), (100, 1e30), (4096, top)):
+        w[n, K - 1] = v
+    assert _call(x, w, y) == _lib.OK
+    ref = (x.double() @ w.double().t()).float()  # past fp32's range: infinite
+    finite = x.isfinite().all(1, keepdim=True) & w.isfinite().all(1)
+    assert torch.equal(y.isnan(), ref.isnan())
+    assert torch.equal(y[~finite & ~ref.isnan()], ref[~finite & ~ref.isnan()])
+    work = x.double().abs() @ w.double().abs().t()
+    ok = finite & (work < top)
+    assert bool(((y.double() - ref.double()).abs() <= (K + 8) * 2.0**-24 * work)[ok].all())
+    rows = [m for m in range(M) if m not in (0, 7, 33, 40, 41, M - 1)]
+    cols = [n for n in range(N) if n not in (2, 100, 4096)]
+    assert torch.equal(y[rows][:, cols], plain[rows][:, cols])
+
+
 def test_head_refusals(dev):
     x, w, y = (torch.zeros(s, device=dev) for s in ((65, 64), (4096, 64), (65, 4096)))
     L = _lib.lib()
