@@ -284,8 +284,7 @@ extern "C" size_t tiq_gemm_w8_workspace(int x_dtype, int64_t M, int64_t K, int64
     if ((x_dtype != TIQ_F32 && x_dtype != TIQ_BF16) || K <= 0 || K % 64 != 0 || N <= 0) return 0;
     if (!(x_dtype == TIQ_F32 ? M >= kGemmMinRows || w4_planes_rows(M, K, N) : bf16_gemm_rows(M, K, N))) return 0;
     if (x_dtype == TIQ_F32)
-        return std::max(split_workspace(M, K), digits_workspace(M, K)) +
-               std::max(staged_split_workspace(M, N, 3 * K), digits_split_workspace(M, N, K));
+        return std::max(split_workspace(M, K), digits_workspace(M, K)) + digits_split_workspace(M, N, K);
     return staged_split_workspace(M, N, K);
 }
 

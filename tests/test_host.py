@@ -326,3 +326,14 @@ def test_decode_linear_takes_the_reductions_reach():
     assert not L.tiq_decode_linear_takes(f32t, 8, 224, 50257, 0, 0)
     assert L.tiq_decode_linear_takes(f32, 8, 2048, 50257, 0, 0)
     assert not L.tiq_decode_linear_takes(f32, 8, 2080, 50257, 0, 0)
+
+
+@pytest.mark.parametrize("wf", [_lib.WF_INT8, _lib.WF_INT4, _lib.WF_INT4G])
+def test_fp32_workspace_holds_planes_and_the_digit_products_slices(wf):
+    """Nothing for slices that no product writes: 6 bytes an element of x (the planes),
+    and fp32 slices only where the digit planes' product is split over K."""
+    L = _lib.load()
+    assert L.tiq_linear_workspace(wf, _lib.F32, 512, 1600, 4800) == 6 * 512 * 1600   # 608 tiles
+    assert L.tiq_linear_workspace(wf, _lib.F32, 4096, 6400, 1600) == 6 * 4096 * 6400
+    # 128 rows of 3072 x 768: 24 tiles, eight splits of 48 k64 steps
+    assert L.tiq_linear_workspace(wf, _lib.F32, 128, 3072, 768) == 6 * 128 * 3072 + 8 * 4 * 128 * 768
