@@ -194,7 +194,7 @@ int launch_staged_gemm(const LinearArgs& a, int choice) {
 }
 
 int launch_staged_gemm_split(const LinearArgs& a, void* ws, size_t ws_bytes) {
-    if ((a.fmt != kW8 && a.fmt != kW4) || !staged_supported_impl(a)) return TIQ_EUNSUPPORTED;
+    if ((a.fmt != kW8 && a.fmt != kW4) || a.kw || !staged_supported_impl(a)) return TIQ_EUNSUPPORTED;
     // 48 tiles or more and a short K: the slices' trip through memory costs
     // more than the idle CUs (GPT-2-XL at M = 256 with N >= 4800 and at
     // M = 1024 with N = K = 1600: 7-11% slower split; M = 512, N = K = 1600,
@@ -210,11 +210,11 @@ int launch_staged_gemm_split(const LinearArgs& a, void* ws, size_t ws_bytes) {
     if (a.fmt == kW4)
         hipLaunchKernelGGL((gemm_staged<128, 128, 2, kW4, float>), grid, dim3(256), 0, a.stream,
                            static_cast<const uint16_t*>(a.x), a.ldx, a.w, a.ldw, a.scale, a.bias, part, (int64_t)a.N,
-                           (int)a.M, (int)a.N, (int)a.K, (int)(a.kw ? a.kw : a.K), nullptr, 0, nullptr);
+                           (int)a.M, (int)a.N, (int)a.K, (int)a.K, nullptr, 0, nullptr);
     else
         hipLaunchKernelGGL((gemm_staged<128, 128, 2, kW8, float>), grid, dim3(256), 0, a.stream,
                            static_cast<const uint16_t*>(a.x), a.ldx, a.w, a.ldw, a.scale, a.bias, part, (int64_t)a.N,
-                           (int)a.M, (int)a.N, (int)a.K, (int)(a.kw ? a.kw : a.K), nullptr, 0, nullptr);
+                           (int)a.M, (int)a.N, (int)a.K, (int)a.K, nullptr, 0, nullptr);
     int rc = launch_status();
     if (rc != TIQ_OK) return rc;
     return launch_splitk_reduce(a, part, S, a.scale);

@@ -155,11 +155,11 @@ bool digits_rows(WFormat fmt, int64_t M, int64_t K, int64_t N) {
     return w4_planes_rows(M, K, N) && (fmt == kW4 || M * N * K >= 24000000);
 }
 
-// fp32 activations through the matrix cores: int8 and reference-layout int4
-// weights as exact integer products of digit planes (gemm_digits.hip), else
-// (group-wise int4, or K past the int32 sums) split into three bf16 planes for
-// a GEMM that takes the three-plane problem; TIQ_EUNSUPPORTED otherwise (the
-// caller falls back). gelu_in: the product takes gelu_tanh(x).
+// fp32 activations through the matrix cores: as exact integer products of digit
+// planes (gemm_digits.hip), else (K past their int32 sums, 65536, or weights past
+// 32-bit offsets) split into three bf16 planes for a GEMM that takes the
+// three-plane problem; TIQ_EUNSUPPORTED otherwise (groups that are no multiple of
+// 64 columns, say: the caller falls back). gelu_in: the product takes gelu_tanh(x).
 int run_linear_split(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu_in = false) {
     if (a.x_dtype != TIQ_F32 || a.fmt == kF32 || a.K % 4 != 0) return TIQ_EUNSUPPORTED;
     const bool few = a.M < kGemmMinRows;  // below the documented row count: the workspace is optional

@@ -168,3 +168,29 @@ def test_digit_planes_extreme_rows(dev):
         assert bool(yb[m].isnan().all())
     keep = [m for m in range(M) if m not in (7, 9, 11)]
     assert torch.equal(yb[keep], y[keep])
+
+
+# Past the 65536 columns whose digit sums fit int32: three bf16 planes and the bf16
+# GEMMs (the staged one; the LDS one for groups). Bound: one rounding a product of
+# the three planes' sums in the worst order, two more an output.
+@pytest.mark.parametrize("fmt", ["int8", "int4", "g128"])
+@torch.no_grad()
+def test_columns_past_the_digit_sums(dev, fmt):
+    K, N, M = 65664, 96, 130
+    gen = torch.Generator(device=dev).manual_seed(3)
+    lin = torch.nn.Linear(K, N, device=dev)
+    lin.weight.data = torch.randn(N, K, generator=gen, device=dev) * 0.02
+    mod = g.quantize_linear(lin, 8 if fmt == "int8" else 4, group_size=128 if fmt == "g128" else None)[0]
+    if fmt == "int8":
+        w = mod.codes.double() * mod.scale.double().unsqueeze(1)
+    else:
+        w = g.unpack_int4(mod.codes, N * K).view(N, K).double()
+        w *= mod.scale.double().repeat_interleave(128, dim=1) if fmt == "g128" else mod.scale.double().unsqueeze(1)
+    x = torch.randn(M, K, generator=gen, device=dev)
+    x[:, ::97] *= 1e4  # nothing is held relative to the row's largest
+    for y, v in ((mod(x), x), (mod.forward_gelu_in(x), g.model.gelu_tanh(x))):
+        ref = v.double() @ w.t() + mod.bias.double()
+        err = (y.double() - ref).abs()
+        work = v.double().abs() @ w.abs().t() + mod.bias.double().abs()
+        assert bool((err <= (K + 2) * 2.0**-24 * work).all())
+        assert err.norm() <= 3.0 * K**0.5 * 2.0**-24 * ref.norm()
