@@ -1018,6 +1018,7 @@ int launch_gemv(const LinearArgs& a) {
         case kF32: return dispatch_types<kF32>(a);
         // operand-tile layouts are read by the batched decode kernels only
         case kW8T:
+        case kW4T:
         case kF32T: return TIQ_EUNSUPPORTED;
     }
     return TIQ_EINVAL;

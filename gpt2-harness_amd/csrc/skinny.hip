@@ -373,9 +373,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
     const uint16_t* x3t = reinterpret_cast<const uint16_t*>(x) + (int64_t)blockIdx.y * (K / 32) * 6 * 64 * 8 + lane * 8;
     // row-major: row n0 + r, + 2 WB u per unit; tiles: this row tile's 1 KB
     // blocks (N % 32 == 0, the host checks), + 1024 u per unit
-    const uint8_t* wr = WF == kW8T || WF == kW4T
-                            ? w + ((int64_t)blockIdx.x * U * 64 + lane) * WB
-                                   : w + (int64_t)min(n0 + r, N - 1) * ldw + WB * h;
+    const uint8_t* wr = WF == kW8T || WF == kW4T ? w + ((int64_t)blockIdx.x * U * 64 + lane) * WB
+                                                 : w + (int64_t)min(n0 + r, N - 1) * ldw + WB * h;
 
     const int cnt = u1 - u0;  // <= kUnits (the host checks K)
     constexpr int kUnits = XM == kXBf16 ? kXbUnits : max_units<WF>();
@@ -579,7 +578,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void skinny_kernel(
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const u32x4 t = xrow_ok ? xv[e] : u32x4{0u, 0u, 0u, 0u};
-                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(code_frag(wv[0], e), __builtin_bit_cast(bf16x8, t), acc, 0, 0,
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(code_frag(wv[0], e), __builtin_bit_cast(bf16x8, t), acc, 0, 0,
                                                           0);
         }
     };

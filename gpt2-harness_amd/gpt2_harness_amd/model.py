@@ -371,7 +371,6 @@ class Block(nn.Module):
         x = x + self._drop(self.attn(self.ln_1(x), cache))
         return x + self._drop(self.mlp(self.ln_2(x)))
 
-
     def _prefill(self, x: torch.Tensor, cache: KVCache | None) -> torch.Tensor | None:
         """The block over a prompt's rows with quantized Linears: both
         LayerNorms inside the Linear that follows, both residual adds at the end
