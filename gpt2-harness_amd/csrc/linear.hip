@@ -73,10 +73,12 @@ bool w4_planes_rows(int64_t M, int64_t K, int64_t N) {
 // tile (us, GEMV / GEMM: int8 1600 x 4800 M = 100 166 / 17, 6400 x 1600 M = 24
 // 35 / 14; int4 768 x 2304 M = 8 12.0 / 9.7, 1024 x 4096 M = 64 85 / 11). Up to 16 rows on
 // matrices under 2048 rows the GEMV's direct kernel is ahead (3072 x 768 M = 16
-// 6.8 / 12) until the product is large (6400 x 1600 M = 16 30 / 16).
+// 6.8 / 12) until the product is large (6400 x 1600 M = 16 30 / 16). Up to four rows
+// its one pass over the weights is ahead at every size (1600 x 6400, M = 4: int4 6.8 / 16.6,
+// group-wise 12.7 / 18.4; M = 2: int8 4.5 / 14.3).
 bool bf16_gemm_rows(int64_t M, int64_t K, int64_t N) {
     const int64_t work = M * N * K;
-    return M >= kGemmMinRows || M > 64 || (M > 16 || N >= 2048 ? work >= 14000000 : work >= 100000000);
+    return M > 64 || (M > 4 && (M > 16 || N >= 2048 ? work >= 14000000 : work >= 100000000));
 }
 
 LinearArgs make_args(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx, const uint8_t* w, int64_t ldw,

@@ -337,3 +337,13 @@ def test_fp32_workspace_holds_planes_and_the_digit_products_slices(wf):
     assert L.tiq_linear_workspace(wf, _lib.F32, 4096, 6400, 1600) == 6 * 4096 * 6400
     # 128 rows of 3072 x 768: 24 tiles, eight splits of 48 k64 steps
     assert L.tiq_linear_workspace(wf, _lib.F32, 128, 3072, 768) == 6 * 128 * 3072 + 8 * 4 * 128 * 768
+
+
+def test_up_to_four_bf16_rows_keep_the_decode_gemv():
+    """No product of up to four rows is large enough for the GEMM (whose split-K
+    workspace says which rows take it); from five on it takes wide matrices."""
+    L = _lib.load()
+    for K, N in ((1600, 4800), (1280, 5120), (6400, 1600), (1600, 50304), (12800, 12800)):
+        assert all(L.tiq_gemm_w8_workspace(_lib.BF16, M, K, N) == 0 for M in (1, 2, 3, 4))
+    assert L.tiq_gemm_w8_workspace(_lib.BF16, 5, 1600, 4800) > 0
+    assert L.tiq_gemm_w8_workspace(_lib.BF16, 65, 768, 768) > 0
