@@ -147,14 +147,21 @@ size_t split_workspace(int64_t M, int64_t K) { return (size_t)(M * 3 * K * 2 + 2
 // int8 has the batched kernel up to 64 rows, which holds a wavefront's whole
 // share of K and reads every activation plane for each 32-row tile: past 32
 // rows of a long K the planes win (us, batched / planes: 1600 x 4800 M = 64 21 /
-// 15, 6400 x 1600 M = 32 32 / 20; 768 x 3072 M = 64 7.5 / 10.7); from 65 rows the
+// 15, 6400 x 1600 M = 32 32 / 20, 3072 x 768 M = 48 17.2 / 12.5; 768 x 3072 M = 64 7.5 / 10.7
+// and, with few rows of weights, 1600 x 1600 M = 64 10.6 / 12.1); from 65 rows the
 // only other kernel is the decode GEMV (77 rows, 768 x 3072: 56 / 11). int4 as
 // w4_planes_rows, group-wise also only from the size at which its GEMV falls
-// behind (768 x 768: M = 32 10.9 / 14.2, M = 48 16.4 / 14.4).
+// behind (768 x 768: M = 32 10.9 / 14.2, M = 48 16.4 / 14.4) and, where K is too short
+// to be split and so one long chain of folds, not up to 8 rows (1024 x 4096 10.8 / 15.5,
+// 1280 x 5120 15.7 / 18.0) or, between, 12 (1024 x 4096 15.8 / 16.5; 768 x 3072 15.2 / 13.7,
+// 1280 x 5120 20.7 / 18.7).
 bool digits_rows(WFormat fmt, int64_t M, int64_t K, int64_t N) {
     if (M >= kGemmMinRows) return true;
-    if (fmt == kW8) return M > 64 || (M > 32 && K >= 1536) || (M == 32 && K >= 3072);
-    return w4_planes_rows(M, K, N) && (fmt == kW4 || M * N * K >= 24000000);
+    if (fmt == kW8) return M > 64 || (M > 32 && K >= 1536 && (K >= 2048 || N >= 2048)) || (M == 32 && K >= 3072);
+    if (!w4_planes_rows(M, K, N)) return false;
+    if (fmt == kW4) return true;
+    if (K < 1536 && M <= (K >= 1024 && K < 1280 ? 12 : 8)) return false;
+    return M * N * K >= 24000000;
 }
 
 // fp32 activations through the matrix cores: as exact integer products of digit

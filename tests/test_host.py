@@ -347,3 +347,23 @@ def test_up_to_four_bf16_rows_keep_the_decode_gemv():
         assert all(L.tiq_gemm_w8_workspace(_lib.BF16, M, K, N) == 0 for M in (1, 2, 3, 4))
     assert L.tiq_gemm_w8_workspace(_lib.BF16, 5, 1600, 4800) > 0
     assert L.tiq_gemm_w8_workspace(_lib.BF16, 65, 768, 768) > 0
+
+
+def test_fp32_rows_that_keep_their_row_kernels():
+    """Below 128 rows the digit planes (whose workspace says which rows take them) only
+    where they are ahead: not 33..64 int8 rows of a small matrix, not 8 (at 1024 columns
+    12) group-wise rows of a K that is not split."""
+    L = _lib.load()
+
+    def takes(wf, M, K, N):
+        return L.tiq_linear_workspace(wf, _lib.F32, M, K, N) > 0
+
+    for M in (33, 64):
+        assert not takes(_lib.WF_INT8, M, 1600, 1600)
+        assert takes(_lib.WF_INT8, M, 1600, 4800) and takes(_lib.WF_INT8, M, 3072, 768)
+    assert takes(_lib.WF_INT8, 65, 1600, 1600)
+    assert not takes(_lib.WF_INT4G, 8, 1024, 4096) and not takes(_lib.WF_INT4G, 12, 1024, 4096)
+    assert takes(_lib.WF_INT4G, 13, 1024, 4096)
+    assert not takes(_lib.WF_INT4G, 8, 1280, 5120) and takes(_lib.WF_INT4G, 9, 1280, 5120)
+    assert takes(_lib.WF_INT4G, 8, 1600, 4800)
+    assert takes(_lib.WF_INT4, 8, 1024, 4096)
