@@ -947,6 +947,9 @@ size_t digits_split_workspace(int64_t M, int64_t N, int64_t K) {
     return S > 1 ? round256((size_t)(S * M * N * 4)) : 0;
 }
 
+// A product that is split for want of tiles leaves its key and value columns to the caller.
+bool digits_write_kv(int64_t M, int64_t K, int64_t N) { return N % 192 == 0 && digits_splits(M, N, K) == 1; }
+
 bool digits_supported(const LinearArgs& a) {
     if (a.x_dtype != TIQ_F32 || (a.fmt != kW8 && a.fmt != kW4 && a.fmt != kW4G) || a.kw) return false;
     // group-wise: whole k64 steps a group, rows of whole nibble pairs
@@ -962,9 +965,8 @@ bool digits_supported(const LinearArgs& a) {
 int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu, const PrefillFusion& f) {
     if (!digits_supported(a)) return TIQ_EUNSUPPORTED;
     if (f.ln_w && (a.K > kDigitsLnMaxK || !aligned(f.ln_w, 16) || !aligned(f.ln_b, 16))) return TIQ_EUNSUPPORTED;
-    // rows of a sequence by multiplication: m T < 2^32; a product that is split
-    // for want of tiles leaves its key and value columns to the caller
-    if (f.k && (a.N % 192 != 0 || a.M * f.T > 0xffffffffLL || digits_splits(a.M, a.N, a.K) > 1)) return TIQ_EUNSUPPORTED;
+    // rows of a sequence by multiplication: m T < 2^32
+    if (f.k && (!digits_write_kv(a.M, a.K, a.N) || a.M * f.T > 0xffffffffLL)) return TIQ_EUNSUPPORTED;
     const size_t need = digits_workspace(a.M, a.K);
     if (!ws || ws_bytes < need || !aligned(ws, 16)) return TIQ_EWORKSPACE;
     uint8_t* xt = static_cast<uint8_t*>(ws);

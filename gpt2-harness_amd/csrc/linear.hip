@@ -344,6 +344,12 @@ extern "C" int tiq_linear_gelu_in_ws(const float* x, int64_t M, int64_t K, int64
     return run_linear_split(a, workspace, workspace_bytes, true);
 }
 
+extern "C" int tiq_linear_prefill_writes_kv(int w_format, int64_t M, int64_t K, int64_t N) {
+    if (w_format != TIQ_WF_INT8 && w_format != TIQ_WF_INT4 && w_format != TIQ_WF_INT4_GROUPWISE) return 0;
+    if (M <= 0 || K <= 0 || K % 64 != 0 || N <= 0 || !digits_rows((WFormat)w_format, M, K, N)) return 0;
+    return digits_write_kv(M, K, N);
+}
+
 extern "C" int tiq_linear_prefill_ws(const float* x, int64_t M, int64_t K, int64_t ldx, const void* w, int w_format,
                                      const float* scale, const uint16_t* scale_f16, int group, const float* bias,
                                      int64_t N, float* y, int64_t ldy, const float* ln_weight, const float* ln_bias,

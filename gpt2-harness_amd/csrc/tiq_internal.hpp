@@ -172,6 +172,8 @@ constexpr int64_t kDigitsLnMaxK = 2048;
 size_t digits_workspace(int64_t M, int64_t K);
 size_t digits_split_workspace(int64_t M, int64_t N, int64_t K);
 bool digits_supported(const LinearArgs& a);
+// Whether the product can put a c_attn's key and value columns into the caches.
+bool digits_write_kv(int64_t M, int64_t K, int64_t N);
 int launch_digits(const LinearArgs& a, void* ws, size_t ws_bytes, bool gelu, const PrefillFusion& fuse = {});
 
 }  // namespace tiq

@@ -78,6 +78,7 @@ SIGNATURES: dict[str, tuple[list, object]] = {
                               _i32),
     "tiq_linear_prefill_ws": ([_vp, _i64, _i64, _i64, _vp, _i32, _vp, _vp, _i32, _vp, _i64, _vp, _i64, _vp, _vp, _f32,
                                _i32, _vp, _i64, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _sz, _vp], _i32),
+    "tiq_linear_prefill_writes_kv": ([_i32, _i64, _i64, _i64], _i32),
     "tiq_linear_f32_workspace": ([_i64, _i64, _i64], _sz),
     "tiq_linear_f32_ws": ([_vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _vp, _sz, _vp], _i32),
     "tiq_prefill_attention": ([_vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64,

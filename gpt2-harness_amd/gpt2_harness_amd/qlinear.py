@@ -126,6 +126,10 @@ class QuantLinear(nn.Module):
             _lib.check(rc, f"quantized linear over gelu_tanh ({self.fmt}, M={M}, K={K}, N={N})")
         return y.view(*lead, N)
 
+    def writes_kv(self, M: int) -> bool:
+        """Whether :meth:`forward_prefill` over ``M`` rows takes ``kv``."""
+        return bool(_lib.lib().tiq_linear_prefill_writes_kv(_WF[self.fmt], M, self.in_features, self.out_features))
+
     def forward_prefill(self, x2: torch.Tensor, ln: nn.LayerNorm | None = None, gelu: bool = False,
                         residual: torch.Tensor | None = None,
                         kv: tuple[torch.Tensor, torch.Tensor, int] | None = None) -> torch.Tensor | None:

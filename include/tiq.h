@@ -528,6 +528,8 @@ int tiq_linear_prefill_ws(const float* x, int64_t M, int64_t K, int64_t ldx, con
                           int gelu_in, const float* residual, int64_t ld_residual, float* k_out, float* v_out,
                           int64_t kv_sb, int64_t kv_sh, int64_t kv_st, int64_t T, void* workspace,
                           size_t workspace_bytes, void* stream);
+/* 1 where tiq_linear_prefill_ws takes k_out for this shape, else 0. */
+int tiq_linear_prefill_writes_kv(int w_format, int64_t M, int64_t K, int64_t N);
 
 /* y = x w^T, fp32 rows against fp32 weights: the tied lm_head over every
  * position of a batch (model.py:585) on the bf16 matrix cores, both operands as

@@ -205,6 +205,26 @@ def test_caches_with_an_update_of_their_own(dev):
                                                        else type(cache)(1)), blk.attn(x))
 
 
+@torch.no_grad()
+def test_no_attempt_where_the_product_is_split(dev, monkeypatch):
+    """The attention asks before it makes room and calls: a product split over K, or
+    rows that are not its, would refuse the cache writes."""
+    calls = []
+    real = g.QuantLinear.forward_prefill
+    monkeypatch.setattr(g.QuantLinear, "forward_prefill", lambda self, *a, **k: (calls.append(1), real(self, *a, **k))[1])
+    for fmt, C, M, takes in (("g128", 1600, 24, False), ("g128", 1600, 300, True), ("int8", 768, 24, False),
+                             ("int8", 768, 65, True), ("int4", 1600, 129, True)):
+        blk, x = _block(fmt, dev, C), _rows(M, C, dev).view(1, M, C)
+        cache = KVCache(1)
+        assert blk.attn.c_attn.writes_kv(M) == takes
+        calls.clear()
+        y = blk.attn(x, cache)
+        assert len(calls) == takes and cache.length(0) == M
+        k, v = (torch.zeros(1, C // 64, M, 64, device=dev) for _ in range(2))
+        assert (real(blk.attn.c_attn, x.view(M, C), kv=(k, v, M)) is not None) == takes
+        assert _rel(y, blk.attn(x).double()) <= 2.0**-20
+
+
 def test_arguments(dev):
     lin = _linear(768, 2304, "int8", dev)
     L, M, K, N = _lib.lib(), 128, 768, 2304
