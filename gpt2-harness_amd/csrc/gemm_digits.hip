@@ -23,13 +23,13 @@
 // columns has: N(0, 1) with one element T, such outputs, K = 768: T = 1e3 3.0e-7 of
 // their norm, 1e5 3.5e-5, where an fp32 chain has 5e-7 at any T. So a row whose
 // largest element is more than kFar^2 sqrt(K) times the square of the mean square
-// root of its other elements (of each pair of neighbours the larger; no zeros) keeps
-// its fp32 bits, a byte a plane in the
-// digits' place and size, and rs < 0 marks it: the product computes its outputs once
-// more, by fp32 sums (wide_rows). The line lies where the digits' error on such
-// outputs reaches the chain's, which grows with sqrt(K) (one large element among
-// N(0, 1): T = 1400 at K = 768); the mean square root weighs a row's many elements and
-// not its few: a hidden row after GELU, mostly small, stays on this side.
+// root of its other elements (of each pair of neighbours the larger) keeps its fp32
+// bits, a byte a plane in the digits' place and size, and rs < 0 marks it: the product
+// computes its outputs once more, by fp32 sums (wide_rows). The line lies where the
+// digits' error on such outputs reaches the chain's, which grows with sqrt(K) (one
+// large element among N(0, 1): T = 1400 at K = 768); the mean square root weighs a
+// row's many elements and not its few: a hidden row after GELU, mostly small, stays on
+// this side (rows with less than 3% of their elements above zero do not).
 //
 // Why four int8 planes: int8 MFMAs run at twice the bf16 rate, so four planes
 // cost two bf16 passes over the product instead of three, and the codes enter
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
     static_assert(!LN || IT > 0, "LayerNorm needs the row in registers");
     static_assert(R == 8 || R == 4, "whole quads of rows");
     constexpr int WV = kSplitThreads / 64, CT = kSplitThreads / R;  // 16-column chunks a pass
-    __shared__ float4 stat[WV][R];
+    __shared__ float2 stat[WV][R];
     __shared__ float ls[2][WV][R];
     const int tid = threadIdx.x, row = tid % R, c0 = tid / R;
     const int m = blockIdx.x * R + row;
@@ -189,22 +189,18 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
         }
     };
     uint32_t mx = 0;
-    // over pairs of neighbours: the sum of their larger elements' square roots, how
-    // many are not zero (each element by itself is twice the instructions: the GELU'd
-    // split of 4096 x 6400 47 -> 53 us, by pairs 52)
-    float root = 0.f, count = 0.f;
+    // the sum, over pairs of neighbours, of their larger elements' square roots (each
+    // element by itself takes twice the instructions)
+    float root = 0.f;
     auto measure = [&](const float (&e)[16], bool mine) {
         float s = 0.f;
-        uint32_t n = 0;
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
             const uint32_t b = max(abs_bits(e[i]), abs_bits(e[i + 1]));
             mx = max(mx, b);
-            n += min(b, 1u);
             s += rough_root(b);
         }
         root += mine ? s : 0.f;
-        count += mine ? (float)n : 0.f;
     };
     float v[IT ? IT : 1][16];
     if constexpr (IT > 0) {
@@ -263,22 +259,20 @@ __global__ __launch_bounds__(kSplitThreads) void split_digits_kernel(const float
     }
     mx = max_across<R>(mx);
     root = sum_across<R>(root);
-    count = sum_across<R>(count);
-    if ((tid & 63) < R) stat[tid >> 6][row] = make_float4(__uint_as_float(mx), root, count, 0.f);
+    if ((tid & 63) < R) stat[tid >> 6][row] = make_float2(__uint_as_float(mx), root);
     __syncthreads();
-    root = count = 0.f;
+    root = 0.f;
 #pragma unroll
     for (int w = 0; w < WV; ++w) {
-        const float4 t = stat[w][row];
+        const float2 t = stat[w][row];
         mx = max(mx, __float_as_uint(t.x));
         root += t.y;
-        count += t.z;
     }
     const bool finite = mx < 0x7f800000u;
-    // the other elements' mean square root against the largest's; rows below 2^-97
-    // would need powers of two that are not normal
+    // the other pairs' sum of square roots against the largest's, whose share of it
+    // is line; rows below 2^-97 would need powers of two that are not normal
     const float top = rough_root(mx);
-    const int far = (count > 1.f) & (top * (count - 1.f) > line * (root - top));
+    const int far = top > line * (root - top);
     const int tiny = (mx != 0) & (mx < (127u - 97) << 23);
     const bool wide = (finite & (far | tiny)) | (!finite & (M < kInfRows));
     const int e = max((int)(mx >> 23) - 127, -97);
@@ -898,7 +892,7 @@ constexpr int64_t kSplitWideRows = 1280;
 
 template <bool NIB>
 int launch_split_digits(const LinearArgs& a, uint8_t* xt, float* rs, bool gelu, const PrefillFusion& f) {
-    const float line = kFar * sqrtf(sqrtf((float)a.K));
+    const float line = kFar * sqrtf(sqrtf((float)a.K)) / (0.5f * (float)a.K);
     auto launch = [&](auto kernel, int rows) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)((a.M + rows - 1) / rows)), dim3(kSplitThreads), 0, a.stream,
                            static_cast<const float*>(a.x), a.ldx, (int)a.M, (int)a.K, xt, rs, gelu, line, f.ln_w,

@@ -123,7 +123,7 @@ def test_wide_rows_in_a_block(dev, fmt):
     assert torch.equal(mod.forward_prefill(x, gelu=True, residual=res), res + mod(gelu_tanh(x)))
 
 
-# few large elements among zeros stay digits; subnormal rows and single elements
+# single elements among zeros, subnormal rows
 @torch.no_grad()
 def test_sparse_and_tiny_rows(dev):
     K, N = 768, 256
