@@ -219,7 +219,7 @@ bool bf16_split_rows(const LinearArgs& a) {
 
 using namespace tiq;
 
-extern "C" int tiq_version(void) { return 131; }
+extern "C" int tiq_version(void) { return 132; }
 
 extern "C" const char* tiq_status_string(int status) {
     switch (status) {

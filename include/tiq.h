@@ -253,10 +253,10 @@ int tiq_linear_w4g(const void* x, int x_dtype, int64_t M, int64_t K, int64_t ldx
  * 319,352,355 at M = B*T). With bf16 x, M >= 128 and a workspace of
  * tiq_gemm_w8_workspace(TIQ_BF16, M, K, N) bytes both split a product with few
  * output tiles over K (group-wise: whole groups a split), the fp32 slices
- * summed in a fixed order. Fewer fp32 rows take the planes too where
- * tiq_gemm_w8_workspace(TIQ_F32, M, K, N) gives a size for them (planes, then
- * the fp32 slices of a product split over K); with a smaller workspace such a
- * call computes what tiq_linear_w4 / tiq_linear_w4g compute. Where the
+ * summed in a fixed order; so are 5 to 127 bf16 rows of large products. Fewer
+ * fp32 rows take the planes too where tiq_linear_workspace gives a size for
+ * them (planes, then the fp32 slices of a product split over K); with a smaller
+ * workspace such a call computes what tiq_linear_w4 / tiq_linear_w4g compute. Where the
  * GEMM does not take the shape (K % 64, group % 64), and for bf16 x or
  * M < 128 without a workspace, they compute what tiq_linear_w4 /
  * tiq_linear_w4g compute. With fp32 x, M >= 128 and a
