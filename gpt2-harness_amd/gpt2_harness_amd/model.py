@@ -299,8 +299,10 @@ class CausalSelfAttention(nn.Module):
             x2 = x.view(B * T, C)
             # (a cache of another class, or whose update a caller replaced, is filled through it)
             plain = type(cache) is KVCache and "update" not in cache.__dict__
+            # (asked for few rows only: from 256 on no GPT-2 width's product is split, and a
+            # refusal costs no more than the attempt)
             if (plain and self.head_dim == 64 and self.c_attn.out_features == 3 * 64 * self.n_head
-                    and self.c_attn.writes_kv(B * T)):
+                    and (B * T >= 256 or self.c_attn.writes_kv(B * T))):
                 slots = cache._append_slots(self.layer_idx, B, self.n_head, T, x)
                 q = None if slots is None else self.c_attn.forward_prefill(x2, ln=ln, kv=(*slots, T))
                 if q is not None:
